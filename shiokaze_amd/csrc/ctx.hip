@@ -207,6 +207,24 @@ void fill_true_residual(shk_result *res, const double rr[4]) {
     res->true_relres_l2 = rr[2] > 0 ? std::sqrt(rr[1] / rr[2]) : 0.0;
 }
 
+template <class T>
+int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces, double tol_rel,
+                   int64_t max_iter, bool &ran) {
+    ran = false;
+    if (c->profile) return SHK_OK;  // ProfileKernels times the launches of the two-kernel iteration
+    const ResidentPlan p = resident_plan<T>(op, c->device, c->cus);
+    if (p.blocks < 1) return SHK_OK;
+    HIPC(c, c->slots.ensure(resident_slot_words()));
+    HIPC(c, resident_cg<T>(c->stream, p, op, rhs, sig, x, faces, c->slots.p, c->state.p, c->h_state, tol_rel, max_iter,
+                           c->device, c->cus));
+    ran = c->h_state->aborted == 0;
+    return SHK_OK;
+}
+template int solve_resident<float>(shk_ctx *, const BrickOp<float> &, const float *, const double *, float *, float *,
+                                   double, int64_t, bool &);
+template int solve_resident<double>(shk_ctx *, const BrickOp<double> &, const double *, const double *, double *,
+                                    double *, double, int64_t, bool &);
+
 // FP64 Krylov on the brick stencil: plain CG, or Jacobi PCG as CG on the
 // symmetrically scaled system (x = sig * x_scaled).
 int solve_fp64(shk_ctx *c, shk_result *res) {
@@ -219,23 +237,30 @@ int solve_fp64(shk_ctx *c, shk_result *res) {
         op.kappa = c->kappa64.p;
         op.kdiag = c->kdiag64.p;
     }
-    // the FP64 stencil holds 3 workgroups per CU, not 4: all kernels of the solve run on
-    // that many, so that the stencil's last quarter does not run as a second round
-    const Grid g = make_grid(c->grid.n, dir_spmv_resident<double, double>(c->grid, op));
-    const Reduction red = reduction(c);
-    launch_cg_init<double, double>(c->stream, g, c->b64.p, sig, c->x64.p, c->r64.p, c->s64.p, red, c->prm.residual,
-                                   c->prm.max_iterations);
-    double *S[2] = {c->s64.p, c->t64.p};
-    int m = 0;
-    launch_dir_spmv<double, double>(c->stream, g, op, c->r64.p, S[0], S[1], c->q64.p, red);
-    ++m;
-    int rc = drive(c, [&]() {
-        launch_axpy_norm<double>(c->stream, g, sig, c->x64.p, c->r64.p, S[m & 1], c->q64.p, red, c->next_events());
-        launch_dir_spmv<double, double>(c->stream, g, op, c->r64.p, S[m & 1], S[(m + 1) & 1], c->q64.p, red, c->next_events());
+    int rc;
+    bool ran = false;
+    if ((rc = solve_resident<double>(c, op, c->b64.p, sig, c->x64.p, c->q64.p, c->prm.residual, c->prm.max_iterations,
+                                     ran)))
+        return rc;
+    if (!ran) {
+        // the FP64 stencil holds 3 workgroups per CU, not 4: all kernels of the solve run on
+        // that many, so that the stencil's last quarter does not run as a second round
+        const Grid g = make_grid(c->grid.n, dir_spmv_resident<double, double>(c->grid, op));
+        const Reduction red = reduction(c);
+        launch_cg_init<double, double>(c->stream, g, c->b64.p, sig, c->x64.p, c->r64.p, c->s64.p, red, c->prm.residual,
+                                       c->prm.max_iterations);
+        double *S[2] = {c->s64.p, c->t64.p};
+        int m = 0;
+        launch_dir_spmv<double, double>(c->stream, g, op, c->r64.p, S[0], S[1], c->q64.p, red);
         ++m;
-    });
-    if (rc) return rc;
-    if (jac) launch_unscale(c->stream, g.n, c->x64.p, c->sig64.p);
+        rc = drive(c, [&]() {
+            launch_axpy_norm<double>(c->stream, g, sig, c->x64.p, c->r64.p, S[m & 1], c->q64.p, red, c->next_events());
+            launch_dir_spmv<double, double>(c->stream, g, op, c->r64.p, S[m & 1], S[(m + 1) & 1], c->q64.p, red, c->next_events());
+            ++m;
+        });
+        if (rc) return rc;
+    }
+    if (jac) launch_unscale(c->stream, c->grid.n, c->x64.p, c->sig64.p);
     res->count = c->h_state->iter;
     res->status = c->h_state->status;
     res->reresid = c->h_state->rnorm0 > 0 ? c->h_state->rnorm / c->h_state->rnorm0 : c->h_state->rnorm;
@@ -272,18 +297,24 @@ int solve_mixed(shk_ctx *c, shk_result *res) {
     while (r_inf > tol_abs && outer < std::max(1, c->prm.outer_max)) {
         double inner_rel = std::max(c->prm.inner_residual, 0.5 * tol_abs / r_inf);
         if (inner_rel > 0.5) inner_rel = 0.5;
-        launch_cg_init<float, float>(c->stream, g, c->rs32.p, nullptr, c->x32.p, c->r32.p, c->s32.p, red, inner_rel,
-                                     c->prm.max_iterations - total);
-        float *S[2] = {c->s32.p, c->t32.p};
-        int m = 0;
-        launch_dir_spmv<float, float>(c->stream, g, op, c->r32.p, S[0], S[1], c->q32.p, red);
-        ++m;
-        rc = drive(c, [&]() {
-            launch_axpy_norm<float>(c->stream, g, nullptr, c->x32.p, c->r32.p, S[m & 1], c->q32.p, red, c->next_events());
-            launch_dir_spmv<float, float>(c->stream, g, op, c->r32.p, S[m & 1], S[(m + 1) & 1], c->q32.p, red, c->next_events());
+        bool ran = false;
+        if ((rc = solve_resident<float>(c, op, c->rs32.p, nullptr, c->x32.p, c->q32.p, inner_rel,
+                                        c->prm.max_iterations - total, ran)))
+            return rc;
+        if (!ran) {
+            launch_cg_init<float, float>(c->stream, g, c->rs32.p, nullptr, c->x32.p, c->r32.p, c->s32.p, red, inner_rel,
+                                         c->prm.max_iterations - total);
+            float *S[2] = {c->s32.p, c->t32.p};
+            int m = 0;
+            launch_dir_spmv<float, float>(c->stream, g, op, c->r32.p, S[0], S[1], c->q32.p, red);
             ++m;
-        });
-        if (rc) return rc;
+            rc = drive(c, [&]() {
+                launch_axpy_norm<float>(c->stream, g, nullptr, c->x32.p, c->r32.p, S[m & 1], c->q32.p, red, c->next_events());
+                launch_dir_spmv<float, float>(c->stream, g, op, c->r32.p, S[m & 1], S[(m + 1) & 1], c->q32.p, red, c->next_events());
+                ++m;
+            });
+            if (rc) return rc;
+        }
         total += c->h_state->iter;
         ++outer;
         const int st = c->h_state->status;
@@ -368,6 +399,8 @@ int create_impl(int nx, int ny, int nz, int bx, double dx, int device, shk_ctx *
     };
     hipError_t e;
     if ((e = hipSetDevice(device)) != hipSuccess) return bail(e, "hipSetDevice");
+    if ((e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess)
+        return bail(e, "hipDeviceGetAttribute");
     // the device address of this device's allocation-free solve scratch (noalloc.hip)
     if ((e = shk::scratch_bind(device)) != hipSuccess) return bail(e, "hipGetSymbolAddress(scratch)");
     if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess)
@@ -449,6 +482,7 @@ void shk_destroy(shk_ctx *c) {
     for (auto &b : c->csr_i) b.release();
     for (auto &b : c->csr_d) b.release();
     c->state.release();
+    c->slots.release();
     if (c->h_state) (void)hipHostFree(c->h_state);
     if (c->h_misc) (void)hipHostFree(c->h_misc);
     for (auto &ev : c->ev)

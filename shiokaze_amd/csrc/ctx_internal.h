@@ -142,6 +142,8 @@ struct shk_ctx {
     DevBuf<int64_t> csr_i[2];
     DevBuf<double> csr_d[3];
     shk::Grid grid;
+    int cus = 0;                       // compute units of the device
+    DevBuf<unsigned long long> slots;  // exchange slots of the resident solve
     DevBuf<SolveState> state;
     SolveState *h_state = nullptr;
     double *h_misc = nullptr;
@@ -207,6 +209,12 @@ int drive(shk_ctx *c, F &&f, int interval = 0) {
     return drive_impl(c, [](void *p) { (*static_cast<F *>(p))(); }, &f, interval);
 }
 Reduction reduction(shk_ctx *c);
+// CG of op with the right-hand side rhs (FP64 with sig: the scaled system) into x on the
+// chip in one launch; ran = false when it has to be run another way.  faces: scratch of
+// at least 384 elements per brick.  The final state is in c->h_state.
+template <class T>
+int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces, double tol_rel,
+                   int64_t max_iter, bool &ran);
 BrickOp<double> op64(shk_ctx *c);
 BrickOp<float> op32(shk_ctx *c);
 // r = b - A x (FP64); out = {max|r|, sum r^2, sum b^2, max|b|}; optionally the

@@ -99,6 +99,24 @@ template <class T>
 void launch_axpy_norm(hipStream_t st, const Grid &g, const double *sig, T *x, T *r, const T *s, const T *q,
                       Reduction red, KEvents ev = {});
 
+// The whole CG solve in one launch with the vectors on the chip (resident.hip), for brick
+// operators with kappa (and kdiag).  The plan has blocks = 0 when the system does not fit;
+// sig as in launch_cg_init (FP64 with a unit diagonal only).  faces: n_active * 384
+// elements of scratch, slots: resident_slot_words().  Synchronises; *h_state then holds
+// the final state, and h_state->aborted says that the solve has to be run another way.
+struct ResidentPlan {
+    int bpw = 0;     // bricks per wave
+    int blocks = 0;  // workgroups, at most one per CU
+};
+constexpr int kResidentAborted = -1;
+size_t resident_slot_words();
+template <class T>
+ResidentPlan resident_plan(const BrickOp<T> &op, int device, int cus);
+template <class T>
+hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig,
+                       T *x, T *faces, unsigned long long *slots, SolveState *state, SolveState *h_state,
+                       double tol_rel, int64_t max_iter, int device, int cus);
+
 // r = b - A x in FP64 (unscaled operator with its diagonal); part holds 4*blocks
 // partials; out = {max|r|, sum r^2, sum b^2, max|b|}.  Optionally rs = (float)
 // (sig * r) (or (float) r without sig): the next inner solve's right-hand side.

@@ -1,0 +1,605 @@
+// resident.hip -- the whole CG solve of a brick system in one launch (see krylov.h).
+//
+// What bounds the two-kernel iteration (krylov.hip) depends on the size.  Small systems:
+// two launches of about 5 us each however little they do (fold of the partials, loads,
+// stores, one after another).  Systems that fit the caches: ten vector streams per
+// iteration, 52 bytes per cell in FP32.  One MI355X holds 128 MB of vector registers and
+// 40 MB of LDS, so up to a few million unknowns the four CG vectors fit on the chip:
+// here every wave keeps its bricks' r, s and q in registers (x too when they leave room,
+// else in LDS) for the whole solve, and one iteration moves only the brick faces:
+//   sigma = s.q            grid-wide exchange 1 (also: nobody reads old faces any more)
+//   x += alpha s; r -= alpha q; the faces of r go to memory
+//   rho = r.r, max|r|      grid-wide exchange 2 (also: the faces of r have arrived)
+//   the neighbours' faces of r are read; s = r + beta s, and the same on the halo planes
+//   of s, which stay in registers; q = A s
+// The arithmetic per cell is k_dir_spmv's and k_axpy_norm's; only the order in which the
+// partial sums are folded differs (one fixed order per launch shape, the same in every
+// workgroup).
+//
+// Exchange: each workgroup publishes its pair of partials in its own slot and one wave of
+// every workgroup polls all slots (a slot that holds the sentinel has not arrived yet),
+// so one exchange costs one store and one load through memory instead of a counter and
+// a second read.  Four slot sets rotate: passing exchange e proves that everybody has
+// finished reading set e - 2 = e + 2 (mod 4), which is cleared then.  Slots and faces are
+// written and read with agent-scope accesses (past the XCDs' private L2s); a workgroup's
+// face stores are complete (vmcnt 0 in every wave) before it arrives.
+//
+// Measured against the two-kernel iteration, whole projections to 1e-6: 32x36x28 mixed
+// Jacobi 2.56 -> 1.19 ms, 100x77x90 FP64 Jacobi 6.59 -> 4.33 ms, 256^3 mixed Jacobi 33.5 ->
+// 20.2 ms, 600x450 (2D) mixed Jacobi 21.1 -> 11.1 ms.
+//
+// All workgroups have to be on the chip at once.  A launch takes at most one workgroup
+// per CU, the launches of a process share that budget (CuBudget), and a wait that lasts
+// kWaitTicks gives up: every workgroup then leaves, the state says kResidentAborted and
+// the caller runs the two-kernel solve instead.
+#include <hip/hip_runtime.h>
+
+#include <condition_variable>
+#include <mutex>
+
+#include "krylov.h"
+#include "shk_projection.h"
+
+namespace shk {
+
+namespace {
+
+constexpr int RT = 512;               // threads of a workgroup: 8 waves, 2 per SIMD
+constexpr int RW = RT / kWave;        // waves of a workgroup
+constexpr int NT = kBrickCells;
+constexpr int kMaxWg = 256;           // slots of one exchange
+constexpr unsigned long long kEmpty = 0xFFF8DEADBEEF0001ull;  // a NaN that no sum produces
+constexpr unsigned long long kWaitTicks = 1ull << 26;         // 0.67 s of the 100 MHz clock
+
+__device__ inline void st_agent(unsigned long long *p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned long long ld_agent(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_face(float *p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_face(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ inline T ld_face(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct ExchLds {
+    double sum[RW], mx[RW];
+    double tot[2];
+    int gone;
+};
+
+// Sum of `v` and maximum of `m` over the grid, the same bits in every thread; false when a
+// wait gave up.  Every memory access issued before is complete when others pass.
+__device__ inline bool exchange(double v, double m, unsigned e, unsigned long long *slots, ExchLds &l, double &sum,
+                                double &mx) {
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, G = gridDim.x;
+    v = wave_sum(v);
+    m = wave_max(m);
+    if (lane == 0) {
+        l.sum[wave] = v;
+        l.mx[wave] = m;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (wave == 0) {
+        double ps = 0.0, pm = 0.0;
+#pragma unroll
+        for (int w = 0; w < RW; ++w) {
+            ps += l.sum[w];
+            pm = fmax(pm, l.mx[w]);
+        }
+        int gone = 0;
+        if (G > 1) {
+            unsigned long long *set = slots + (size_t)(e & 3) * (2 * kMaxWg);
+            if (lane < 2) {
+                unsigned long long bits = (unsigned long long)__double_as_longlong(lane ? pm : ps);
+                if (bits == kEmpty) bits ^= 2;
+                st_agent(set + lane * kMaxWg + blockIdx.x, bits);
+            }
+            unsigned long long a[kMaxWg / kWave], b[kMaxWg / kWave];
+            const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+            for (;;) {
+                bool ok = true;
+#pragma unroll
+                for (int c = 0; c < kMaxWg / kWave; ++c) {
+                    a[c] = b[c] = 0ull;
+                    const int w = lane + kWave * c;
+                    if (w < G) {
+                        a[c] = ld_agent(set + w);
+                        b[c] = ld_agent(set + kMaxWg + w);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < kMaxWg / kWave; ++c) ok = ok && a[c] != kEmpty && b[c] != kEmpty;
+                if (__all(ok)) break;
+                if (__builtin_amdgcn_s_memrealtime() - t0 > kWaitTicks) {
+                    gone = 1;
+                    break;
+                }
+            }
+            ps = pm = 0.0;
+#pragma unroll
+            for (int c = 0; c < kMaxWg / kWave; ++c) {
+                ps += __longlong_as_double((long long)a[c]);
+                pm = fmax(pm, __longlong_as_double((long long)b[c]));
+            }
+            ps = wave_sum(ps);
+            pm = wave_max(pm);
+            // this workgroup's slot of the set that exchange e + 2 uses
+            if (lane < 2) st_agent(slots + (size_t)((e + 2) & 3) * (2 * kMaxWg) + lane * kMaxWg + blockIdx.x, kEmpty);
+        }
+        if (lane == 0) {
+            l.tot[0] = ps;
+            l.tot[1] = pm;
+            l.gone = gone;
+        }
+    }
+    __syncthreads();
+    sum = l.tot[0];
+    mx = l.tot[1];
+    return l.gone == 0;
+}
+
+template <class T>
+__device__ inline T lane_get(T v, int src) {
+    return __shfl(v, src & (kWave - 1), kWave);
+}
+
+// the value of the lane before (CTRL 0x138, wave_shr:1) or after (0x130, wave_shl:1): a DPP
+// move, no LDS access; the ends get 0 (a halo value replaces them)
+template <int CTRL>
+__device__ inline float lane_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ inline double lane_shift(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+
+// Hides a wave-uniform value's origin, so that the addresses formed from it are computed
+// where they are used (scalar instructions) and not kept in registers through the solve.
+__device__ inline int here(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// LDS accesses of one wave are executed in order: keep the compiler from moving them
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The brick's face planes of r for the neighbours that exist: x planes as (y = a, z = c) at
+// a + Y c, y planes as (x = a, z = c) at a + X c, z planes (x, y) at the lane.  The lateral
+// planes lie across registers and lanes: they pass through the wave's LDS scratch.
+template <class T, int BX>
+__device__ inline void publish(const T (&r)[8], T *scr, T *face, int lane, const int (&nb)[6]) {
+    using B = BrickShape<BX>;
+    constexpr int X = B::X, Y = B::Y;
+    const int i = lane % X, j = lane / X;
+    if (i == 0 || i == X - 1) {
+        T *p = scr + (i ? 64 : 0) + j;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) p[Y * k] = r[k];
+    }
+    if constexpr (Y > 1) {
+        if (j == 0 || j == Y - 1) {
+            T *p = scr + (j ? 192 : 128) + i;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) p[X * k] = r[k];
+        }
+    }
+    wave_lds_fence();
+    const bool xl = lane < Y * 8;
+    if (nb[0] >= 0 && xl) st_face(face + lane, scr[lane]);
+    if (nb[1] >= 0 && xl) st_face(face + 64 + lane, scr[64 + lane]);
+    if constexpr (Y > 1) {
+        if (nb[2] >= 0) st_face(face + 128 + lane, scr[128 + lane]);
+        if (nb[3] >= 0) st_face(face + 192 + lane, scr[192 + lane]);
+    }
+    if (nb[4] >= 0) st_face(face + 256 + lane, r[0]);
+    if (nb[5] >= 0) st_face(face + 320 + lane, r[7]);
+    wave_lds_fence();
+}
+
+template <class T, bool UNIT, int BX, bool SCALED, int BPW>
+__global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *__restrict__ rhs,
+                                                       const double *__restrict__ sig, T *__restrict__ xout,
+                                                       T *__restrict__ faces, unsigned long long *__restrict__ slots,
+                                                       SolveState *__restrict__ st, double tol_rel, int64_t max_iter) {
+    using B = BrickShape<BX>;
+    constexpr int X = B::X, Y = B::Y;
+    constexpr bool XREG = BPW * (int)sizeof(T) <= 8;  // x in registers too
+    __shared__ ExchLds xl_;
+    __shared__ T scratch[RW][256];
+    __shared__ T halo[RW * BPW][256];  // the lateral halo planes of s (-x, +x, -y, +y)
+    __shared__ T xs[XREG ? 1 : RW * BPW * NT];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int i = lane % X, j = lane / X;
+    const bool xl = lane < Y * 8;
+    const int slot0 = (blockIdx.x * RW + wave) * BPW;
+    T *scr = scratch[wave];
+    // where an edge lane reads its halo value of z = k: + Y k (x planes), + X k (y planes)
+    const int hxo = (i == 0 ? 0 : 64) + j, hyo = (j == 0 ? 128 : 192) + i;
+    const bool xlo = i == 0, xhi = i == X - 1, ylo = j == 0, yhi = j == Y - 1;
+    T r[BPW][8], s[BPW][8], q[BPW][8], hz[BPW][2], x[XREG ? BPW : 1][8];
+    int nb[BPW][6];
+    unsigned e = 0;
+    double acc = 0.0, mx = 0.0;
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+        const int slot = slot0 + b;
+        const bool on = slot < op.n_active;
+#pragma unroll
+        for (int f = 0; f < 6; ++f) nb[b][f] = on ? __builtin_amdgcn_readfirstlane(op.nbr[6 * slot + f]) : -1;
+        hz[b][0] = hz[b][1] = T(0);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) halo[wave * BPW + b][64 * f + lane] = T(0);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            T rv = T(0);
+            if (on) {
+                const T bv = (rhs + (int64_t)slot * NT)[lane + 64 * k];
+                const double sg = SCALED ? (sig + (int64_t)slot * NT)[lane + 64 * k] : 1.0;
+                rv = SCALED ? (T)(sg * (double)bv) : bv;
+                // with a scaled system the stop test is on the unscaled residual: max|b|
+                mx = fmax(mx, SCALED ? (sg > 0.0 ? fabs((double)bv) : 0.0) : fabs((double)rv));
+            }
+            r[b][k] = s[b][k] = rv;
+            q[b][k] = T(0);
+            if constexpr (XREG)
+                x[b][k] = T(0);
+            else
+                xs[((wave * BPW + b) * 8 + k) * 64 + lane] = T(0);
+            acc += (double)rv * (double)rv;
+        }
+        if (on) publish<T, BX>(r[b], scr, faces + (int64_t)slot * 384, lane, nb[b]);
+    }
+    double rho = 0.0, rn = 0.0, sigma = 0.0, alpha = 0.0, beta = 0.0;
+    bool alive = exchange(acc, mx, e++, slots, xl_, rho, rn);
+    const double rnorm0 = rn;
+    const double tol_abs = (tol_rel < 1e-30 ? 1e-30 : tol_rel) * rnorm0;  // pcg_solver.h:235
+    int64_t it = 0;
+    int status = SHK_OK;
+    bool done = !alive;
+    // pcg_solver.h:254-271: zero rhs, rho == 0, NaN (as k_finish_init)
+    if (rnorm0 == 0.0) {
+        done = true;
+    } else if (rho == 0.0) {
+        done = true;
+        status = SHK_BREAKDOWN;
+    } else if (rho != rho) {
+        done = true;
+        status = SHK_NAN;
+    } else if (max_iter <= 0) {
+        done = true;
+        status = SHK_NOT_CONVERGED;
+    }
+    while (!done) {
+        // the neighbours' faces of r: s = r + beta s on the halo planes and the cells
+        const T bt = (T)beta;
+        T hr[BPW][6];
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) {
+            int n[6];
+#pragma unroll
+            for (int f = 0; f < 6; ++f) n[f] = here(nb[b][f]);
+            hr[b][0] = n[0] >= 0 && xl ? ld_face(faces + (int64_t)n[0] * 384 + 64 + lane) : T(0);
+            hr[b][1] = n[1] >= 0 && xl ? ld_face(faces + (int64_t)n[1] * 384 + lane) : T(0);
+            hr[b][2] = hr[b][3] = T(0);
+            if constexpr (Y > 1) {
+                hr[b][2] = n[2] >= 0 ? ld_face(faces + (int64_t)n[2] * 384 + 192 + lane) : T(0);
+                hr[b][3] = n[3] >= 0 ? ld_face(faces + (int64_t)n[3] * 384 + 128 + lane) : T(0);
+            }
+            hr[b][4] = n[4] >= 0 ? ld_face(faces + (int64_t)n[4] * 384 + 320 + lane) : T(0);
+            hr[b][5] = n[5] >= 0 ? ld_face(faces + (int64_t)n[5] * 384 + 256 + lane) : T(0);
+        }
+        if (it > 0) {  // the first direction is r itself
+#pragma unroll
+            for (int b = 0; b < BPW; ++b)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) s[b][k] = r[b][k] + bt * s[b][k];
+        }
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) {
+            T *hp = halo[wave * BPW + b];
+#pragma unroll
+            for (int f = 0; f < (Y > 1 ? 4 : 2); ++f) hp[64 * f + lane] = hr[b][f] + bt * hp[64 * f + lane];
+            hz[b][0] = hr[b][4] + bt * hz[b][0];
+            hz[b][1] = hr[b][5] + bt * hz[b][1];
+        }
+        wave_lds_fence();
+        acc = 0.0;
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) {
+            __builtin_amdgcn_sched_barrier(0);  // one brick at a time: registers
+            const int slot = here(slot0) + b;
+            if (slot >= op.n_active) continue;
+            const T *hp = halo[wave * BPW + b];
+            const T kv = op.kappa[slot];
+            if (kv != T(0)) {
+                const T kd = UNIT ? T(0) : op.kdiag[slot];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const T sk = s[b][k];
+                    const T hx = hp[hxo + Y * k];
+                    const T lf = lane_shift<0x138>(sk), rt = lane_shift<0x130>(sk);  // every lane takes part
+                    const T xm = xlo ? hx : lf, xp = xhi ? hx : rt;
+                    T ym = T(0), yp = T(0);
+                    if constexpr (Y > 1) {
+                        const T hy = hp[hyo + X * k];
+                        const T dn = lane_get(sk, lane - X), up = lane_get(sk, lane + X);
+                        ym = ylo ? hy : dn;
+                        yp = yhi ? hy : up;
+                    }
+                    const T zm = k > 0 ? s[b][k - 1] : hz[b][0];
+                    const T zp = k < 7 ? s[b][k + 1] : hz[b][1];
+                    T qv = UNIT ? sk : kd * sk;
+                    qv -= kv * xm + kv * xp + kv * ym + kv * yp + kv * zm + kv * zp;
+                    q[b][k] = qv;
+                    acc += (double)sk * (double)qv;
+                }
+                continue;
+            }
+            // the couplings of the other bricks are read again every iteration (they stay in
+            // the L2s); those of the +x / +y / +z faces live in the neighbour bricks
+            const T *cx = op.cx + (int64_t)slot * NT, *cy = op.cy + (int64_t)slot * NT, *cz = op.cz + (int64_t)slot * NT;
+            const T *dg = UNIT ? nullptr : op.diag + (int64_t)slot * NT;
+            const int n[6] = {0, here(nb[b][1]), 0, here(nb[b][3]), 0, here(nb[b][5])};
+            // a cell's +x / +y coupling is its neighbour's low one, in the next brick for the edge
+            // lanes (without one the halo value is 0, and any finite coupling will do)
+            const T *cxn = cx + (xhi ? lane : lane + 1), *cyn = cy + (yhi ? lane : lane + X);
+            if (n[1] >= 0) cxn = xhi ? op.cx + (int64_t)n[1] * NT + X * j : cxn;
+            if (n[3] >= 0) cyn = yhi ? op.cy + (int64_t)n[3] * NT + i : cyn;
+            const T czh = n[5] >= 0 ? (op.cz + (int64_t)n[5] * NT)[lane] : T(0);
+            T czk = cz[lane];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if constexpr (BPW * sizeof(T) > 8)
+                    if ((k & 1) == 0) __builtin_amdgcn_sched_barrier(0);
+                const T sk = s[b][k];
+                const T cxv = cx[lane + 64 * k];
+                const T cyv = Y > 1 ? cy[lane + 64 * k] : T(0);
+                const T czp = k < 7 ? cz[lane + 64 * (k + 1)] : czh;
+                const T hx = hp[hxo + Y * k];
+                const T lf = lane_shift<0x138>(sk), rt = lane_shift<0x130>(sk);
+                const T xm = xlo ? hx : lf, xp = xhi ? hx : rt;
+                const T cxp = cxn[64 * k];
+                T ym = T(0), yp = T(0), cyp = T(0);
+                if constexpr (Y > 1) {
+                    const T hy = hp[hyo + X * k];
+                    const T dn = lane_get(sk, lane - X), up = lane_get(sk, lane + X);
+                    ym = ylo ? hy : dn;
+                    yp = yhi ? hy : up;
+                    cyp = cyn[64 * k];
+                }
+                const T zm = k > 0 ? s[b][k - 1] : hz[b][0];
+                const T zp = k < 7 ? s[b][k + 1] : hz[b][1];
+                T qv = UNIT ? sk : dg[lane + 64 * k] * sk;
+                qv -= cxv * xm + cxp * xp + cyv * ym + cyp * yp + czk * zm + czp * zp;
+                czk = czp;
+                q[b][k] = qv;
+                acc += (double)sk * (double)qv;
+            }
+        }
+        if (!(alive = exchange(acc, 0.0, e++, slots, xl_, sigma, mx))) break;
+        if (!(sigma > 0.0)) {
+            status = sigma != sigma ? SHK_NAN : SHK_BREAKDOWN;
+            break;
+        }
+        alpha = rho / sigma;
+        ++it;
+        const T a = (T)alpha;
+        acc = 0.0;
+        mx = 0.0;
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int slot = here(slot0) + b;
+            if (slot >= op.n_active) continue;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if constexpr (XREG)
+                    x[b][k] += a * s[b][k];
+                else
+                    xs[((wave * BPW + b) * 8 + k) * 64 + lane] += a * s[b][k];
+                const T rv = r[b][k] - a * q[b][k];
+                r[b][k] = rv;
+                acc += (double)rv * (double)rv;
+                if constexpr (SCALED) {
+                    const double sg = (sig + (int64_t)slot * NT)[lane + 64 * k];
+                    if (sg > 0.0) mx = fmax(mx, fabs((double)rv) / sg);
+                } else {
+                    mx = fmax(mx, fabs((double)rv));
+                }
+            }
+            int n[6];
+#pragma unroll
+            for (int f = 0; f < 6; ++f) n[f] = here(nb[b][f]);
+            publish<T, BX>(r[b], scr, faces + (int64_t)slot * 384, lane, n);
+        }
+        double rho_new;
+        if (!(alive = exchange(acc, mx, e++, slots, xl_, rho_new, rn))) break;
+        // the stop test of pcg_solver.h:281-284 and beta of :287-289 (as direction_step)
+        if (rn <= tol_abs) {
+            done = true;
+        } else if (rho_new != rho_new) {
+            status = SHK_NAN;
+            done = true;
+        } else if (it >= max_iter) {
+            status = SHK_NOT_CONVERGED;
+            done = true;
+        } else {
+            beta = rho_new / rho;
+            rho = rho_new;
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+        const int slot = slot0 + b;
+        if (slot >= op.n_active) continue;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            (xout + (int64_t)slot * NT)[lane + 64 * k] = XREG ? x[XREG ? b : 0][k]
+                                                            : xs[XREG ? 0 : ((wave * BPW + b) * 8 + k) * 64 + lane];
+    }
+    if (!alive) status = kResidentAborted;
+    // an aborted wait is seen by some workgroups only: any of them says so
+    if (threadIdx.x == 0 && (blockIdx.x == 0 || !alive)) {
+        if (blockIdx.x == 0) {
+            st->rho_k1 = rho;
+            st->rho_k2 = rho;
+            st->alpha = alpha;
+            st->beta = beta;
+            st->sigma = sigma;
+            st->rnorm = rn;
+            st->rnorm0 = rnorm0;
+            st->tol_abs = tol_abs;
+            st->iter = it;
+            st->max_iter = max_iter;
+            st->done = 1;
+            st->status = status;
+        }
+        if (!alive) st->aborted = 1;
+    }
+}
+
+__global__ void k_resident_begin(SolveState *st, unsigned long long *slots) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 4 * 2 * kMaxWg) slots[i] = kEmpty;
+    if (i == 0) st->aborted = 0;
+}
+
+// Workgroups of resident launches in flight per device: their sum never exceeds the CUs,
+// so that every launch gets all of its workgroups onto the chip.
+struct CuBudget {
+    std::mutex m;
+    std::condition_variable cv;
+    int used = 0;
+};
+constexpr int kMaxDevices = 64;
+CuBudget g_budget[kMaxDevices];
+
+// Bricks per wave the kernels are built for.  The registers of a wave at 2 waves per SIMD
+// (256) hold 6 FP32 bricks (r, s, q and the halo of s: 30 each) or 2 FP64 ones.
+constexpr int kBpwF32[] = {1, 2, 3, 4, 6};
+constexpr int kBpwF64[] = {1, 2};
+
+template <class T, bool UNIT, int BX, bool SCALED, int BPW>
+void launch_one(hipStream_t st, int blocks, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces,
+                unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter) {
+    hipLaunchKernelGGL((k_cg_resident<T, UNIT, BX, SCALED, BPW>), dim3(blocks), dim3(RT), 0, st, op, rhs, sig, x,
+                       faces, slots, state, tol_rel, max_iter);
+}
+
+template <class T, bool UNIT, int BX, bool SCALED>
+void launch_bpw(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig, T *x,
+                T *faces, unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter) {
+#define SHK_RES(N)                                                                                                  \
+    case N:                                                                                                         \
+        launch_one<T, UNIT, BX, SCALED, N>(st, p.blocks, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter); \
+        break
+    if constexpr (sizeof(T) == 4) {
+        switch (p.bpw) {
+            SHK_RES(1);
+            SHK_RES(2);
+            SHK_RES(3);
+            SHK_RES(4);
+            SHK_RES(6);
+        }
+    } else {
+        switch (p.bpw) {
+            SHK_RES(1);
+            SHK_RES(2);
+        }
+    }
+#undef SHK_RES
+}
+
+}  // namespace
+
+size_t resident_slot_words() { return 4 * 2 * kMaxWg; }
+
+template <class T>
+ResidentPlan resident_plan(const BrickOp<T> &op, int device, int cus) {
+    ResidentPlan p;
+    if (device < 0 || device >= kMaxDevices || op.n_active < 1 || !op.kappa || (op.diag && !op.kdiag)) return p;
+    const int cap = cus < kMaxWg ? cus : kMaxWg;
+    auto fits = [&](int bpw) {
+        const int blocks = (op.n_active + RW * bpw - 1) / (RW * bpw);
+        if (blocks > cap) return false;
+        p.bpw = bpw;
+        p.blocks = blocks;
+        return true;
+    };
+    if constexpr (sizeof(T) == 4) {
+        for (int b : kBpwF32)
+            if (fits(b)) break;
+    } else {
+        for (int b : kBpwF64)
+            if (fits(b)) break;
+    }
+    return p;
+}
+
+template <class T>
+hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig,
+                       T *x, T *faces, unsigned long long *slots, SolveState *state, SolveState *h_state,
+                       double tol_rel, int64_t max_iter, int device, int cus) {
+    CuBudget &bud = g_budget[device];
+    {
+        std::unique_lock<std::mutex> lk(bud.m);
+        bud.cv.wait(lk, [&] { return bud.used + p.blocks <= cus; });
+        bud.used += p.blocks;
+    }
+    hipLaunchKernelGGL(k_resident_begin, dim3((4 * 2 * kMaxWg + 255) / 256), dim3(256), 0, st, state, slots);
+    const bool unit = op.diag == nullptr, flat = op.bx == 64;
+    if constexpr (sizeof(T) == 4) {
+        if (unit && flat)
+            launch_bpw<T, true, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else if (unit)
+            launch_bpw<T, true, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else if (flat)
+            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else
+            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+    } else {
+        if (unit && flat)
+            launch_bpw<T, true, 64, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else if (unit)
+            launch_bpw<T, true, 8, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else if (flat)
+            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+        else
+            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+    }
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(h_state, state, sizeof(SolveState), hipMemcpyDeviceToHost, st);
+    const hipError_t e2 = hipStreamSynchronize(st);  // also after an error: the budget covers what runs
+    {
+        std::lock_guard<std::mutex> lk(bud.m);
+        bud.used -= p.blocks;
+    }
+    bud.cv.notify_all();
+    return e != hipSuccess ? e : e2;
+}
+
+template ResidentPlan resident_plan<float>(const BrickOp<float> &, int, int);
+template ResidentPlan resident_plan<double>(const BrickOp<double> &, int, int);
+template hipError_t resident_cg<float>(hipStream_t, const ResidentPlan &, const BrickOp<float> &, const float *,
+                                       const double *, float *, float *, unsigned long long *, SolveState *,
+                                       SolveState *, double, int64_t, int, int);
+template hipError_t resident_cg<double>(hipStream_t, const ResidentPlan &, const BrickOp<double> &, const double *,
+                                        const double *, double *, double *, unsigned long long *, SolveState *,
+                                        SolveState *, double, int64_t, int, int);
+
+}  // namespace shk

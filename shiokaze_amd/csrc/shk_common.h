@@ -41,6 +41,8 @@ struct SolveState {
     int64_t max_iter;
     int32_t done;     // 1 once converged, capped or broken down
     int32_t status;   // shk_status
+    int32_t aborted;  // 1: a resident solve gave up waiting for its workgroups (resident.hip)
+    int32_t pad;
 };
 
 // Device-side control of one inner flexible-CG solve (the learned preconditioner's):
