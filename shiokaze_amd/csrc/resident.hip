@@ -25,8 +25,10 @@
 // face stores are complete (vmcnt 0 in every wave) before it arrives.
 //
 // Measured against the two-kernel iteration, whole projections to 1e-6: 32x36x28 mixed
-// Jacobi 2.56 -> 1.19 ms, 100x77x90 FP64 Jacobi 6.59 -> 4.33 ms, 256^3 mixed Jacobi 33.5 ->
-// 20.2 ms, 600x450 (2D) mixed Jacobi 21.1 -> 11.1 ms.
+// Jacobi 2.38 -> 0.90 ms, 100x77x90 FP64 Jacobi 6.9 -> 2.8 ms, 256^3 mixed Jacobi 32.1 ->
+// 13.3 ms, 600x450 (2D) mixed Jacobi 20.3 -> 7.2 ms.  One iteration at 256^3 takes 48.5
+// thousand cycles (52 us before): 16 the stencil, 17 the two exchanges with the wait for
+// the slowest workgroup, 7 the halo planes, 9 the update and the faces.
 //
 // All workgroups have to be on the chip at once.  A launch takes at most one workgroup
 // per CU, the launches of a process share that budget (CuBudget), and a wait that lasts
@@ -48,6 +50,12 @@ constexpr int RT = 512;               // threads of a workgroup: 8 waves, 2 per 
 constexpr int RW = RT / kWave;        // waves of a workgroup
 constexpr int NT = kBrickCells;
 constexpr int kMaxWg = 256;           // slots of one exchange
+// Every slot has kRep copies, and workgroup g polls copy g % kRep: with one copy 256 polling
+// workgroups wait for the same few cache lines (2.8 us per exchange; 2.0 with 4 to 16
+// copies; 32 workgroups 1.9 and 1.45).  The copies' spacing keeps them off one memory
+// channel.  A slot is a pair of words, kMaxWg apart: sum and maximum.
+constexpr int kRep = 8;
+constexpr int kRepWords = 2 * kMaxWg + 32, kSetWords = kRep * kRepWords, kSlotWords = 4 * kSetWords;
 constexpr unsigned long long kEmpty = 0xFFF8DEADBEEF0001ull;  // a NaN that no sum produces
 constexpr unsigned long long kWaitTicks = 1ull << 26;         // 0.67 s of the 100 MHz clock
 
@@ -68,22 +76,51 @@ __device__ inline T ld_face(const T *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <int CTRL>
+__device__ inline double dpp64(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ inline double lane_of(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// Sum / maximum over the wave, the same in every lane: DPP moves within the rows of 16
+// (neighbours, pairs, half rows, rows), then the four rows in order.  The shuffles of
+// wave_sum take about five times as long, and an exchange has two of these in a row.
+struct OpAdd {
+    __device__ static double f(double a, double b) { return a + b; }
+};
+struct OpMax {
+    __device__ static double f(double a, double b) { return fmax(a, b); }
+};
+template <class OP>
+__device__ inline double wave_all(double v) {
+    v = OP::f(v, dpp64<0xB1>(v));   // quad_perm 1,0,3,2
+    v = OP::f(v, dpp64<0x4E>(v));   // quad_perm 2,3,0,1
+    v = OP::f(v, dpp64<0x141>(v));  // row_half_mirror
+    v = OP::f(v, dpp64<0x140>(v));  // row_mirror
+    return OP::f(OP::f(lane_of(v, 0), lane_of(v, 16)), OP::f(lane_of(v, 32), lane_of(v, 48)));
+}
+
 struct ExchLds {
     double sum[RW], mx[RW];
     double tot[2];
     int gone;
 };
 
-// Sum of `v` and maximum of `m` over the grid, the same bits in every thread; false when a
-// wait gave up.  Every memory access issued before is complete when others pass.
+// Sum of `v` (and, with MAX, the maximum of `m`) over the grid, the same bits in every
+// thread; false when a wait gave up.  Every memory access issued before is complete when
+// others pass.
+template <bool MAX>
 __device__ inline bool exchange(double v, double m, unsigned e, unsigned long long *slots, ExchLds &l, double &sum,
                                 double &mx) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, G = gridDim.x;
-    v = wave_sum(v);
-    m = wave_max(m);
+    v = wave_all<OpAdd>(v);
+    if constexpr (MAX) m = wave_all<OpMax>(m);
     if (lane == 0) {
         l.sum[wave] = v;
-        l.mx[wave] = m;
+        if constexpr (MAX) l.mx[wave] = m;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -92,16 +129,19 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
 #pragma unroll
         for (int w = 0; w < RW; ++w) {
             ps += l.sum[w];
-            pm = fmax(pm, l.mx[w]);
+            if constexpr (MAX) pm = fmax(pm, l.mx[w]);
         }
         int gone = 0;
         if (G > 1) {
-            unsigned long long *set = slots + (size_t)(e & 3) * (2 * kMaxWg);
-            if (lane < 2) {
-                unsigned long long bits = (unsigned long long)__double_as_longlong(lane ? pm : ps);
+            // lanes 0..7 store the sum's copies, lanes 8..15 the maximum's
+            const int copy = (lane & (kRep - 1)) * kRepWords + (lane >= kRep ? kMaxWg : 0) + blockIdx.x;
+            unsigned long long *set = slots + (size_t)(e & 3) * kSetWords;
+            if (lane < (MAX ? 2 : 1) * kRep) {
+                unsigned long long bits = (unsigned long long)__double_as_longlong(lane >= kRep ? pm : ps);
                 if (bits == kEmpty) bits ^= 2;
-                st_agent(set + lane * kMaxWg + blockIdx.x, bits);
+                st_agent(set + copy, bits);
             }
+            const unsigned long long *mine = set + (size_t)(blockIdx.x % kRep) * kRepWords;
             unsigned long long a[kMaxWg / kWave], b[kMaxWg / kWave];
             const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
             for (;;) {
@@ -111,8 +151,8 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
                     a[c] = b[c] = 0ull;
                     const int w = lane + kWave * c;
                     if (w < G) {
-                        a[c] = ld_agent(set + w);
-                        b[c] = ld_agent(set + kMaxWg + w);
+                        a[c] = ld_agent(mine + w);
+                        if constexpr (MAX) b[c] = ld_agent(mine + kMaxWg + w);
                     }
                 }
 #pragma unroll
@@ -123,16 +163,16 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
                     break;
                 }
             }
+            // this workgroup's slot of the set that exchange e + 2 uses
+            if (lane < 2 * kRep) st_agent(slots + (size_t)((e + 2) & 3) * kSetWords + copy, kEmpty);
             ps = pm = 0.0;
 #pragma unroll
             for (int c = 0; c < kMaxWg / kWave; ++c) {
                 ps += __longlong_as_double((long long)a[c]);
-                pm = fmax(pm, __longlong_as_double((long long)b[c]));
+                if constexpr (MAX) pm = fmax(pm, __longlong_as_double((long long)b[c]));
             }
-            ps = wave_sum(ps);
-            pm = wave_max(pm);
-            // this workgroup's slot of the set that exchange e + 2 uses
-            if (lane < 2) st_agent(slots + (size_t)((e + 2) & 3) * (2 * kMaxWg) + lane * kMaxWg + blockIdx.x, kEmpty);
+            ps = wave_all<OpAdd>(ps);
+            if constexpr (MAX) pm = wave_all<OpMax>(pm);
         }
         if (lane == 0) {
             l.tot[0] = ps;
@@ -142,7 +182,7 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
     }
     __syncthreads();
     sum = l.tot[0];
-    mx = l.tot[1];
+    if constexpr (MAX) mx = l.tot[1];
     return l.gone == 0;
 }
 
@@ -159,8 +199,7 @@ __device__ inline float lane_shift(float v) {
 }
 template <int CTRL>
 __device__ inline double lane_shift(double v) {
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
-                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+    return dpp64<CTRL>(v);
 }
 
 // Hides a wave-uniform value's origin, so that the addresses formed from it are computed
@@ -168,6 +207,14 @@ __device__ inline double lane_shift(double v) {
 __device__ inline int here(int v) {
     asm volatile("" : "+s"(v));
     return v;
+}
+
+// acc += v, with PIN not moved behind later cells: the compiler would otherwise keep every
+// cell's factors as doubles (two registers each) until the end of the brick
+template <bool PIN>
+__device__ inline void add_here(double &acc, double v) {
+    acc += v;
+    if constexpr (PIN) asm volatile("" : "+v"(acc));
 }
 
 // LDS accesses of one wave are executed in order: keep the compiler from moving them
@@ -210,6 +257,51 @@ __device__ inline void publish(const T (&r)[8], T *scr, T *face, int lane, const
     wave_lds_fence();
 }
 
+// The couplings of a cell column: low x, high x, low y, high y, low z (the high z ones are
+// the next cell's low ones; c.top is the one above the brick) and the diagonal.
+template <class T, bool UNIT>
+struct Couplings {
+    T x[8], xp[8], y[8], yp[8], z[8], top, d[UNIT ? 1 : 8];
+};
+// where they lie, as 32-bit byte offsets (a resident system is far below 4 GB); a cell's +x /
+// +y coupling is its neighbour's low one, in the next brick for the edge lanes (without one
+// the halo value is 0, and any finite coupling will do)
+template <class T, bool UNIT, int BX>
+struct CouplingAt {
+    const char *cx, *cy, *cz, *dg;
+    uint32_t own, xp, yp, up;
+    bool open;
+    __device__ CouplingAt(const BrickOp<T> &op, int slot, const int (&nb)[6], int lane) {
+        constexpr int X = BrickShape<BX>::X, Y = BrickShape<BX>::Y;
+        const int i = lane % X, j = lane / X;
+        cx = (const char *)op.cx;
+        cy = (const char *)op.cy;
+        cz = (const char *)op.cz;
+        dg = (const char *)op.diag;
+        const int base = slot * NT;
+        open = nb[5] >= 0;
+        const int xi = i < X - 1 ? base + lane + 1 : (nb[1] >= 0 ? nb[1] * NT + X * j : base + lane);
+        const int yi = j < Y - 1 ? base + lane + X : (nb[3] >= 0 ? nb[3] * NT + i : base + lane);
+        own = (uint32_t)(base + lane) * (uint32_t)sizeof(T);
+        xp = (uint32_t)xi * (uint32_t)sizeof(T);
+        yp = (uint32_t)yi * (uint32_t)sizeof(T);
+        up = (uint32_t)((open ? nb[5] : slot) * NT + lane) * (uint32_t)sizeof(T);
+    }
+    __device__ static T at(const char *p, uint32_t off, int k) {
+        return *reinterpret_cast<const T *>(p + off + 64 * k * (int)sizeof(T));
+    }
+    __device__ void load(Couplings<T, UNIT> &c, int k) const {
+        constexpr int Y = BrickShape<BX>::Y;
+        c.x[k] = at(cx, own, k);
+        c.xp[k] = at(cx, xp, k);
+        c.y[k] = Y > 1 ? at(cy, own, k) : T(0);
+        c.yp[k] = Y > 1 ? at(cy, yp, k) : T(0);
+        c.z[k] = at(cz, own, k);
+        if (!UNIT) c.d[UNIT ? 0 : k] = at(dg, own, k);
+        if (k == 7) c.top = open ? at(cz, up, 0) : T(0);
+    }
+};
+
 template <class T, bool UNIT, int BX, bool SCALED, int BPW>
 __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *__restrict__ rhs,
                                                        const double *__restrict__ sig, T *__restrict__ xout,
@@ -217,7 +309,10 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
                                                        SolveState *__restrict__ st, double tol_rel, int64_t max_iter) {
     using B = BrickShape<BX>;
     constexpr int X = B::X, Y = B::Y;
-    constexpr bool XREG = BPW * (int)sizeof(T) <= 8;  // x in registers too
+    // with few bricks x and the couplings stay in registers too; else the couplings are read
+    // every iteration (they stay in the L2s), two cells of a column ahead of their use
+    constexpr bool XREG = BPW * (int)sizeof(T) <= 8, CREG = XREG;
+    constexpr int NC = CREG ? BPW : 1;
     __shared__ ExchLds xl_;
     __shared__ T scratch[RW][256];
     __shared__ T halo[RW * BPW][256];  // the lateral halo planes of s (-x, +x, -y, +y)
@@ -226,22 +321,35 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = lane % X, j = lane / X;
     const bool xl = lane < Y * 8;
-    const int slot0 = (blockIdx.x * RW + wave) * BPW;
+    // bricks blockIdx + G (wave + 8 b): those with couplings of their own lie together (walls,
+    // the surface) and cost several times a uniform brick, so they are dealt out one by one
+    const int slot0 = blockIdx.x + gridDim.x * wave, stride = gridDim.x * RW;
     T *scr = scratch[wave];
     // where an edge lane reads its halo value of z = k: + Y k (x planes), + X k (y planes)
     const int hxo = (i == 0 ? 0 : 64) + j, hyo = (j == 0 ? 128 : 192) + i;
     const bool xlo = i == 0, xhi = i == X - 1, ylo = j == 0, yhi = j == Y - 1;
     T r[BPW][8], s[BPW][8], q[BPW][8], hz[BPW][2], x[XREG ? BPW : 1][8];
     int nb[BPW][6];
+    T kap[BPW], kd[BPW];
+    Couplings<T, UNIT> cpl[NC];
+    T isg[SCALED && CREG ? BPW : 1][8];  // 1 / sig for the stop test
     unsigned e = 0;
     double acc = 0.0, mx = 0.0;
 #pragma unroll
     for (int b = 0; b < BPW; ++b) {
-        const int slot = slot0 + b;
+        const int slot = slot0 + stride * b;
         const bool on = slot < op.n_active;
 #pragma unroll
         for (int f = 0; f < 6; ++f) nb[b][f] = on ? __builtin_amdgcn_readfirstlane(op.nbr[6 * slot + f]) : -1;
         hz[b][0] = hz[b][1] = T(0);
+        kap[b] = on ? op.kappa[slot] : T(1);
+        kd[b] = !UNIT && on ? op.kdiag[slot] : T(0);
+        if constexpr (CREG)
+            if (kap[b] == T(0)) {
+                const CouplingAt<T, UNIT, BX> at(op, slot, nb[b], lane);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) at.load(cpl[CREG ? b : 0], k);
+            }
 #pragma unroll
         for (int f = 0; f < 4; ++f) halo[wave * BPW + b][64 * f + lane] = T(0);
 #pragma unroll
@@ -251,6 +359,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
                 const T bv = (rhs + (int64_t)slot * NT)[lane + 64 * k];
                 const double sg = SCALED ? (sig + (int64_t)slot * NT)[lane + 64 * k] : 1.0;
                 rv = SCALED ? (T)(sg * (double)bv) : bv;
+                if constexpr (SCALED && CREG) isg[b][k] = sg > 0.0 ? (T)(1.0 / sg) : T(0);
                 // with a scaled system the stop test is on the unscaled residual: max|b|
                 mx = fmax(mx, SCALED ? (sg > 0.0 ? fabs((double)bv) : 0.0) : fabs((double)rv));
             }
@@ -265,7 +374,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
         if (on) publish<T, BX>(r[b], scr, faces + (int64_t)slot * 384, lane, nb[b]);
     }
     double rho = 0.0, rn = 0.0, sigma = 0.0, alpha = 0.0, beta = 0.0;
-    bool alive = exchange(acc, mx, e++, slots, xl_, rho, rn);
+    bool alive = exchange<true>(acc, mx, e++, slots, xl_, rho, rn);
     const double rnorm0 = rn;
     const double tol_abs = (tol_rel < 1e-30 ? 1e-30 : tol_rel) * rnorm0;  // pcg_solver.h:235
     int64_t it = 0;
@@ -287,22 +396,16 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
     while (!done) {
         // the neighbours' faces of r: s = r + beta s on the halo planes and the cells
         const T bt = (T)beta;
-        T hr[BPW][6];
+        if constexpr (!CREG)
+            if (kap[0] == T(0)) {
+                int n[6];
 #pragma unroll
-        for (int b = 0; b < BPW; ++b) {
-            int n[6];
-#pragma unroll
-            for (int f = 0; f < 6; ++f) n[f] = here(nb[b][f]);
-            hr[b][0] = n[0] >= 0 && xl ? ld_face(faces + (int64_t)n[0] * 384 + 64 + lane) : T(0);
-            hr[b][1] = n[1] >= 0 && xl ? ld_face(faces + (int64_t)n[1] * 384 + lane) : T(0);
-            hr[b][2] = hr[b][3] = T(0);
-            if constexpr (Y > 1) {
-                hr[b][2] = n[2] >= 0 ? ld_face(faces + (int64_t)n[2] * 384 + 192 + lane) : T(0);
-                hr[b][3] = n[3] >= 0 ? ld_face(faces + (int64_t)n[3] * 384 + 128 + lane) : T(0);
+                for (int f = 0; f < 6; ++f) n[f] = here(nb[0][f]);
+                const CouplingAt<T, UNIT, BX> at(op, here(slot0), n, lane);
+                at.load(cpl[0], 0);
+                at.load(cpl[0], 1);
             }
-            hr[b][4] = n[4] >= 0 ? ld_face(faces + (int64_t)n[4] * 384 + 320 + lane) : T(0);
-            hr[b][5] = n[5] >= 0 ? ld_face(faces + (int64_t)n[5] * 384 + 256 + lane) : T(0);
-        }
+        constexpr int HG = BPW > 4 ? (BPW + 1) / 2 : BPW;  // bricks whose faces are in flight at once
         if (it > 0) {  // the first direction is r itself
 #pragma unroll
             for (int b = 0; b < BPW; ++b)
@@ -310,26 +413,61 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
                 for (int k = 0; k < 8; ++k) s[b][k] = r[b][k] + bt * s[b][k];
         }
 #pragma unroll
-        for (int b = 0; b < BPW; ++b) {
-            T *hp = halo[wave * BPW + b];
+        for (int g = 0; g < BPW; g += HG) {
+            __builtin_amdgcn_sched_barrier(0);
+            T hr[HG][6];
 #pragma unroll
-            for (int f = 0; f < (Y > 1 ? 4 : 2); ++f) hp[64 * f + lane] = hr[b][f] + bt * hp[64 * f + lane];
-            hz[b][0] = hr[b][4] + bt * hz[b][0];
-            hz[b][1] = hr[b][5] + bt * hz[b][1];
+            for (int u = 0; u < HG; ++u) {
+                const int b = g + u < BPW ? g + u : g;
+                int n[6];
+#pragma unroll
+                for (int f = 0; f < 6; ++f) n[f] = here(nb[b][f]);
+                hr[u][0] = n[0] >= 0 && xl ? ld_face(faces + (int64_t)n[0] * 384 + 64 + lane) : T(0);
+                hr[u][1] = n[1] >= 0 && xl ? ld_face(faces + (int64_t)n[1] * 384 + lane) : T(0);
+                hr[u][2] = hr[u][3] = T(0);
+                if constexpr (Y > 1) {
+                    hr[u][2] = n[2] >= 0 ? ld_face(faces + (int64_t)n[2] * 384 + 192 + lane) : T(0);
+                    hr[u][3] = n[3] >= 0 ? ld_face(faces + (int64_t)n[3] * 384 + 128 + lane) : T(0);
+                }
+                hr[u][4] = n[4] >= 0 ? ld_face(faces + (int64_t)n[4] * 384 + 320 + lane) : T(0);
+                hr[u][5] = n[5] >= 0 ? ld_face(faces + (int64_t)n[5] * 384 + 256 + lane) : T(0);
+            }
+#pragma unroll
+            for (int u = 0; u < HG; ++u) {
+                if (g + u >= BPW) continue;
+                const int b = g + u < BPW ? g + u : g;
+                T *hp = halo[wave * BPW + b];
+#pragma unroll
+                for (int f = 0; f < (Y > 1 ? 4 : 2); ++f) hp[64 * f + lane] = hr[u][f] + bt * hp[64 * f + lane];
+                hz[b][0] = hr[u][4] + bt * hz[b][0];
+                hz[b][1] = hr[u][5] + bt * hz[b][1];
+            }
         }
         wave_lds_fence();
         acc = 0.0;
 #pragma unroll
         for (int b = 0; b < BPW; ++b) {
             __builtin_amdgcn_sched_barrier(0);  // one brick at a time: registers
-            const int slot = here(slot0) + b;
+            const int slot = here(slot0) + stride * b;
             if (slot >= op.n_active) continue;
             const T *hp = halo[wave * BPW + b];
-            const T kv = op.kappa[slot];
-            if (kv != T(0)) {
-                const T kd = UNIT ? T(0) : op.kdiag[slot];
+            const bool next = !CREG && b + 1 < BPW && slot + stride < op.n_active && kap[b + 1 < BPW ? b + 1 : b] == T(0);
+            int nn[6];
+            if constexpr (!CREG) {
+#pragma unroll
+                for (int f = 0; f < 6; ++f) nn[f] = here(nb[b + 1 < BPW ? b + 1 : b][f]);
+            }
+            if (kap[b] != T(0)) {
+                if (next) {
+                    const CouplingAt<T, UNIT, BX> at(op, slot + stride, nn, lane);
+                    at.load(cpl[0], 0);
+                    at.load(cpl[0], 1);
+                }
+                const T kv = kap[b];
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
+                    if constexpr (!CREG)
+                        if ((k & 1) == 0) __builtin_amdgcn_sched_barrier(0);
                     const T sk = s[b][k];
                     const T hx = hp[hxo + Y * k];
                     const T lf = lane_shift<0x138>(sk), rt = lane_shift<0x130>(sk);  // every lane takes part
@@ -343,55 +481,55 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
                     }
                     const T zm = k > 0 ? s[b][k - 1] : hz[b][0];
                     const T zp = k < 7 ? s[b][k + 1] : hz[b][1];
-                    T qv = UNIT ? sk : kd * sk;
+                    T qv = UNIT ? sk : kd[b] * sk;
                     qv -= kv * xm + kv * xp + kv * ym + kv * yp + kv * zm + kv * zp;
                     q[b][k] = qv;
-                    acc += (double)sk * (double)qv;
+                    add_here<!CREG>(acc, (double)sk * (double)qv);
                 }
                 continue;
             }
-            // the couplings of the other bricks are read again every iteration (they stay in
-            // the L2s); those of the +x / +y / +z faces live in the neighbour bricks
-            const T *cx = op.cx + (int64_t)slot * NT, *cy = op.cy + (int64_t)slot * NT, *cz = op.cz + (int64_t)slot * NT;
-            const T *dg = UNIT ? nullptr : op.diag + (int64_t)slot * NT;
-            const int n[6] = {0, here(nb[b][1]), 0, here(nb[b][3]), 0, here(nb[b][5])};
-            // a cell's +x / +y coupling is its neighbour's low one, in the next brick for the edge
-            // lanes (without one the halo value is 0, and any finite coupling will do)
-            const T *cxn = cx + (xhi ? lane : lane + 1), *cyn = cy + (yhi ? lane : lane + X);
-            if (n[1] >= 0) cxn = xhi ? op.cx + (int64_t)n[1] * NT + X * j : cxn;
-            if (n[3] >= 0) cyn = yhi ? op.cy + (int64_t)n[3] * NT + i : cyn;
-            const T czh = n[5] >= 0 ? (op.cz + (int64_t)n[5] * NT)[lane] : T(0);
-            T czk = cz[lane];
+            Couplings<T, UNIT> &c = cpl[CREG ? b : 0];
+            int n[6];
+#pragma unroll
+            for (int f = 0; f < 6; ++f) n[f] = CREG ? -1 : here(nb[b][f]);
+            const CouplingAt<T, UNIT, BX> at(op, slot, n, lane);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                if constexpr (BPW * sizeof(T) > 8)
-                    if ((k & 1) == 0) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (!CREG)
+                    if ((k & 1) == 0) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (k < 6) {
+                            at.load(c, k + 2 < 8 ? k + 2 : 7);
+                            at.load(c, k + 3 < 8 ? k + 3 : 7);
+                        }
+                    }
                 const T sk = s[b][k];
-                const T cxv = cx[lane + 64 * k];
-                const T cyv = Y > 1 ? cy[lane + 64 * k] : T(0);
-                const T czp = k < 7 ? cz[lane + 64 * (k + 1)] : czh;
                 const T hx = hp[hxo + Y * k];
                 const T lf = lane_shift<0x138>(sk), rt = lane_shift<0x130>(sk);
                 const T xm = xlo ? hx : lf, xp = xhi ? hx : rt;
-                const T cxp = cxn[64 * k];
-                T ym = T(0), yp = T(0), cyp = T(0);
+                T ym = T(0), yp = T(0);
                 if constexpr (Y > 1) {
                     const T hy = hp[hyo + X * k];
                     const T dn = lane_get(sk, lane - X), up = lane_get(sk, lane + X);
                     ym = ylo ? hy : dn;
                     yp = yhi ? hy : up;
-                    cyp = cyn[64 * k];
                 }
                 const T zm = k > 0 ? s[b][k - 1] : hz[b][0];
                 const T zp = k < 7 ? s[b][k + 1] : hz[b][1];
-                T qv = UNIT ? sk : dg[lane + 64 * k] * sk;
-                qv -= cxv * xm + cxp * xp + cyv * ym + cyp * yp + czk * zm + czp * zp;
-                czk = czp;
+                const T czp = k < 7 ? c.z[k < 7 ? k + 1 : 7] : c.top;
+                T qv = UNIT ? sk : c.d[UNIT ? 0 : k] * sk;
+                qv -= c.x[k] * xm + c.xp[k] * xp + c.y[k] * ym + c.yp[k] * yp + c.z[k] * zm + czp * zp;
                 q[b][k] = qv;
-                acc += (double)sk * (double)qv;
+                add_here<!CREG>(acc, (double)sk * (double)qv);
+                if constexpr (!CREG)
+                    if (k == 5 && next) {
+                        const CouplingAt<T, UNIT, BX> an(op, slot + stride, nn, lane);
+                        an.load(cpl[0], 0);
+                        an.load(cpl[0], 1);
+                    }
             }
         }
-        if (!(alive = exchange(acc, 0.0, e++, slots, xl_, sigma, mx))) break;
+        if (!(alive = exchange<false>(acc, 0.0, e++, slots, xl_, sigma, mx))) break;
         if (!(sigma > 0.0)) {
             status = sigma != sigma ? SHK_NAN : SHK_BREAKDOWN;
             break;
@@ -404,7 +542,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
 #pragma unroll
         for (int b = 0; b < BPW; ++b) {
             __builtin_amdgcn_sched_barrier(0);
-            const int slot = here(slot0) + b;
+            const int slot = here(slot0) + stride * b;
             if (slot >= op.n_active) continue;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -414,10 +552,16 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
                     xs[((wave * BPW + b) * 8 + k) * 64 + lane] += a * s[b][k];
                 const T rv = r[b][k] - a * q[b][k];
                 r[b][k] = rv;
-                acc += (double)rv * (double)rv;
+                add_here<!CREG>(acc, (double)rv * (double)rv);
                 if constexpr (SCALED) {
-                    const double sg = (sig + (int64_t)slot * NT)[lane + 64 * k];
-                    if (sg > 0.0) mx = fmax(mx, fabs((double)rv) / sg);
+                    T is;
+                    if constexpr (CREG) {
+                        is = isg[b][k];
+                    } else {
+                        const double sg = (sig + (int64_t)slot * NT)[lane + 64 * k];
+                        is = sg > 0.0 ? (T)(1.0 / sg) : T(0);
+                    }
+                    mx = fmax(mx, fabs((double)(rv * is)));
                 } else {
                     mx = fmax(mx, fabs((double)rv));
                 }
@@ -428,7 +572,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
             publish<T, BX>(r[b], scr, faces + (int64_t)slot * 384, lane, n);
         }
         double rho_new;
-        if (!(alive = exchange(acc, mx, e++, slots, xl_, rho_new, rn))) break;
+        if (!(alive = exchange<true>(acc, mx, e++, slots, xl_, rho_new, rn))) break;
         // the stop test of pcg_solver.h:281-284 and beta of :287-289 (as direction_step)
         if (rn <= tol_abs) {
             done = true;
@@ -445,7 +589,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
     }
 #pragma unroll
     for (int b = 0; b < BPW; ++b) {
-        const int slot = slot0 + b;
+        const int slot = slot0 + stride * b;
         if (slot >= op.n_active) continue;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
@@ -475,7 +619,7 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
 
 __global__ void k_resident_begin(SolveState *st, unsigned long long *slots) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 4 * 2 * kMaxWg) slots[i] = kEmpty;
+    if (i < kSlotWords) slots[i] = kEmpty;
     if (i == 0) st->aborted = 0;
 }
 
@@ -527,7 +671,7 @@ void launch_bpw(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, con
 
 }  // namespace
 
-size_t resident_slot_words() { return 4 * 2 * kMaxWg; }
+size_t resident_slot_words() { return kSlotWords; }
 
 template <class T>
 ResidentPlan resident_plan(const BrickOp<T> &op, int device, int cus) {
@@ -561,7 +705,7 @@ hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &
         bud.cv.wait(lk, [&] { return bud.used + p.blocks <= cus; });
         bud.used += p.blocks;
     }
-    hipLaunchKernelGGL(k_resident_begin, dim3((4 * 2 * kMaxWg + 255) / 256), dim3(256), 0, st, state, slots);
+    hipLaunchKernelGGL(k_resident_begin, dim3((kSlotWords + 255) / 256), dim3(256), 0, st, state, slots);
     const bool unit = op.diag == nullptr, flat = op.bx == 64;
     if constexpr (sizeof(T) == 4) {
         if (unit && flat)

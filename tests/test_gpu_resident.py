@@ -73,7 +73,9 @@ def test_resident_matches_two_kernels(shape, precision, precond):
         bmax = float(sy["rhs"].abs().max())
         # the recurrence residual of an FP64 solve differs from the true one by rounding
         assert float(_apply(sy, xs[0] - xs[1]).abs().max()) <= 2 * tol * bmax * (1 + 1e-3)
-        assert abs(its[0] - its[1]) <= max(3, 0.05 * its[1])
+        # 20 random renumberings of the unknowns alone spread the plain CG of the small shapes
+        # over 246..270, 558..593 and 1322..1397 iterations (the oracle's CPU solve)
+        assert abs(its[0] - its[1]) <= max(3, 0.1 * its[1])
 
 
 def test_resident_outcomes():
