@@ -208,6 +208,8 @@ struct UnetNet {
          *dcat2 = nullptr, *dbott = nullptr, *dp3 = nullptr, *de2 = nullptr, *dp2 = nullptr, *de1 = nullptr,
          *dp1 = nullptr, *de0 = nullptr, *tmp = nullptr;
     float *u = nullptr, *du = nullptr;
+    float *wpart = nullptr;  // partial weight gradients of one layer
+    int64_t wpart_cap = 0;
     // fine-level training work arrays
     int64_t fine_cap = 0;
     float *fz = nullptr, *fe = nullptr, *fae = nullptr, *ftmp = nullptr;
@@ -266,6 +268,18 @@ int ensure_grid(UnetNet *n, Grid3 m) {
     return SHK_OK;
 }
 
+// scratch of the largest layer's weight gradient on the current grid
+int ensure_wgrad(UnetNet *n) {
+    static const int level[kLayers] = {0, 1, 2, 3, 2, 1, 0, 0};
+    int64_t want = 0;
+    for (int l = 0; l < kLayers; ++l)
+        want = std::max(want, conv_wgrad_part_elems(n->L[level[l]], kSpec[l].cin, kSpec[l].cout));
+    if (want <= n->wpart_cap) return SHK_OK;
+    UHIP(n, dalloc(n->wpart, (size_t)want));
+    n->wpart_cap = want;
+    return SHK_OK;
+}
+
 int ensure_fine(UnetNet *n, int64_t nf) {
     if (nf <= n->fine_cap) return SHK_OK;
     UHIP(n, dalloc(n->fz, (size_t)nf));
@@ -303,7 +317,8 @@ void dgrad(UnetNet *n, int l, Grid3 g, const bf16 *dz, bf16 *dx) {
     launch_conv_fwd(n->stream, g, dz, kSpec[l].cout, n->pkt[l], nullptr, kSpec[l].cin, false, dx, nullptr);
 }
 void wgrad(UnetNet *n, int l, Grid3 g, const bf16 *x, const bf16 *dz) {
-    launch_conv_wgrad(n->stream, g, x, kSpec[l].cin, dz, kSpec[l].cout, n->grad + n->woff[l], n->grad + n->boff[l]);
+    launch_conv_wgrad(n->stream, g, x, kSpec[l].cin, dz, kSpec[l].cout, n->grad + n->woff[l], n->grad + n->boff[l],
+                      n->wpart);
 }
 
 // forward on the features already in n->feat; u = network output (FP32, level 0)
@@ -453,6 +468,7 @@ void unet_net_destroy(UnetNet *n) {
     for (auto p : acts) dfree(*p);
     dfree(n->u);
     dfree(n->du);
+    dfree(n->wpart);
     dfree(n->fz);
     dfree(n->fe);
     dfree(n->fae);
@@ -541,6 +557,7 @@ int unet_net_train(UnetNet *n, Grid3 fine, const float *r, const float *mask, co
                            n->ftmp, n->fae);
     }
     launch_prolong_bwd(n->stream, n->L[0], n->fae, mask, rms, n->du);
+    if ((rc = ensure_wgrad(n))) return rc;
     backward(n);
     if (lr > 0.0f) {
         n->step += 1;
@@ -1224,8 +1241,14 @@ int shk_nn_conv3d_backward(int nx, int ny, int nz, const void *x, int cin, const
         if (e != hipSuccess) return SHK_HIP_ERROR;
     }
     if (dw) {
-        launch_conv_wgrad(nullptr, g, static_cast<const bf16 *>(x), cin, static_cast<const bf16 *>(dz), cout, dw, db);
-        if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) return SHK_HIP_ERROR;
+        float *part = nullptr;
+        if (hipMalloc((void **)&part, sizeof(float) * conv_wgrad_part_elems(g, cin, cout)) != hipSuccess)
+            return SHK_OUT_OF_MEMORY;
+        launch_conv_wgrad(nullptr, g, static_cast<const bf16 *>(x), cin, static_cast<const bf16 *>(dz), cout, dw, db,
+                          part);
+        const bool bad = hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess;
+        (void)hipFree(part);
+        if (bad) return SHK_HIP_ERROR;
     }
     return SHK_OK;
 }

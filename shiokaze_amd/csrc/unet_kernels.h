@@ -101,9 +101,10 @@ void launch_conv_head(hipStream_t st, Grid3 g, const bf16 *x, const uint32_t *wp
 void launch_head_pack(hipStream_t st, const float *w, int cout, uint32_t *wpk);
 
 // dw[tap][ci][co] += sum_v x[v + tap][ci] * dz[v][co]; db[co] += sum_v dz[v][co]
-// (FP32 atomics, split over voxel chunks).
+// (db nullable; part: conv_wgrad_part_elems floats of scratch).  cin a multiple of 8, cout of 16.
+int64_t conv_wgrad_part_elems(Grid3 g, int cin, int cout);
 void launch_conv_wgrad(hipStream_t st, Grid3 g, const bf16 *x, int cin, const bf16 *dz, int cout, float *dw,
-                       float *db);
+                       float *db, float *part);
 
 // dz = dy * (y > 0) in place on dy (ReLU backward), n elements.
 void launch_relu_bwd(hipStream_t st, int64_t n, const bf16 *y, bf16 *dy);

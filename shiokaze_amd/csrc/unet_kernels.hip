@@ -789,83 +789,167 @@ __global__ void k_head_pack(const float *__restrict__ w, int cout, uint32_t *__r
 
 // ---------------------------------------------------------------- weight gradient
 
-// One wave per (voxel chunk, tap, 16x16 (co, ci) tile): D[co][ci] = sum over the
-// chunk's voxels of dz[v][co] * x[v + tap][ci]; the tile is added with FP32 atomics.
-constexpr int kWgradChunk = 512;  // voxels per wave (16 MFMA steps of 32)
+// dW[tap][ci][co] = sum over the voxels of x[v + tap][ci] dz[v][co] as MFMAs whose K is the
+// voxels.  What bounded the one-wave-per-tap form was its loads: a channels-last tensor
+// holds a fragment's eight voxels of one channel eight pixels apart, 16 two-byte loads per
+// MFMA, every voxel read again for each of the 27 taps.  Here a block transposes a tile of
+// dz (16 outputs) and of x with its halo (16 inputs) once through LDS, voxel pairs of one
+// channel to a dword, and each of its four waves keeps all 27 taps' 16 x 16 accumulators:
+// a row of x in LDS serves its three x taps from six dwords (the shifted fragments are
+// funnel shifts of the aligned one).  K = 32 voxels is XW consecutive voxels of 32 / XW rows
+// (XW 32, 16 or 8 by the grid's x extent, whichever wastes least, so that the deep levels'
+// 16^3 and 8^3 grids fill their fragments).  The blocks of one (ci, co) tile take every
+// splits-th spatial tile and write their sums to `part`; k_wgrad_reduce adds them in order,
+// so the gradient no longer depends on the order of atomics.  The bias gradient is one more
+// MFMA with ones.  Training sample at 128^3: the eight weight gradients 1566 -> 214 us (46 of them the reduction), the
+// bias gradients (1024 blocks of atomics on 16..128 addresses) 2144 us -> none of their own.
+template <int XW>
+struct WgradTile {
+    static constexpr int KR = 32 / XW;                 // rows of one K step
+    static constexpr int RY = XW == 32 ? 4 : 8, RZ = XW == 8 ? 8 : 4;  // output rows: 16 K steps
+    static constexpr int HR = (RY + 2) * (RZ + 2);     // rows of x with the halo
+    static constexpr int PW = XW / 2 + 2;              // dwords of a row: voxels -2 .. XW + 1
+    static constexpr int SX = HR * PW + 2;             // per channel; 2 mod 4: 16 channels on distinct banks
+    static constexpr int SZ = RY * RZ * XW / 2 + 4;    // per output channel of dz; 16-byte rows
+    static constexpr int kLds = 16 * (SX + SZ);        // dwords
+    static_assert(SX % 4 == 2 && SZ % 8 == 4 && RY * RZ / KR == 16, "layout");
+};
+constexpr int kWgradTaps = 28;  // 27 taps and the bias
 
-__global__ __launch_bounds__(64) void k_conv_wgrad(Grid3 g, const uint16_t *__restrict__ x, int cin,
-                                                   const uint16_t *__restrict__ dz, int cout, float *__restrict__ dw) {
-    const int lane = threadIdx.x;
-    const int n = lane & 15, kq = lane >> 4;
-    const int64_t nvox = g.vox();
-    const int64_t c0 = (int64_t)blockIdx.x * kWgradChunk;
-    const int tap = blockIdx.y;
-    const int ci_tiles = (cin + 15) / 16;
-    const int co0 = (blockIdx.z / ci_tiles) * 16;
-    const int ci0 = (blockIdx.z % ci_tiles) * 16;
-    int dx, dy, dz_;
-    tap_offset(tap, dx, dy, dz_);
-    const int co = co0 + n;  // A row of this lane
-    const int ci = ci0 + n;  // B column of this lane
-    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int step = 0; step < kWgradChunk; step += 32) {
-        const int64_t vs = c0 + step + 8 * kq;
-        Frag a, b;
-        a.u = make_uint4(0u, 0u, 0u, 0u);
-        b.u = make_uint4(0u, 0u, 0u, 0u);
-        uint16_t av[8], bv[8];
-        int64_t v = vs;
-        int vx = (int)(v % g.nx), vy = (int)((v / g.nx) % g.ny), vz = (int)(v / ((int64_t)g.nx * g.ny));
+__device__ inline uint4 load8(const uint16_t *p, int vec) {
+    if (vec) return *reinterpret_cast<const uint4 *>(p);
+    return make_uint4(p[0] | ((uint32_t)p[1] << 16), p[2] | ((uint32_t)p[3] << 16), p[4] | ((uint32_t)p[5] << 16),
+                      p[6] | ((uint32_t)p[7] << 16));
+}
+// eight channels of voxels a and b -> eight dwords (a | b << 16) at stride
+__device__ inline void put_pairs(uint32_t *dst, int stride, uint4 a, uint4 b) {
+    const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            av[j] = 0;
-            bv[j] = 0;
-            if (v < nvox) {
-                av[j] = dz[v * cout + co];
-                const int xx = vx + dx, yy = vy + dy, zz = vz + dz_;
-                if (ci < cin && xx >= 0 && xx < g.nx && yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz)
-                    bv[j] = x[(((int64_t)zz * g.ny + yy) * g.nx + xx) * cin + ci];
-            }
-            ++v;
-            if (++vx == g.nx) {
-                vx = 0;
-                if (++vy == g.ny) {
-                    vy = 0;
-                    ++vz;
-                }
-            }
-        }
-        a.u.x = av[0] | ((uint32_t)av[1] << 16);
-        a.u.y = av[2] | ((uint32_t)av[3] << 16);
-        a.u.z = av[4] | ((uint32_t)av[5] << 16);
-        a.u.w = av[6] | ((uint32_t)av[7] << 16);
-        b.u.x = bv[0] | ((uint32_t)bv[1] << 16);
-        b.u.y = bv[2] | ((uint32_t)bv[3] << 16);
-        b.u.z = bv[4] | ((uint32_t)bv[5] << 16);
-        b.u.w = bv[6] | ((uint32_t)bv[7] << 16);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc, 0, 0, 0);
+    for (int c = 0; c < 4; ++c) {
+        dst[(2 * c) * stride] = (av[c] & 0xffffu) | (bv[c] << 16);
+        dst[(2 * c + 1) * stride] = (av[c] >> 16) | (bv[c] & 0xffff0000u);
     }
-    // lane holds D[co0 + 4*kq + j][ci0 + n]
-    if (ci < cin) {
+}
+
+template <int XW>
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad(Grid3 g, const uint16_t *__restrict__ x, int cin, int xvec,
+                                                       const uint16_t *__restrict__ dz, int cout, int dvec, int tx,
+                                                       int ty, int ntiles, float *__restrict__ part) {
+    using W = WgradTile<XW>;
+    constexpr int RY = W::RY, RZ = W::RZ, PW = W::PW, SX = W::SX, SZ = W::SZ, KR = W::KR;
+    __shared__ __attribute__((aligned(16))) uint32_t lds[W::kLds];
+    uint32_t *zs = lds, *xs = lds + 16 * SZ;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 15, kq = lane >> 4;
+    const int ci_tiles = (cin + 15) / 16;
+    const int co0 = (blockIdx.y / ci_tiles) * 16, ci0 = (blockIdx.y % ci_tiles) * 16;
+    f32x4 acc[27], accb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int cc = co0 + 4 * kq + j;
-            atomicAdd(&dw[((int64_t)tap * cin + ci) * cout + cc], acc[j]);
+    for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    Frag ones;
+    ones.u = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int x0 = (tile % tx) * XW, y0 = (tile / tx % ty) * RY, z0 = (tile / (tx * ty)) * RZ;
+        __syncthreads();  // the previous tile's fragments have been read
+        for (int t = tid; t < RY * RZ * XW; t += 256) {  // (voxel pair, 8 channels) of dz
+            const int g8 = t & 1, m = (t >> 1) % (XW / 2), row = (t >> 1) / (XW / 2);
+            const int yy = y0 + row % RY, zz = z0 + row / RY, xx = x0 + 2 * m;
+            uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+            if (yy < g.ny && zz < g.nz) {
+                const uint16_t *p = dz + (((int64_t)zz * g.ny + yy) * g.nx + xx) * cout + co0 + 8 * g8;
+                if (xx < g.nx) a = load8(p, dvec);
+                if (xx + 1 < g.nx) b = load8(p + cout, dvec);
+            }
+            put_pairs(zs + (8 * g8) * SZ + row * (XW / 2) + m, SZ, a, b);
+        }
+#pragma unroll 2
+        for (int t = tid; t < W::HR * PW * 2; t += 256) {
+            const int g8 = t & 1, m = (t >> 1) % PW, row = (t >> 1) / PW;
+            const int yy = y0 - 1 + row % (RY + 2), zz = z0 - 1 + row / (RY + 2), xx = x0 - 2 + 2 * m;
+            uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+            if (yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz && ci0 + 8 * g8 < cin) {
+                const int64_t v = ((int64_t)zz * g.ny + yy) * g.nx;
+                if (xx >= 0 && xx < g.nx) a = load8(x + (v + xx) * cin + ci0 + 8 * g8, xvec);
+                if (xx + 1 >= 0 && xx + 1 < g.nx) b = load8(x + (v + xx + 1) * cin + ci0 + 8 * g8, xvec);
+            }
+            put_pairs(xs + (8 * g8) * SX + row * PW + m, SX, a, b);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+            const int r = (4 * wave + q) * KR + kq / (XW / 8), xo = (kq % (XW / 8)) * 4;  // row, first dword
+            Frag a;
+            a.u = *reinterpret_cast<const uint4 *>(zs + n * SZ + r * (XW / 2) + xo);
+            const uint32_t *xr = xs + n * SX + ((r / RY) * (RY + 2) + r % RY) * PW + xo;
+            if (ci0 == 0) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, ones.v, accb, 0, 0, 0);
+#pragma unroll
+            for (int dzz = 0; dzz < 3; ++dzz)
+#pragma unroll
+                for (int dyy = 0; dyy < 3; ++dyy) {
+                    const uint2 *p = reinterpret_cast<const uint2 *>(xr + (dzz * (RY + 2) + dyy) * PW);
+                    const uint2 e0 = p[0], e1 = p[1], e2 = p[2];
+                    const uint32_t d[6] = {e0.x, e0.y, e1.x, e1.y, e2.x, e2.y};
+                    const int t = 9 * dzz + 3 * dyy;
+                    Frag b;
+                    b.u = make_uint4(__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
+                                     __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(d[4], d[3], 16));
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[t], 0, 0, 0);
+                    b.u = make_uint4(d[1], d[2], d[3], d[4]);
+                    acc[t + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[t + 1], 0, 0, 0);
+                    b.u = make_uint4(__builtin_amdgcn_alignbit(d[2], d[1], 16), __builtin_amdgcn_alignbit(d[3], d[2], 16),
+                                     __builtin_amdgcn_alignbit(d[4], d[3], 16), __builtin_amdgcn_alignbit(d[5], d[4], 16));
+                    acc[t + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[t + 2], 0, 0, 0);
+                }
+        }
+    }
+    // the four waves' sums, seven taps at a time; a lane holds D[co0 + 4 kq + j][ci0 + n]
+    float *out = part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (kWgradTaps * 256);
+    float *buf = reinterpret_cast<float *>(lds);
+#pragma unroll
+    for (int t0 = 0; t0 < kWgradTaps; t0 += 7) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            *reinterpret_cast<f32x4 *>(buf + (wave * 7 + u) * 256 + n * 16 + 4 * kq) = t0 + u < 27 ? acc[t0 + u < 27 ? t0 + u : 0] : accb;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 7; ++u) {
+            float s = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) s += buf[(w * 7 + u) * 256 + tid];
+            out[(t0 + u) * 256 + tid] = s;
         }
     }
 }
 
-__global__ __launch_bounds__(256) void k_bias_grad(int64_t nvox, const uint16_t *__restrict__ dz, int cout,
-                                                   float *__restrict__ db) {
-    // thread (block-local) t handles channel t % cout over a strided set of voxels
-    const int c = threadIdx.x % cout;
-    const int lanes_per_c = blockDim.x / cout;
-    const int sub = threadIdx.x / cout;
-    if (sub >= lanes_per_c) return;
-    float acc = 0.0f;
-    for (int64_t v = (int64_t)blockIdx.x * lanes_per_c + sub; v < nvox; v += (int64_t)gridDim.x * lanes_per_c)
-        acc += bits_f32(dz[v * cout + c]);
-    atomicAdd(&db[c], acc);
+// dw[tap][ci][co] += the sums of the tile's blocks; the bias from its ones column.  Sixteen
+// slices of the blocks (every 16th one) are summed side by side, four elements per thread,
+// and added in order: with one pair of tiles there are only 28 blocks, and one thread per
+// element walking up to 512 partials alone took as long as the gradient itself.
+constexpr int kWgradSlices = 16;
+__global__ __launch_bounds__(64 * kWgradSlices) void k_wgrad_reduce(const float *__restrict__ part, int splits, int cin,
+                                                                     int cout, float *__restrict__ dw,
+                                                                     float *__restrict__ db) {
+    __shared__ f32x4 sums[kWgradSlices][64];
+    const int tap = blockIdx.x, ci_tiles = (cin + 15) / 16;
+    const int co0 = (blockIdx.y / ci_tiles) * 16, ci0 = (blockIdx.y % ci_tiles) * 16;
+    const int e = threadIdx.x & 63, slice = threadIdx.x >> 6;
+    if (tap == 27 && (!db || ci0 != 0)) return;  // the whole block
+    const float *p = part + (int64_t)blockIdx.y * splits * (kWgradTaps * 256) + tap * 256 + 4 * e;
+    f32x4 s = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int k = slice; k < splits; k += kWgradSlices)
+        s += *reinterpret_cast<const f32x4 *>(p + (int64_t)k * (kWgradTaps * 256));
+    sums[slice][e] = s;
+    __syncthreads();
+    const int ci = ci0 + e / 4, co = co0 + 4 * (e % 4);
+    if (slice != 0 || ci >= cin || (tap == 27 && ci != 0)) return;
+    s = sums[0][e];
+#pragma unroll
+    for (int k = 1; k < kWgradSlices; ++k) s += sums[k][e];
+    float *out = tap == 27 ? db + co : dw + ((int64_t)tap * cin + ci) * cout + co;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] += s[j];
 }
 
 // ---------------------------------------------------------------- elementwise / resampling
@@ -1670,16 +1754,44 @@ void launch_conv_rows(hipStream_t st, Grid3 g, const bf16 *x, int cin, const bf1
                            relu ? 1 : 0, U(y), xc, c1, tx, ty, stop);
 }
 
+namespace {
+struct WgradPlan {
+    int xw, tx, ty, tiles, splits, pairs;
+};
+// The voxels of a K step along x: 32, or 16 or 8 where that pads the rows less (rows of 24:
+// 24 instead of 32).  Blocks: about three per CU over the (ci, co) tiles, so that the
+// partial sums (28 KB per block) stay small beside the tensors.
+WgradPlan wgrad_plan(Grid3 g, int cin, int cout) {
+    WgradPlan p;
+    p.xw = 32;
+    for (int w : {16, 8})
+        if ((g.nx + w - 1) / w * w < (g.nx + p.xw - 1) / p.xw * p.xw) p.xw = w;
+    const int ry = p.xw == 32 ? 4 : 8, rz = p.xw == 8 ? 8 : 4;
+    p.tx = (g.nx + p.xw - 1) / p.xw;
+    p.ty = (g.ny + ry - 1) / ry;
+    p.tiles = p.tx * p.ty * ((g.nz + rz - 1) / rz);
+    p.pairs = (cout / 16) * ((cin + 15) / 16);
+    const int want = (2 * 256 + p.pairs - 1) / p.pairs;
+    p.splits = p.tiles < want ? p.tiles : want;
+    return p;
+}
+}  // namespace
+
+int64_t conv_wgrad_part_elems(Grid3 g, int cin, int cout) {
+    const WgradPlan p = wgrad_plan(g, cin, cout);
+    return (int64_t)p.pairs * p.splits * (kWgradTaps * 256);
+}
+
 void launch_conv_wgrad(hipStream_t st, Grid3 g, const bf16 *x, int cin, const bf16 *dz, int cout, float *dw,
-                       float *db) {
-    const int64_t chunks = (g.vox() + kWgradChunk - 1) / kWgradChunk;
-    const dim3 grid((unsigned)chunks, 27, (unsigned)((cout / 16) * ((cin + 15) / 16)));
-    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(64), 0, st, g, U(x), cin, U(dz), cout, dw);
-    if (db) {
-        const int64_t nb = (g.vox() + 255) / 256;
-        hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)(nb < 1024 ? nb : 1024)), dim3(256), 0, st, g.vox(), U(dz),
-                           cout, db);
-    }
+                       float *db, float *part) {
+    const WgradPlan p = wgrad_plan(g, cin, cout);
+    const dim3 grid((unsigned)p.splits, (unsigned)p.pairs);
+    // 16-byte loads where the tensors allow them (cin and cout are multiples of 8)
+    const int xvec = reinterpret_cast<uintptr_t>(x) % 16 == 0, dvec = reinterpret_cast<uintptr_t>(dz) % 16 == 0;
+    auto kern = p.xw == 32 ? k_conv_wgrad<32> : (p.xw == 16 ? k_conv_wgrad<16> : k_conv_wgrad<8>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, g, U(x), cin, xvec, U(dz), cout, dvec, p.tx, p.ty, p.tiles, part);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(kWgradTaps, (unsigned)p.pairs), dim3(64 * kWgradSlices), 0, st, part,
+                       p.splits, cin, cout, dw, db);
 }
 
 void launch_relu_bwd(hipStream_t st, int64_t n, const bf16 *y, bf16 *dy) {
