@@ -15,11 +15,13 @@
 // 50-100): fp contraction is off and float quotients are taken in double and rounded
 // once, which equals the correctly rounded float quotient.  The results are bit-for-
 // bit those of the reference's arithmetic on the same inputs.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdint>
 #include <initializer_list>
 
+#include "bands.h"
 #include "ctx_internal.h"
 #include "shk_common.h"
 
@@ -30,6 +32,8 @@ struct LiquidWork {
     DevBuf<uint8_t> band[3];
     DevBuf<unsigned long long> count;
     DevBuf<unsigned int> slots;
+    DevBuf<uint32_t> list;        // a narrow band's cells (bands.h)
+    DevBuf<unsigned int> counts;  // its length, counted cells
     DevBuf<double> part;
     std::vector<double> h_part;
     void release() {
@@ -42,6 +46,8 @@ struct LiquidWork {
         }
         count.release();
         slots.release();
+        list.release();
+        counts.release();
         part.release();
     }
 };
@@ -86,25 +92,13 @@ __device__ inline float rd(const float *a, const uint8_t *m, int64_t q) {
     return act ? v : 0.0f;
 }
 
-// (i, j, k) of a linear index with 32-bit unsigned arithmetic (shk_create bounds the
-// cells by 2^31, so every face array has fewer than 2^32 entries)
-// Exact division of a 32-bit index by an extent n without a divide sequence:
-// floor(q / n) = floor(m q / 2^64) with m = ceil(2^64 / n) for every 32-bit q and
-// 2 <= n < 2^32 (Lemire, Kaser and Kurz, "Faster remainder by direct computation",
-// 2019).  m is computed on the host; n = 1 takes q itself.
-struct Div32 {
-    uint32_t n;
-    uint64_t m;
-};
-inline Div32 div32(int n) { return Div32{(uint32_t)n, n > 1 ? ~0ull / (uint64_t)n + 1 : 0ull}; }
-__device__ inline uint32_t quot(uint32_t q, Div32 d) {
-    return d.n > 1 ? (uint32_t)__umul64hi(d.m, (uint64_t)q) : q;
+// off the mask: the array's background value
+__device__ inline float rd_bg(const float *a, const uint8_t *m, int64_t q, float bg) {
+    const float v = a[q];
+    const uint8_t act = m ? m[q] : 1;
+    return act ? v : bg;
 }
 
-// the x and y extents of an index space (a face or cell array), for decompose
-struct Split {
-    Div32 x, y;
-};
 inline Split split_of(FS s) { return Split{div32(s.nx), div32(s.ny)}; }
 struct Split3 {  // the three face arrays
     Split a[3];
@@ -112,14 +106,6 @@ struct Split3 {  // the three face arrays
 inline Split cells_split(const Dims &d) { return split_of(FS{d.nx, d.ny, d.nz}); }
 inline Split3 faces_split(const Dims &d) {
     return Split3{{split_of(face_fs(d, 0)), split_of(face_fs(d, 1)), split_of(face_fs(d, 2))}};
-}
-
-__device__ inline void decompose(int64_t q, Split sp, int &i, int &j, int &k) {
-    const uint32_t u = (uint32_t)q;
-    const uint32_t t = quot(u, sp.x);
-    i = (int)(u - t * sp.x.n);
-    k = (int)quot(t, sp.y);
-    j = (int)(t - (uint32_t)k * sp.y.n);
 }
 
 __device__ inline int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -223,7 +209,7 @@ __device__ inline double weno6(double x, const double f[6]) {
 // WENO3::interpolate(array, p), order 6 (WENO3.h:92-122): the position clamped into the
 // array, then interp6 along x for each of the 6 x 6 rows around it, along y, along z,
 // every read clamped to the array (m == nullptr reads every value as stored)
-__device__ inline double weno3(const float *a, const uint8_t *m, FS s, const double p[3]) {
+__device__ inline double weno3(const float *a, const uint8_t *m, FS s, const double p[3], float bg = 0.0f) {
 #pragma clang fp contract(off)
     const double x = fmax(0.0, fmin(s.nx - 1., p[0]));
     const double y = fmax(0.0, fmin(s.ny - 1., p[1]));
@@ -239,7 +225,7 @@ __device__ inline double weno3(const float *a, const uint8_t *m, FS s, const dou
 #pragma unroll
             for (int ii = 0; ii < 6; ++ii) {
                 const int64_t q = s.at(min(max(i + ii - 2, 0), s.nx - 1), jc, kc);
-                v[ii] = m ? (double)rd(a, m, q) : (double)a[q];
+                v[ii] = (double)rd_bg(a, m, q, bg);
             }
             vv[jj] = weno6(x - i, v);
         }
@@ -651,83 +637,92 @@ __device__ inline bool cell_velocity(const Dims &d, const CFaces &f, int i, int 
 
 // MacCormack advection of the active cells of a cell-centred level set by the MAC
 // velocity (macadvection3.cpp:178-277, advect_scalar as the level-set tracker calls
-// it).  Forward pass (lo != 0): out = semi-Lagrangian value (vec3d departure), the
-// limiter's bounds (min from FLT_MAX, max from FLT_MIN) and the narrow-band flag of
-// the level set before the step at the departure point.  Backward pass (fin_out !=
-// 0): the semi-Lagrangian value of q0 over -dt, combined into the final value.
-// Inactive cells of the output are left alone (they keep what they read).
+// it), over the list of those cells (what bounded one thread per cell of the grid was the
+// 65,536 workgroups of 256^3, of which a few percent had work: 58 us per pass).
+// Forward pass (lo != 0): out = semi-Lagrangian value (vec3d departure), the limiter's
+// bounds (min from FLT_MAX, max from FLT_MIN) and the narrow-band flag of the level set
+// before the step at the departure point.  Backward pass (fin_out != 0): the
+// semi-Lagrangian value of q0 over -dt, combined into the final value.  q0 is a new array
+// of the level set's type (macadvection3.cpp:248): off the band (mq, null: none) it reads
+// the background value.  Inactive cells of the output are left alone, and the passes read
+// no output of their own, so that the caller's array needs no copy.
 template <bool WENO>
-__global__ __launch_bounds__(kNT) void k_advect_cell(Dims d, Split sp, double dx, double dt, const float *q, const uint8_t *mq,
+__global__ __launch_bounds__(kNT) void k_advect_cell(Dims d, Split sp, double dx, double dt, const uint32_t *list,
+                                                     const unsigned int *count, const float *q, const uint8_t *mq,
                                                      CFaces vel, const float *fluid, int trim, float *out, float *lo,
                                                      float *hi, uint8_t *band, const float *fin_qin,
                                                      const float *fin_lo, const float *fin_hi,
-                                                     const uint8_t *fin_band, const float *fin_q0, float *fin_out,
-                                                     int fill_inactive, float background) {
+                                                     const uint8_t *fin_band, float *fin_out, float background) {
 #pragma clang fp contract(off)
     const FS cs{d.nx, d.ny, d.nz};
-    const int64_t c = blockIdx.x * (int64_t)kNT + threadIdx.x;
-    if (c >= cs.n()) return;
-    if (!mq[c]) {
-        // q_0 is a new array of the level set's type (macadvection3.cpp:248): outside
-        // the band it reads the background value
-        if (fill_inactive) out[c] = background;
-        return;
-    }
-    int i, j, k;
-    decompose(c, sp, i, j, k);
-    double u[3];
-    const bool moving = cell_velocity(d, vel, i, j, k, u);
-    double p[3] = {(double)i, (double)j, (double)k};
-    float value = q[c];
-    int ci = 0, cj = 0, ck = 0;
-    float vals[8];
-    if (moving) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) p[a] = p[a] - dt * u[a] / dx;
-        double coef[8];
-        interp_coef(cs, p, ci, cj, ck, coef);
-        float acc = 0.0f;
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            vals[n] = q[corner(cs, ci, cj, ck, n)];
-            if (coef[n] != 0.0) acc = (float)((double)acc + (double)vals[n] * coef[n]);
-        }
-        value = WENO ? (float)weno3(q, nullptr, cs, p) : acc;  // WENO=1 (macadvection3.cpp:193-194)
-    }
-    if (out) out[c] = value;
-    if (lo) {
+    const unsigned int len = *count;
+    for (unsigned int at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) {
+        const int64_t c = list[at];
+        int i, j, k;
+        decompose(c, sp, i, j, k);
+        double u[3];
+        const bool moving = cell_velocity(d, vel, i, j, k, u);
+        double p[3] = {(double)i, (double)j, (double)k};
+        const float here = q[c];
+        float value = here;
+        int ci = 0, cj = 0, ck = 0;
+        float vals[8];
         if (moving) {
-            double mn = FLT_MAX, mx = FLT_MIN;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) p[a] = p[a] - dt * u[a] / dx;
+            double coef[8];
+            interp_coef(cs, p, ci, cj, ck, coef);
+            float acc = 0.0f;
 #pragma unroll
             for (int n = 0; n < 8; ++n) {
-                mn = fmin(mn, (double)vals[n]);
-                mx = fmax(mx, (double)vals[n]);
+                vals[n] = rd_bg(q, mq, corner(cs, ci, cj, ck, n), background);
+                if (coef[n] != 0.0) acc = (float)((double)acc + (double)vals[n] * coef[n]);
             }
-            lo[c] = (float)mn;
-            hi[c] = (float)mx;
-            band[c] = (double)interp(fluid, nullptr, cs, p) > -dx * (double)trim;
-        } else {
-            lo[c] = q[c];
-            hi[c] = q[c];
-            band[c] = (double)fluid[c] > -dx * (double)trim;
+            // WENO=1 (macadvection3.cpp:193-194)
+            value = WENO ? (float)weno3(q, mq, cs, p, background) : acc;
+        }
+        if (out) out[c] = value;
+        if (lo) {
+            if (moving) {
+                double mn = FLT_MAX, mx = FLT_MIN;
+#pragma unroll
+                for (int n = 0; n < 8; ++n) {
+                    mn = fmin(mn, (double)vals[n]);
+                    mx = fmax(mx, (double)vals[n]);
+                }
+                lo[c] = (float)mn;
+                hi[c] = (float)mx;
+                band[c] = (double)interp(fluid, nullptr, cs, p) > -dx * (double)trim;
+            } else {
+                lo[c] = here;
+                hi[c] = here;
+                band[c] = (double)fluid[c] > -dx * (double)trim;
+            }
+        }
+        if (fin_out) {
+            float r;
+            if (fin_band[c]) {
+                r = here;
+            } else {
+                const double mn = fin_lo[c], mx = fin_hi[c], q0 = here;
+                const double corr = 0.5 * ((double)fin_qin[c] - (double)value);
+                if (q0 + corr < mn)
+                    r = (float)mn;
+                else if (q0 + corr > mx)
+                    r = (float)mx;
+                else
+                    r = (float)(q0 + corr);
+            }
+            fin_out[c] = r;
         }
     }
-    if (fin_out) {
-        float r;
-        if (fin_band[c]) {
-            r = fin_q0[c];
-        } else {
-            const double mn = fin_lo[c], mx = fin_hi[c], q0 = fin_q0[c];
-            const double corr = 0.5 * ((double)fin_qin[c] - (double)value);
-            if (q0 + corr < mn)
-                r = (float)mn;
-            else if (q0 + corr > mx)
-                r = (float)mx;
-            else
-                r = (float)(q0 + corr);
-        }
-        fin_out[c] = r;
-    }
+}
+
+// dst = src on the list's cells
+__global__ __launch_bounds__(kNT) void k_put_cells(const uint32_t *list, const unsigned int *count, const float *src,
+                                                   float *dst) {
+    const unsigned int len = *count;
+    for (unsigned int at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) dst[list[at]] = src[list[at]];
 }
 
 // ---------------------------------------------------------------- gravity, activity
@@ -809,10 +804,28 @@ int64_t max_faces(const Dims &d) {
 // a snapshot of phi, one dilation of the band, and combine_levelset with the offset dx
 // (:66-86; convert_to_cell :48-65).
 
-__global__ void k_exls_exist(int64_t nn, const float *__restrict__ solid, const uint8_t *__restrict__ sband,
-                             unsigned long long *__restrict__ flag) {
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nn; q += (int64_t)gridDim.x * blockDim.x)
-        if ((!sband || sband[q]) && solid[q] < 0.0f) *flag = 1ull;  // every writer stores the same value
+// the node mask first, eight nodes per thread: the level set is read only where it is active,
+// and nothing once a node has been found (every writer stores the same value)
+__global__ __launch_bounds__(kNT) void k_exls_exist(int64_t nn, const float *__restrict__ solid,
+                                                    const uint8_t *__restrict__ sband, int vec, unsigned int *flag) {
+    for (int64_t g = blockIdx.x * (int64_t)kNT + threadIdx.x; g * 8 < nn; g += (int64_t)gridDim.x * kNT) {
+        const int64_t q0 = g * 8;
+        uint64_t m = ~0ull;
+        if (sband) {
+            m = 0ull;
+            if (vec && q0 + 8 <= nn)
+                m = *reinterpret_cast<const uint64_t *>(sband + q0);
+            else
+                for (int q = 0; q < 8; ++q)
+                    if (q0 + q < nn) m |= (uint64_t)sband[q0 + q] << (8 * q);
+        }
+        if (!m) continue;
+        if (*(volatile unsigned int *)flag) return;
+        bool below = false;
+        for (int q = 0; q < 8; ++q)
+            if (q0 + q < nn && ((m >> (8 * q)) & 0xff)) below = below || solid[q0 + q] < 0.0f;
+        if (below) *flag = 1u;
+    }
 }
 
 // array_derivative3::derivative<float> (array_derivative3.h:51-122): the trilinear
@@ -863,47 +876,53 @@ __device__ inline void normalize3(double v[3]) {
         for (int d = 0; d < 3; ++d) v[d] /= len;
 }
 
-// pass 2: the band cells inside the solid, from the snapshot `old`
+// pass 2: the band cells inside the solid, over the band's list; out holds the list's cells
+// (the caller's values until k_put_cells has put them back)
 __global__ __launch_bounds__(kNT) void k_exls_wall(Dims d, Split sp, double dx, const float *__restrict__ solid,
-                                                   const float *__restrict__ old, const uint8_t *__restrict__ band,
-                                                   float *__restrict__ phi, float background, int wall,
-                                                   int horizontal) {
+                                                   const uint32_t *__restrict__ list,
+                                                   const unsigned int *__restrict__ count,
+                                                   const float *__restrict__ old, float *__restrict__ out,
+                                                   float background, int wall, int horizontal) {
 #pragma clang fp contract(off)
     const FS s{d.nx, d.ny, d.nz}, ns{d.nx + 1, d.ny + 1, d.nz + 1};
-    const int64_t c = blockIdx.x * (int64_t)kNT + threadIdx.x;
-    if (c >= s.n() || !band[c]) return;
-    int i, j, k;
-    decompose(c, sp, i, j, k);
-    const double p[3] = {i + 0.5, j + 0.5, k + 0.5};
-    const double sl = (double)interp(solid, nullptr, ns, p);
-    if (!(sl < 0.0)) return;
-    if (!wall) {
-        phi[c] = (float)sl;
-        return;
-    }
-    float g[3];
-    derivative_idx(solid, ns, p, g);
-    double nrm[3] = {(double)g[0], (double)g[1], (double)g[2]};
-    normalize3(nrm);
-    if (norm2_3(nrm) == 0.0) {
-        phi[c] = background;
-        return;
-    }
-    const double t = -sl / dx;
-    const double pn[3] = {i + t * nrm[0], j + t * nrm[1], k + t * nrm[2]};
-    float value = interp(old, nullptr, s, pn);
-    // sin(pi/4) as the double the reference computes (gridutility3.cpp:93)
-    const double limit_y = 0.70710678118654746;
-    if (horizontal && nrm[1] < limit_y) {
-        double h[3] = {nrm[0], 0.0, nrm[2]};
-        normalize3(h);
-        if (norm2_3(h) != 0.0) {
-            const double ph[3] = {i + t * h[0], j + t * h[1], k + t * h[2]};
-            const float vh = interp(old, nullptr, s, ph);
-            if (vh < value) value = vh;
+    const unsigned int len = *count;
+    for (unsigned int at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) {
+        const int64_t c = list[at];
+        int i, j, k;
+        decompose(c, sp, i, j, k);
+        const double p[3] = {i + 0.5, j + 0.5, k + 0.5};
+        const double sl = (double)interp(solid, nullptr, ns, p);
+        float value = old[c];
+        if (sl < 0.0) {
+            if (!wall) {
+                value = (float)sl;
+            } else {
+                float g[3];
+                derivative_idx(solid, ns, p, g);
+                double nrm[3] = {(double)g[0], (double)g[1], (double)g[2]};
+                normalize3(nrm);
+                if (norm2_3(nrm) == 0.0) {
+                    value = background;
+                } else {
+                    const double t = -sl / dx;
+                    const double pn[3] = {i + t * nrm[0], j + t * nrm[1], k + t * nrm[2]};
+                    value = interp(old, nullptr, s, pn);
+                    // sin(pi/4) as the double the reference computes (gridutility3.cpp:93)
+                    const double limit_y = 0.70710678118654746;
+                    if (horizontal && nrm[1] < limit_y) {
+                        double h[3] = {nrm[0], 0.0, nrm[2]};
+                        normalize3(h);
+                        if (norm2_3(h) != 0.0) {
+                            const double ph[3] = {i + t * h[0], j + t * h[1], k + t * h[2]};
+                            const float vh = interp(old, nullptr, s, ph);
+                            if (vh < value) value = vh;
+                        }
+                    }
+                }
+            }
         }
+        out[c] = value;
     }
-    phi[c] = value;
 }
 
 // pass 3: one dilation; a new cell >= 0 next to an in-bounds cell below 0 becomes dx
@@ -944,12 +963,11 @@ __global__ __launch_bounds__(kNT) void k_exls_combine(Dims d, Split sp, double d
                                                       const float *__restrict__ phi2,
                                                       const uint8_t *__restrict__ band2, float background,
                                                       float *__restrict__ phi, uint8_t *__restrict__ band,
-                                                      unsigned long long *__restrict__ count) {
+                                                      unsigned int *__restrict__ count) {
 #pragma clang fp contract(off)
     const FS s{d.nx, d.ny, d.nz}, ns{d.nx + 1, d.ny + 1, d.nz + 1};
-    const int64_t c = blockIdx.x * (int64_t)kNT + threadIdx.x;
-    bool act = false;
-    if (c < s.n()) {
+    unsigned int found = 0;
+    for (int64_t c = blockIdx.x * (int64_t)kNT + threadIdx.x; c < s.n(); c += (int64_t)gridDim.x * kNT) {
         int i, j, k;
         decompose(c, sp, i, j, k);
         double v = 0.0;
@@ -969,22 +987,34 @@ __global__ __launch_bounds__(kNT) void k_exls_combine(Dims d, Split sp, double d
         const float neg = -(float)dx - sc;
         const float f = phi2[c];
         const float comb = f < neg ? neg : f;
-        act = band2[c] || any;
+        const bool act = band2[c] || any;
         phi[c] = act ? comb : (comb < 0.0f ? -background : background);
         band[c] = act ? 1 : 0;
+        found += act;
     }
-    const unsigned long long wave_act = __popcll(__ballot(act));
-    if ((threadIdx.x & 63) == 0 && wave_act) atomicAdd(count, wave_act);
+    found = block_count(found);
+    if (threadIdx.x == 0 && found) atomicAdd(count, found);
 }
 
-__global__ void k_exls_fill(unsigned long long *p) { p[0] = 0ull; }
-
-__global__ __launch_bounds__(kNT) void k_count_band(int64_t n, const uint8_t *__restrict__ band,
-                                                    unsigned long long *__restrict__ count) {
-    const int64_t c = blockIdx.x * (int64_t)kNT + threadIdx.x;
-    const bool act = c < n && band[c];
-    const unsigned long long wave_act = __popcll(__ballot(act));
-    if ((threadIdx.x & 63) == 0 && wave_act) atomicAdd(count, wave_act);
+// sixteen cells per thread, one atomic per block (one per wave took 239 us at 256^3, all of
+// them on one address)
+__global__ __launch_bounds__(kNT) void k_count_band(int64_t n, const uint8_t *__restrict__ band, int vec,
+                                                    unsigned int *__restrict__ count) {
+    unsigned int found = 0;
+    for (int64_t g = blockIdx.x * (int64_t)kNT + threadIdx.x; g * 16 < n; g += (int64_t)gridDim.x * kNT) {
+        const int64_t c0 = g * 16;
+        if (vec && c0 + 16 <= n) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(band + c0);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int q = 0; q < 16; ++q) found += (w[q >> 2] >> (8 * (q & 3))) & 0xffu ? 1u : 0u;
+        } else {
+            for (int q = 0; q < 16; ++q)
+                if (c0 + q < n) found += band[c0 + q] ? 1u : 0u;
+        }
+    }
+    found = block_count(found);
+    if (threadIdx.x == 0 && found) atomicAdd(count, found);
 }
 
 bool aligned16(std::initializer_list<const void *> ps) {
@@ -1066,37 +1096,42 @@ int shk_extrapolate_levelset(shk_ctx *c, const float *solid, const uint8_t *soli
     const FS s{d.nx, d.ny, d.nz};
     const int64_t n = s.n(), nn = (int64_t)(d.nx + 1) * (d.ny + 1) * (d.nz + 1);
     LiquidWork *lw = work(c);
-    HIPC(c, lw->count.ensure(2));
-    HIPC(c, lw->a[0].ensure((size_t)n));
-    HIPC(c, lw->a[1].ensure((size_t)n));
-    HIPC(c, lw->band[0].ensure((size_t)n));
+    HIPC(c, lw->counts.ensure(2));
     hipStream_t st = c->stream;
-    unsigned long long *flag = lw->count.p, *cnt_d = lw->count.p + 1;
-    hipLaunchKernelGGL(k_exls_fill, dim3(1), dim3(1), 0, st, flag);
-    hipLaunchKernelGGL(k_exls_fill, dim3(1), dim3(1), 0, st, cnt_d);
-    hipLaunchKernelGGL(k_exls_exist, dim3(1024), dim3(kNT), 0, st, nn, solid, solid_band, flag);
+    unsigned int *flag = lw->counts.p, *cnt_d = lw->counts.p + 1;
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, flag, 2);
+    hipLaunchKernelGGL(k_exls_exist, dim3(std::min(blocks_for((nn + 7) / 8), kBandBlocks)), dim3(kNT), 0, st, nn, solid,
+                       solid_band, (uintptr_t)solid_band % 8 == 0 ? 1 : 0, flag);
+    // the band as it stands, for the case that there is no solid: one round trip for both
+    const unsigned gc = std::min(blocks_for((n + 15) / 16), kBandBlocks);
+    hipLaunchKernelGGL(k_count_band, dim3(gc), dim3(kNT), 0, st, n, band, aligned16({band}) ? 1 : 0, cnt_d);
     HIPC(c, hipGetLastError());
-    unsigned long long exist = 0;
-    HIPC(c, hipMemcpyAsync(&exist, flag, sizeof exist, hipMemcpyDeviceToHost, st));
+    unsigned int got[2] = {0u, 0u};
+    HIPC(c, hipMemcpyAsync(got, flag, sizeof got, hipMemcpyDeviceToHost, st));
     HIPC(c, hipStreamSynchronize(st));
-    const Split sp = cells_split(d);
-    const unsigned gb = blocks_for(n);
-    if (exist) {
-        HIPC(c, hipMemcpyAsync(lw->a[0].p, phi, sizeof(float) * (size_t)n, hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(k_exls_wall, dim3(gb), dim3(kNT), 0, st, d, sp, c->dx, solid, lw->a[0].p, band, phi,
-                           background, c->prm.solid_wall_extrap ? 1 : 0, c->prm.horizontal_extrap ? 1 : 0);
+    unsigned int cnt = got[1];
+    if (got[0]) {
+        const Split sp = cells_split(d);
+        const unsigned gb = blocks_for(n);
+        HIPC(c, lw->a[0].ensure((size_t)n));
+        HIPC(c, lw->a[1].ensure((size_t)n));
+        HIPC(c, lw->band[0].ensure((size_t)n));
+        HIPC(c, lw->list.ensure((size_t)n));
+        hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, flag, 2);  // flag: now the list's length
+        hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(n)), dim3(kBandNT), 0, st, n, band,
+                           aligned16({band}) ? 1 : 0, lw->list.p, flag);
+        const unsigned gl = std::min(gb, kBandBlocks);
+        hipLaunchKernelGGL(k_exls_wall, dim3(gl), dim3(kNT), 0, st, d, sp, c->dx, solid, lw->list.p, flag, phi,
+                           lw->a[0].p, background, c->prm.solid_wall_extrap ? 1 : 0, c->prm.horizontal_extrap ? 1 : 0);
+        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, lw->list.p, flag, lw->a[0].p, phi);
         hipLaunchKernelGGL(k_exls_dilate, dim3(gb), dim3(kNT), 0, st, d, sp, c->dx, phi, band, lw->a[1].p,
                            lw->band[0].p);
-        hipLaunchKernelGGL(k_exls_combine, dim3(gb), dim3(kNT), 0, st, d, sp, c->dx, solid, solid_band, lw->a[1].p,
-                           lw->band[0].p, background, phi, band, cnt_d);
-    } else {
-        // no solid: nothing changes; count the band
-        hipLaunchKernelGGL(k_count_band, dim3(gb), dim3(kNT), 0, st, n, band, cnt_d);
+        hipLaunchKernelGGL(k_exls_combine, dim3(std::min(gb, 4 * kBandBlocks)), dim3(kNT), 0, st, d, sp, c->dx, solid,
+                           solid_band, lw->a[1].p, lw->band[0].p, background, phi, band, cnt_d);
+        HIPC(c, hipGetLastError());
+        HIPC(c, hipMemcpyAsync(&cnt, cnt_d, sizeof cnt, hipMemcpyDeviceToHost, st));
+        HIPC(c, hipStreamSynchronize(st));
     }
-    HIPC(c, hipGetLastError());
-    unsigned long long cnt = 0;
-    HIPC(c, hipMemcpyAsync(&cnt, cnt_d, sizeof cnt, hipMemcpyDeviceToHost, st));
-    HIPC(c, hipStreamSynchronize(st));
     if (active) *active = (int64_t)cnt;
     return SHK_OK;
 }
@@ -1226,26 +1261,33 @@ int shk_advect_levelset(shk_ctx *c, double dt, float *phi, const uint8_t *mphi, 
     LiquidWork *lw = work(c);
     const bool mc = c->prm.maccormack;
     const int64_t G = (int64_t)d.nx * d.ny * d.nz;
-    // scratch: the level set before the step (a[0]), q0 (b[0]), limiter bounds, band
-    HIPC(c, lw->a[0].ensure(G));
-    HIPC(c, hipMemcpyAsync(lw->a[0].p, phi, sizeof(float) * G, hipMemcpyDeviceToDevice, c->stream));
+    // scratch: the band's cells, q0 (b[0]), limiter bounds, band
+    HIPC(c, lw->list.ensure(G));
+    HIPC(c, lw->counts.ensure(2));
+    HIPC(c, lw->b[0].ensure(G));
     if (mc) {
-        HIPC(c, lw->b[0].ensure(G));
         HIPC(c, lw->lo[0].ensure(G));
         HIPC(c, lw->hi[0].ensure(G));
         HIPC(c, lw->band[0].ensure(G));
     }
     const CFaces vel{{u, v, w}, {mu, mv, mw}};
-    const float *qin = lw->a[0].p;
+    hipStream_t st = c->stream;
+    unsigned int *len = lw->counts.p;
+    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, len, 2);
+    hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(G)), dim3(kBandNT), 0, st, G, mphi,
+                       aligned16({mphi}) ? 1 : 0, lw->list.p, len);
+    const unsigned gl = std::min(blocks_for(G), kBandBlocks);
     auto kern = c->prm.weno ? k_advect_cell<true> : k_advect_cell<false>;
-    hipLaunchKernelGGL(kern, dim3(blocks_for(G)), dim3(kNT), 0, c->stream, d, cells_split(d), c->dx, dt, qin, mphi, vel,
-                       qin, c->prm.trim_narrowband, mc ? lw->b[0].p : phi, mc ? lw->lo[0].p : nullptr,
+    hipLaunchKernelGGL(kern, dim3(gl), dim3(kNT), 0, st, d, cells_split(d), c->dx, dt, lw->list.p, len, phi, nullptr,
+                       vel, phi, c->prm.trim_narrowband, lw->b[0].p, mc ? lw->lo[0].p : nullptr,
                        mc ? lw->hi[0].p : nullptr, mc ? lw->band[0].p : nullptr, nullptr, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, mc ? 1 : 0, background);
-    if (mc)
-        hipLaunchKernelGGL(kern, dim3(blocks_for(G)), dim3(kNT), 0, c->stream, d, cells_split(d), c->dx, -dt,
-                           lw->b[0].p, mphi, vel, qin, c->prm.trim_narrowband, nullptr, nullptr, nullptr, nullptr, qin,
-                           lw->lo[0].p, lw->hi[0].p, lw->band[0].p, lw->b[0].p, phi, 0, background);
+                       nullptr, background);
+    if (mc)  // reads q0 and, cell by cell, the level set it replaces
+        hipLaunchKernelGGL(kern, dim3(gl), dim3(kNT), 0, st, d, cells_split(d), c->dx, -dt, lw->list.p, len,
+                           lw->b[0].p, mphi, vel, nullptr, c->prm.trim_narrowband, nullptr, nullptr, nullptr, nullptr,
+                           phi, lw->lo[0].p, lw->hi[0].p, lw->band[0].p, phi, background);
+    else
+        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, lw->list.p, len, lw->b[0].p, phi);
     HIPC(c, hipGetLastError());
     HIPC(c, hipStreamSynchronize(c->stream));
     return SHK_OK;
