@@ -17,12 +17,20 @@
 //   - the coarse matrix is the Galerkin product P'AP of the piecewise-constant
 //     prolongation (exact zeros dropped), until at most kAmgCoarseMax rows remain,
 //     whose matrix is inverted densely (FP64 Cholesky).
-// V-cycle (device, FP64, 2 kernels per level): the pre-smoothing step from zero
-// x = w D^-1 b, its residual and the restriction (sum over the aggregate) in one
-// kernel per coarse row; the prolongation with over-correction alpha and the
-// post-smoothing step in one kernel per row; the dense coarsest solve in one
-// workgroup.  Pre- and post-smoothing are the same symmetric operator, so M is fixed
-// and SPD and plain CG applies.  Every sum runs in one fixed order (deterministic).
+// V-cycle (device, FP64): going down, a level's residual after the pre-smoothing step from
+// zero x = w D^-1 b and its restriction (sum over the aggregate) in one kernel; going up,
+// the post-smoothing of a level and the prolongation (over-correction alpha) of its result
+// to the members of the level above in one kernel; the dense coarsest solve.  Pre- and
+// post-smoothing are the same symmetric operator, so M is fixed and SPD and plain CG
+// applies.  Every sum runs in one fixed order (deterministic).
+//
+// What bounds these kernels is latency: a few thousand rows of 7 to 30 entries, each entry
+// a column, then a gather.  So 16 lanes share an aggregate (4 per member row) and 4 a row,
+// each vector a gather reads is stored ready to use (w D^-1 b by the restriction, the
+// corrected step by the prolongation: one gather per entry, not two or three in a chain),
+// and the levels of at most kAmgTailRows rows run in one workgroup of one launch, barriers
+// between them.  59,400 rows (45x40x33 7-point), per V-cycle: the restrictions 178 -> 27 us,
+// the way up 61 -> 26 us, the coarsest solve 24 -> 6 us with the small levels in its launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,7 +43,12 @@
 namespace shk {
 
 constexpr int64_t kAmgCoarseMax = 128;
-constexpr int kAmgNB = 256;  // threads of the level-0 kernels on the CG grid (NB elsewhere)
+constexpr int kAmgDenseMax = 1024;    // rows of a coarsest level that stopped coarsening
+// levels that run in one workgroup: one round of its 64 aggregates per phase, a chain of five
+// dependent loads; with up to 1024 rows (four rounds) the tail took 43 us, more than the
+// launches it saved
+constexpr int64_t kAmgTailRows = 256;
+constexpr int kAmgNB = 1024;  // threads of the level-0 kernels on the CG grid: a tile of 512 rows in two rounds
 constexpr double kAmgStrong = 0.25;
 constexpr double kAmgStall = 0.8;
 constexpr int kAmgMaxLevels = 40;
@@ -54,7 +67,8 @@ struct AmgLevel {
     DevBuf<int32_t> agg;            // row -> row of the next level
     DevBuf<int64_t> mptr;           // next level's row -> its rows mem[mptr[I] .. mptr[I+1])
     DevBuf<int32_t> mem;
-    DevBuf<double> b, x;            // levels >= 1: the V-cycle's rhs and result
+    DevBuf<double> b;               // levels >= 1: the V-cycle's rhs
+    DevBuf<double> x;               // w D^-1 b (levels >= 1), then the corrected step
 };
 
 struct CsrAmg {
@@ -62,6 +76,7 @@ struct CsrAmg {
     int64_t ncoarse = 0;
     DevBuf<double> cinv;            // dense inverse of the coarsest matrix, row-major
     DevBuf<double> z, pz;           // level-0 result and the r.z partials for CG
+    DevBuf<double> x0;              // level 0: the corrected step
     // content of the matrix the hierarchy was built from: rows, entries and two
     // order-independent 64-bit hashes (XOR and sum) of every (row, column, value) entry
     int64_t key_rows = -1, key_nnz = -1;
@@ -87,6 +102,7 @@ void amg_destroy(CsrAmg *h) {
     }
     h->cinv.release();
     h->z.release();
+    h->x0.release();
     h->pz.release();
     h->hash.release();
     delete h;
@@ -234,73 +250,185 @@ std::vector<double> inv_diag(const HostCsr &A) {
 
 // ---------------------------------------------------------------- V-cycle kernels
 
-template <class IDX>
-__device__ inline double row_apply_smoothed(const int64_t *__restrict__ ptr, const IDX *__restrict__ col,
-                                            const double *__restrict__ val, const double *__restrict__ dinv,
-                                            const double *__restrict__ b, double w, int64_t i) {
-    // sum_j a_ij (w dinv_j b_j): A applied to the pre-smoothing step from zero
+// What the kernels need of a level l: its matrix and vectors, the aggregates (rows of level
+// l + 1) with their members, and the weight
+struct AmgDev {
+    int n, nc;
+    const int64_t *ptr;
+    const int32_t *col;
+    const double *val, *dinv;
+    const double *b;
+    double *x;
+    const int64_t *mptr;   // members of the rows of level l + 1
+    const int32_t *mem;
+};
+
+template <int CTRL>
+__device__ inline double amg_dpp(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+// sums over the 4 lanes of a quad and the 16 lanes of a row, the same in every lane
+__device__ inline double quad_sum(double v) {
+    v += amg_dpp<0xB1>(v);  // quad_perm 1,0,3,2
+    return v + amg_dpp<0x4E>(v);
+}
+__device__ inline double row_sum(double v) {
+    v = quad_sum(v);
+    v += amg_dpp<0x141>(v);  // row_half_mirror
+    return v + amg_dpp<0x140>(v);
+}
+
+// this lane's share (every fourth entry) of sum_j a_ij x_j; x(j) gives a value
+template <class IDX, class X>
+__device__ inline double row_share(const int64_t *__restrict__ ptr, const IDX *__restrict__ col,
+                                   const double *__restrict__ val, int64_t i, int lj, X x) {
+    const int64_t e = ptr[i + 1];
     double a = 0.0;
-    for (int64_t p = ptr[i]; p < ptr[i + 1]; ++p) {
-        const int64_t j = (int64_t)col[p];
-        a += val[p] * (w * dinv[j] * b[j]);
-    }
+#pragma unroll 2
+    for (int64_t p = ptr[i] + lj; p < e; p += 4) a += val[p] * x((int64_t)col[p]);
     return a;
 }
 
-// bc[I] = sum over the rows i of aggregate I of t_i = b_i - (A x)_i, x = w D^-1 b
-template <class IDX>
-__global__ __launch_bounds__(256) void k_amg_down(int64_t nc, const int64_t *__restrict__ mptr,
-                                                  const int32_t *__restrict__ mem, const int64_t *__restrict__ ptr,
-                                                  const IDX *__restrict__ col, const double *__restrict__ val,
-                                                  const double *__restrict__ dinv, const double *__restrict__ b,
-                                                  double w, double *__restrict__ bc, const SolveState *state) {
-    if (state && state->done) return;
-    const int64_t I = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (I >= nc) return;
-    double s = 0.0;
-    for (int64_t m = mptr[I]; m < mptr[I + 1]; ++m) {
-        const int64_t i = mem[m];
-        s += b[i] - row_apply_smoothed(ptr, col, val, dinv, b, w, i);
+// aggregate I of level l (16 lanes): bc = sum over its rows i of b_i - (A x)_i, xc = w D_c^-1 bc;
+// every lane of the row of 16 takes part, on = false adds nothing
+template <class IDX, class X>
+__device__ inline void amg_down_row(bool on, int64_t I, int lane16, const int64_t *__restrict__ mptr,
+                                    const int32_t *__restrict__ mem, const int64_t *__restrict__ ptr,
+                                    const IDX *__restrict__ col, const double *__restrict__ val,
+                                    const double *__restrict__ b, X x, double w, const double *__restrict__ dinvc,
+                                    double *__restrict__ bc, double *__restrict__ xc) {
+    double t = 0.0;
+    const int lj = lane16 & 3;
+    if (on) {
+        const int64_t me = mptr[I + 1];
+        for (int64_t m = mptr[I] + (lane16 >> 2); m < me; m += 4) {
+            const int64_t i = mem[m];
+            const double a = row_share(ptr, col, val, i, lj, x);
+            t += (lj == 0 ? b[i] : 0.0) - a;
+        }
     }
-    bc[I] = s;
-}
-
-// the corrected step x'_j = w dinv_j b_j + alpha xc[agg_j] and the post-smoothing
-// y_i = x'_i + w dinv_i (b_i - sum_j a_ij x'_j)
-template <class IDX>
-__device__ inline double amg_up_row(const int64_t *__restrict__ ptr, const IDX *__restrict__ col,
-                                    const double *__restrict__ val, const double *__restrict__ dinv,
-                                    const int32_t *__restrict__ agg, const double *__restrict__ b,
-                                    const double *__restrict__ xc, double w, double alpha, int64_t i) {
-    double a = 0.0;
-    for (int64_t p = ptr[i]; p < ptr[i + 1]; ++p) {
-        const int64_t j = (int64_t)col[p];
-        a += val[p] * (w * dinv[j] * b[j] + alpha * xc[agg[j]]);
+    t = row_sum(t);
+    if (on && lane16 == 0) {
+        bc[I] = t;
+        xc[I] = w * dinvc[I] * t;
     }
-    const double xi = w * dinv[i] * b[i] + alpha * xc[agg[i]];
-    return xi + w * dinv[i] * (b[i] - a);
 }
 
-template <class IDX>
-__global__ __launch_bounds__(256) void k_amg_up(int64_t n, const int64_t *__restrict__ ptr,
-                                                const IDX *__restrict__ col, const double *__restrict__ val,
-                                                const double *__restrict__ dinv, const int32_t *__restrict__ agg,
-                                                const double *__restrict__ b, const double *__restrict__ xc,
-                                                double w, double alpha, double *__restrict__ y,
-                                                const SolveState *state) {
+// the value y of row I of level l + 1 to its members j on level l: x_j = x_j + alpha y (one
+// member per lane of the quad)
+__device__ inline void amg_prolong_row(int64_t I, int lj, double y, double alpha, const int64_t *__restrict__ mptr,
+                                       const int32_t *__restrict__ mem, double *__restrict__ x) {
+    const int64_t me = mptr[I + 1];
+    for (int64_t m = mptr[I] + lj; m < me; m += 4) x[mem[m]] += alpha * y;
+}
+
+// level 0: x = w D^-1 r (the pre-smoothing step, which the prolongation adds to)
+__global__ __launch_bounds__(256) void k_amg_down0(int64_t nc, const int64_t *__restrict__ mptr,
+                                                   const int32_t *__restrict__ mem, const int64_t *__restrict__ ptr,
+                                                   const int64_t *__restrict__ col, const double *__restrict__ val,
+                                                   const double *__restrict__ dinv, const double *__restrict__ r,
+                                                   double w, double *__restrict__ x, const double *__restrict__ dinvc,
+                                                   double *__restrict__ bc, double *__restrict__ xc,
+                                                   const SolveState *state) {
     if (state && state->done) return;
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    y[i] = amg_up_row(ptr, col, val, dinv, agg, b, xc, w, alpha, i);
+    const int64_t I = blockIdx.x * (int64_t)16 + (threadIdx.x >> 4);
+    const int l16 = threadIdx.x & 15;
+    const bool on = I < nc;
+    amg_down_row<int64_t>(on, I, l16, mptr, mem, ptr, col, val, r, [&](int64_t j) { return w * dinv[j] * r[j]; }, w,
+                          dinvc, bc, xc);
+    if (on && (l16 & 3) == 0)
+        for (int64_t m = mptr[I] + (l16 >> 2); m < mptr[I + 1]; m += 4) {
+            const int64_t i = mem[m];
+            x[i] = w * dinv[i] * r[i];
+        }
 }
 
-// level 0 on the CG grid: z = the post-smoothed result, part[block] = r.z over the
-// block's rows (the partials the next direction kernel folds for beta)
+__device__ inline void amg_down_level(const AmgDev &F, const AmgDev &C, double *cb, double w, int64_t first,
+                                      int64_t stride) {
+    const int l16 = threadIdx.x & 15;
+    const double *x = F.x;
+    // whole rows of 16 lanes leave the loop together
+    for (int64_t I = first; I < F.nc; I += stride)
+        amg_down_row<int32_t>(true, I, l16, F.mptr, F.mem, F.ptr, F.col, F.val, F.b, [x](int64_t j) { return x[j]; }, w,
+                              C.dinv, cb, C.x);
+}
+
+// y_i = x_i + w D_i^-1 (b_i - (A x)_i) of the corrected step x, to the level above (fine's x)
+__device__ inline void amg_up_level(const AmgDev &F, const int64_t *fmptr, const int32_t *fmem, double *fx, double w,
+                                    double alpha, int64_t first, int64_t stride) {
+    const int lj = threadIdx.x & 3;
+    const double *x = F.x;
+    for (int64_t i = first; i < F.n; i += stride) {
+        const double a = quad_sum(row_share(F.ptr, F.col, F.val, i, lj, [x](int64_t j) { return x[j]; }));
+        const double y = x[i] + w * F.dinv[i] * (F.b[i] - a);
+        amg_prolong_row(i, lj, y, alpha, fmptr, fmem, fx);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_amg_down(AmgDev F, AmgDev C, double *cb, double w, const SolveState *state) {
+    if (state && state->done) return;
+    amg_down_level(F, C, cb, w, blockIdx.x * (int64_t)16 + (threadIdx.x >> 4), (int64_t)gridDim.x * 16);
+}
+__global__ __launch_bounds__(256) void k_amg_up(AmgDev F, const int64_t *fmptr, const int32_t *fmem, double *fx,
+                                                double w, double alpha, const SolveState *state) {
+    if (state && state->done) return;
+    amg_up_level(F, fmptr, fmem, fx, w, alpha, blockIdx.x * (int64_t)64 + (threadIdx.x >> 2), (int64_t)gridDim.x * 64);
+}
+
+// The small levels and the coarsest solve in one workgroup: lv[0..count) are levels of the
+// hierarchy, the last one the coarsest; the result goes to the level above lv[0] (fmptr,
+// fmem, fx).  Vectors stay in global memory: one workgroup's barriers order its accesses.
+constexpr int kAmgTailLevels = 10, kAmgTailThreads = 1024;
+struct AmgTail {
+    AmgDev lv[kAmgTailLevels];
+    double *cb[kAmgTailLevels];  // lv[k].b, written
+    int count;
+    const double *cinv;
+    const int64_t *fmptr;
+    const int32_t *fmem;
+    double *fx;
+};
+__global__ __launch_bounds__(kAmgTailThreads) void k_amg_tail(AmgTail T, double w, double alpha,
+                                                              const SolveState *state) {
+    __shared__ double bs[kAmgDenseMax];
+    if (state && state->done) return;
+    const int last = T.count - 1;
+    for (int k = 0; k < last; ++k) {
+        amg_down_level(T.lv[k], T.lv[k + 1], T.cb[k + 1], w, threadIdx.x >> 4, kAmgTailThreads / 16);
+        __syncthreads();
+    }
+    // dense coarsest solve: 16 lanes per row of the inverse
+    const int nc = T.lv[last].n;
+    for (int i = threadIdx.x; i < nc; i += kAmgTailThreads) bs[i] = T.lv[last].b[i];
+    __syncthreads();
+    const int64_t *pm = last > 0 ? T.lv[last - 1].mptr : T.fmptr;
+    const int32_t *pe = last > 0 ? T.lv[last - 1].mem : T.fmem;
+    double *px = last > 0 ? T.lv[last - 1].x : T.fx;
+    const int l16 = threadIdx.x & 15;
+    for (int i = threadIdx.x >> 4; i < nc; i += kAmgTailThreads / 16) {
+        double y = 0.0;
+#pragma unroll 4
+        for (int j = l16; j < nc; j += 16) y += T.cinv[(int64_t)i * nc + j] * bs[j];
+        y = row_sum(y);
+        if (l16 < 4) amg_prolong_row(i, l16, y, alpha, pm, pe, px);
+    }
+    __syncthreads();
+    for (int k = last - 1; k >= 0; --k) {
+        const int64_t *fm = k > 0 ? T.lv[k - 1].mptr : T.fmptr;
+        const int32_t *fe = k > 0 ? T.lv[k - 1].mem : T.fmem;
+        double *fx = k > 0 ? T.lv[k - 1].x : T.fx;
+        amg_up_level(T.lv[k], fm, fe, fx, w, alpha, threadIdx.x >> 2, kAmgTailThreads / 4);
+        __syncthreads();
+    }
+}
+
+// level 0 on the CG grid: z = the post-smoothed result of the corrected step x, part[block] =
+// r.z over the block's rows (the partials the next direction kernel folds for beta)
 __global__ __launch_bounds__(kAmgNB) void k_amg_up0(int64_t n, int per, const int64_t *__restrict__ ptr,
                                                 const int64_t *__restrict__ col, const double *__restrict__ val,
-                                                const double *__restrict__ dinv, const int32_t *__restrict__ agg,
-                                                const double *__restrict__ r, const double *__restrict__ xc,
-                                                double w, double alpha, double *__restrict__ z,
+                                                const double *__restrict__ dinv, const double *__restrict__ r,
+                                                const double *__restrict__ x, double w, double *__restrict__ z,
                                                 double *__restrict__ part, const SolveState *state) {
     __shared__ double lds[kAmgNB / kWave];
     if (state && state->done) return;
@@ -308,11 +436,16 @@ __global__ __launch_bounds__(kAmgNB) void k_amg_up0(int64_t n, int per, const in
     const int tiles = blocks_for(n);
     const int t0 = (int)blockIdx.x * per, t1 = t0 + per < tiles ? t0 + per : tiles;
     const int64_t end = (int64_t)t1 * kBrickCells < n ? (int64_t)t1 * kBrickCells : n;
+    const int lj = threadIdx.x & 3;
     double acc = 0.0;
-    for (int64_t e = (int64_t)t0 * kBrickCells + threadIdx.x; e < end; e += kAmgNB) {
-        const double ze = amg_up_row(ptr, col, val, dinv, agg, r, xc, w, alpha, e);
-        z[e] = ze;
-        acc += ze * r[e];
+    // whole quads leave the loop together
+    for (int64_t e = (int64_t)t0 * kBrickCells + (threadIdx.x >> 2); e < end; e += kAmgNB / 4) {
+        const double a = quad_sum(row_share(ptr, col, val, e, lj, [x](int64_t j) { return x[j]; }));
+        if (lj == 0) {
+            const double ze = x[e] + w * dinv[e] * (r[e] - a);
+            z[e] = ze;
+            acc += ze * r[e];
+        }
     }
     const double s = block_sum<kAmgNB>(acc, lds);
     if (threadIdx.x == 0 && part) part[blockIdx.x] = s;
@@ -334,15 +467,17 @@ __global__ __launch_bounds__(kAmgNB) void k_amg_partials(int64_t n, int per, con
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// x = Cinv b on the coarsest level (one workgroup)
+// x = Cinv b of a matrix that is its own coarsest level (one workgroup, 16 lanes per row)
 __global__ __launch_bounds__(256) void k_amg_coarse(int64_t nc, const double *__restrict__ cinv,
                                                     const double *__restrict__ b, double *__restrict__ x,
                                                     const SolveState *state) {
     if (state && state->done) return;
-    for (int64_t i = threadIdx.x; i < nc; i += blockDim.x) {
+    const int l16 = threadIdx.x & 15;
+    for (int64_t i = threadIdx.x >> 4; i < nc; i += 16) {
         double s = 0.0;
-        for (int64_t j = 0; j < nc; ++j) s += cinv[i * nc + j] * b[j];
-        x[i] = s;
+        for (int64_t j = l16; j < nc; j += 16) s += cinv[i * nc + j] * b[j];
+        s = row_sum(s);
+        if (l16 == 0) x[i] = s;
     }
 }
 
@@ -471,7 +606,7 @@ int amg_setup(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int64_t *co
     }
     // the coarsest level: dense inverse
     AmgLevel &C = h->lv.back();
-    if (C.n > 1024)
+    if (C.n > kAmgDenseMax)
         return c->fail(SHK_BAD_ARG, "multigrid: the matrix does not coarsen below %lld rows", (long long)C.n);
     h->ncoarse = C.n;
     std::vector<double> dense((size_t)C.n * C.n, 0.0);
@@ -485,6 +620,7 @@ int amg_setup(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int64_t *co
     h->key_x = key[0];
     h->key_s = key[1];
     HIPC(c, h->z.ensure((size_t)std::max<int64_t>(rows, 1)));
+    HIPC(c, h->x0.ensure((size_t)std::max<int64_t>(rows, 1)));
     HIPC(c, h->pz.ensure((size_t)kMaxBlocks + 64));
     HIPC(c, hipStreamSynchronize(st));
     return SHK_OK;
@@ -503,29 +639,43 @@ int amg_vcycle(shk_ctx *c, const double *r, const Grid &g, const SolveState *sta
         HIPC(c, hipGetLastError());
         return SHK_OK;
     }
-    // down
-    for (int l = 0; l < L; ++l) {
+    auto dev = [&](int l) {
         AmgLevel &F = h->lv[l];
-        AmgLevel &Cn = h->lv[l + 1];
-        const double *b = l == 0 ? r : F.b.p;
-        if (l == 0)
-            hipLaunchKernelGGL(k_amg_down<int64_t>, dim3(blocks256(F.nc)), dim3(256), 0, st, F.nc, F.mptr.p,
-                               F.mem.p, F.rowptr, F.cols64, F.vals, F.dinv.p, b, w, Cn.b.p, state);
-        else
-            hipLaunchKernelGGL(k_amg_down<int32_t>, dim3(blocks256(F.nc)), dim3(256), 0, st, F.nc, F.mptr.p,
-                               F.mem.p, F.rowptr, F.cols32, F.vals, F.dinv.p, b, w, Cn.b.p, state);
+        return AmgDev{(int)F.n, (int)F.nc, F.rowptr, F.cols32, F.vals, F.dinv.p, F.b.p, F.x.p, F.mptr.p, F.mem.p};
+    };
+    auto blocks = [](int64_t n, int per) { return dim3((unsigned)std::max<int64_t>(1, (n + per - 1) / per)); };
+    AmgLevel &F0 = h->lv[0], &F1 = h->lv[1];
+    hipLaunchKernelGGL(k_amg_down0, blocks(F0.nc, 16), dim3(256), 0, st, F0.nc, F0.mptr.p, F0.mem.p, F0.rowptr,
+                       F0.cols64, F0.vals, F0.dinv.p, r, w, h->x0.p, F1.dinv.p, F1.b.p, F1.x.p, state);
+    // the levels of one launch each, then the tail in one
+    int ls = 1;
+    while (ls < L && (h->lv[ls].n > kAmgTailRows || L - ls + 1 > kAmgTailLevels)) ++ls;
+    for (int l = 1; l < ls; ++l)
+        hipLaunchKernelGGL(k_amg_down, blocks(h->lv[l].nc, 16), dim3(256), 0, st, dev(l), dev(l + 1), h->lv[l + 1].b.p,
+                           w, state);
+    auto above = [&](int l, const int64_t *&m, const int32_t *&e, double *&x) {  // the level above l and its x
+        m = h->lv[l - 1].mptr.p;
+        e = h->lv[l - 1].mem.p;
+        x = l > 1 ? h->lv[l - 1].x.p : h->x0.p;
+    };
+    AmgTail T{};
+    T.count = L - ls + 1;
+    for (int k = 0; k < T.count; ++k) {
+        T.lv[k] = dev(ls + k);
+        T.cb[k] = h->lv[ls + k].b.p;
     }
-    AmgLevel &Cl = h->lv[L];
-    hipLaunchKernelGGL(k_amg_coarse, dim3(1), dim3(256), 0, st, h->ncoarse, h->cinv.p, Cl.b.p, Cl.x.p, state);
-    // up
-    for (int l = L - 1; l >= 1; --l) {
-        AmgLevel &F = h->lv[l];
-        hipLaunchKernelGGL(k_amg_up<int32_t>, dim3(blocks256(F.n)), dim3(256), 0, st, F.n, F.rowptr, F.cols32,
-                           F.vals, F.dinv.p, F.agg.p, F.b.p, h->lv[l + 1].x.p, w, alpha, F.x.p, state);
+    T.cinv = h->cinv.p;
+    above(ls, T.fmptr, T.fmem, T.fx);
+    hipLaunchKernelGGL(k_amg_tail, dim3(1), dim3(kAmgTailThreads), 0, st, T, w, alpha, state);
+    for (int l = ls - 1; l >= 1; --l) {
+        const int64_t *m;
+        const int32_t *e;
+        double *x;
+        above(l, m, e, x);
+        hipLaunchKernelGGL(k_amg_up, blocks(h->lv[l].n, 64), dim3(256), 0, st, dev(l), m, e, x, w, alpha, state);
     }
-    AmgLevel &F0 = h->lv[0];
     hipLaunchKernelGGL(k_amg_up0, dim3(g.blocks), dim3(kAmgNB), 0, st, F0.n, g.per, F0.rowptr, F0.cols64, F0.vals,
-                       F0.dinv.p, F0.agg.p, r, h->lv[1].x.p, w, alpha, h->z.p, h->pz.p, state);
+                       F0.dinv.p, r, h->x0.p, w, h->z.p, h->pz.p, state);
     HIPC(c, hipGetLastError());
     return SHK_OK;
 }
