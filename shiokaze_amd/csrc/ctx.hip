@@ -220,6 +220,21 @@ int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double 
     ran = c->h_state->aborted == 0;
     return SHK_OK;
 }
+int solve_resident_csr(shk_ctx *c, const CsrOp &op, const double *rhs, const double *sig, double *x, double *pub,
+                       unsigned long long *slots, const unsigned long long *longest, bool &ran) {
+    ran = false;
+    if (c->profile || resident_csr_plan(op.rows, 1, c->device, c->cus).blocks < 1) return SHK_OK;
+    unsigned long long len = 0;
+    HIPC(c, hipMemcpyAsync(&len, longest, sizeof len, hipMemcpyDeviceToHost, c->stream));
+    HIPC(c, hipStreamSynchronize(c->stream));
+    const ResidentPlan p = resident_csr_plan(op.rows, (int64_t)len, c->device, c->cus);
+    if (p.blocks < 1) return SHK_OK;
+    HIPC(c, resident_csr(c->stream, p, op, rhs, sig, x, pub, slots, c->state.p, c->h_state, c->prm.residual,
+                         c->prm.max_iterations, c->device, c->cus));
+    ran = c->h_state->aborted == 0;
+    return SHK_OK;
+}
+
 template int solve_resident<float>(shk_ctx *, const BrickOp<float> &, const float *, const double *, float *, float *,
                                    double, int64_t, bool &);
 template int solve_resident<double>(shk_ctx *, const BrickOp<double> &, const double *, const double *, double *,
@@ -1105,43 +1120,54 @@ int solve_csr_device(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int6
     const Grid g = make_grid(rows);
     HIPC(c, hipEventRecord(c->ev[0], c->stream));
     if (amg && (rc = amg_setup(c, rows, rowptr, cols, vals))) return rc;
-    launch_csr_diag(c->stream, op, c->diag64.p, c->sig64.p);
-    CsrOp sop = op;
-    if (jac) {
-        HIPC(c, c->cx64.ensure((size_t)0));
-        // scaled copy of the values: the Jacobi-PCG iterates as CG on D^-1/2 A D^-1/2
-        int64_t nnz = 0;
-        HIPC(c, hipMemcpy(&nnz, rowptr + rows, sizeof(int64_t), hipMemcpyDeviceToHost));
-        if (nnz < 0) return c->fail(SHK_BAD_ARG, "rowptr[rows] is negative");
-        HIPC(c, c->q64.ensure(std::max<int64_t>(rows, 1)));
-        HIPC(c, c->hx64.ensure(std::max<int64_t>(nnz, 1)));
-        launch_csr_scale(c->stream, op, c->sig64.p, c->hx64.p);
-        sop.vals = c->hx64.p;
-    }
+    HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
+    launch_csr_diag(c->stream, op, c->diag64.p, c->sig64.p, c->count.p);
     const double *sig = jac ? c->sig64.p : nullptr;
-    Reduction red = reduction(c);
-    if (amg) red.pz = amg_pz(c->amg);
-    // the vector the next direction is formed from: r, or z = M r
-    const double *dsrc = amg ? amg_z(c->amg) : c->r64.p;
-    launch_cg_init<double, double>(c->stream, g, b, sig, x, c->r64.p, c->s64.p, red, c->prm.residual,
-                                   c->prm.max_iterations);
-    double *S[2] = {c->s64.p, c->t64.p};
-    int m = 0;
-    if (amg && (rc = amg_vcycle(c, c->r64.p, g, c->state.p))) return rc;
-    launch_dir_spmv_csr(c->stream, g, sop, dsrc, S[0], S[1], c->q64.p, red);
-    ++m;
-    rc = drive(
-        c,
-        [&]() {
-            launch_axpy_norm<double>(c->stream, g, sig, x, c->r64.p, S[m & 1], c->q64.p, red, c->next_events());
-            if (amg) (void)amg_vcycle(c, c->r64.p, g, c->state.p);
-            launch_dir_spmv_csr(c->stream, g, sop, dsrc, S[m & 1], S[(m + 1) & 1], c->q64.p, red,
-                                c->next_events());
-            ++m;
-        },
-        amg ? std::min(std::max(1, c->prm.check_interval), 4) : 0);
-    if (rc) return rc;
-    if (jac) launch_unscale(c->stream, rows, x, c->sig64.p);
+    bool ran = false;
+    // Plain CG keeps the two-kernel solve: unscaled, the iteration count follows the order of
+    // the sums (13 940 rows of the 32^3 glugging system: 604 to 638 iterations over ten orders),
+    // so another order would show in it, and it is the option that is used to compare against.
+    if (jac) {
+        HIPC(c, c->slots.ensure(resident_slot_words()));
+        if ((rc = solve_resident_csr(c, op, b, sig, x, c->q64.p, c->slots.p, c->count.p, ran))) return rc;
+    }
+    if (!ran) {
+        CsrOp sop = op;
+        if (jac) {
+            HIPC(c, c->cx64.ensure((size_t)0));
+            // scaled copy of the values: the Jacobi-PCG iterates as CG on D^-1/2 A D^-1/2
+            int64_t nnz = 0;
+            HIPC(c, hipMemcpy(&nnz, rowptr + rows, sizeof(int64_t), hipMemcpyDeviceToHost));
+            if (nnz < 0) return c->fail(SHK_BAD_ARG, "rowptr[rows] is negative");
+            HIPC(c, c->q64.ensure(std::max<int64_t>(rows, 1)));
+            HIPC(c, c->hx64.ensure(std::max<int64_t>(nnz, 1)));
+            launch_csr_scale(c->stream, op, c->sig64.p, c->hx64.p);
+            sop.vals = c->hx64.p;
+        }
+        Reduction red = reduction(c);
+        if (amg) red.pz = amg_pz(c->amg);
+        // the vector the next direction is formed from: r, or z = M r
+        const double *dsrc = amg ? amg_z(c->amg) : c->r64.p;
+        launch_cg_init<double, double>(c->stream, g, b, sig, x, c->r64.p, c->s64.p, red, c->prm.residual,
+                                       c->prm.max_iterations);
+        double *S[2] = {c->s64.p, c->t64.p};
+        int m = 0;
+        if (amg && (rc = amg_vcycle(c, c->r64.p, g, c->state.p))) return rc;
+        launch_dir_spmv_csr(c->stream, g, sop, dsrc, S[0], S[1], c->q64.p, red);
+        ++m;
+        rc = drive(
+            c,
+            [&]() {
+                launch_axpy_norm<double>(c->stream, g, sig, x, c->r64.p, S[m & 1], c->q64.p, red, c->next_events());
+                if (amg) (void)amg_vcycle(c, c->r64.p, g, c->state.p);
+                launch_dir_spmv_csr(c->stream, g, sop, dsrc, S[m & 1], S[(m + 1) & 1], c->q64.p, red,
+                                    c->next_events());
+                ++m;
+            },
+            amg ? std::min(std::max(1, c->prm.check_interval), 4) : 0);
+        if (rc) return rc;
+        if (jac) launch_unscale(c->stream, rows, x, c->sig64.p);
+    }
     HIPC(c, hipEventRecord(c->ev[1], c->stream));
     res->count = c->h_state->iter;
     res->status = c->h_state->status;

@@ -215,6 +215,10 @@ Reduction reduction(shk_ctx *c);
 template <class T>
 int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces, double tol_rel,
                    int64_t max_iter, bool &ran);
+// The same for a CSR system, Jacobi-scaled by sig (x unscaled on return).  longest: 8 bytes of
+// device scratch that launch_csr_diag has filled; slots: resident_slot_words() words.
+int solve_resident_csr(shk_ctx *c, const CsrOp &op, const double *rhs, const double *sig, double *x, double *pub,
+                       unsigned long long *slots, const unsigned long long *longest, bool &ran);
 BrickOp<double> op64(shk_ctx *c);
 BrickOp<float> op32(shk_ctx *c);
 // r = b - A x (FP64); out = {max|r|, sum r^2, sum b^2, max|b|}; optionally the

@@ -117,6 +117,13 @@ hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &
                        T *x, T *faces, unsigned long long *slots, SolveState *state, SolveState *h_state,
                        double tol_rel, int64_t max_iter, int device, int cus);
 
+// The same for a CSR matrix whose longest row has `longest` entries (bpw: rows per thread);
+// sig: solve the scaled system D^-1/2 A D^-1/2 and return the unscaled x.  pub: rows doubles.
+ResidentPlan resident_csr_plan(int64_t rows, int64_t longest, int device, int cus);
+hipError_t resident_csr(hipStream_t st, const ResidentPlan &p, const CsrOp &op, const double *rhs, const double *sig,
+                        double *x, double *pub, unsigned long long *slots, SolveState *state, SolveState *h_state,
+                        double tol_rel, int64_t max_iter, int device, int cus);
+
 // r = b - A x in FP64 (unscaled operator with its diagonal); part holds 4*blocks
 // partials; out = {max|r|, sum r^2, sum b^2, max|b|}.  Optionally rs = (float)
 // (sig * r) (or (float) r without sig): the next inner solve's right-hand side.
@@ -159,7 +166,8 @@ void launch_add_correction(hipStream_t st, int64_t n, double *x, const float *d,
 // x *= sig: back from the scaled unknowns.
 void launch_unscale(hipStream_t st, int64_t n, double *x, const double *sig);
 // diag[row] = A[row,row], sig[row] = 1/sqrt(diag) (0 if not positive).
-void launch_csr_diag(hipStream_t st, const CsrOp &op, double *diag, double *sig);
+// longest (nullable, must be 0 before): the entries of the longest row.
+void launch_csr_diag(hipStream_t st, const CsrOp &op, double *diag, double *sig, unsigned long long *longest = nullptr);
 // out = values of D^-1/2 A D^-1/2 on A's pattern.
 void launch_csr_scale(hipStream_t st, const CsrOp &op, const double *sig, double *out);
 

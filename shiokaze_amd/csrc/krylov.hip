@@ -692,8 +692,16 @@ __global__ __launch_bounds__(NT) void k_unscale(int64_t n, double *__restrict__ 
     if (e < n) x[e] *= sig[e];
 }
 
-__global__ __launch_bounds__(NT) void k_csr_diag(CsrOp op, double *__restrict__ diag, double *__restrict__ sig) {
+__global__ __launch_bounds__(NT) void k_csr_diag(CsrOp op, double *__restrict__ diag, double *__restrict__ sig,
+                                                 unsigned long long *__restrict__ longest) {
+    __shared__ double lds[NT / kWave];
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
+    if (longest) {
+        // a length below zero (rowptr out of order) counts as one that fits nowhere
+        const int64_t n = e < op.rows ? op.rowptr[e + 1] - op.rowptr[e] : 0;
+        const double len = block_max<NT>(n < 0 ? 1e18 : (double)n, lds);
+        if (threadIdx.x == 0) atomicMax(longest, (unsigned long long)len);
+    }
     if (e < op.rows) {
         double dv = 0.0;
         for (int64_t p = op.rowptr[e]; p < op.rowptr[e + 1]; ++p)
@@ -929,8 +937,8 @@ void launch_unscale(hipStream_t st, int64_t n, double *x, const double *sig) {
     hipLaunchKernelGGL(k_unscale, dim3(blocks_for(n)), dim3(NT), 0, st, n, x, sig);
 }
 
-void launch_csr_diag(hipStream_t st, const CsrOp &op, double *diag, double *sig) {
-    hipLaunchKernelGGL(k_csr_diag, dim3(blocks_for(op.rows)), dim3(NT), 0, st, op, diag, sig);
+void launch_csr_diag(hipStream_t st, const CsrOp &op, double *diag, double *sig, unsigned long long *longest) {
+    hipLaunchKernelGGL(k_csr_diag, dim3(blocks_for(op.rows)), dim3(NT), 0, st, op, diag, sig, longest);
 }
 
 void launch_csr_scale(hipStream_t st, const CsrOp &op, const double *sig, double *out) {

@@ -114,27 +114,37 @@ int shk_solve_csr_noalloc(shk_ctx *c, int64_t rows, const int64_t *rowptr, const
     CsrOp sop = op;
     const Grid g = make_grid(rows);
     HIPC(c, hipEventRecord(c->ev[0], c->stream));
-    launch_csr_diag(c->stream, op, diag, sig);
-    if (jac) {
-        // the Jacobi-PCG iterates as CG on D^-1/2 A D^-1/2 (scaled copy of the values)
-        double *hv = take((size_t)std::max<int64_t>(nnz, 1));
-        launch_csr_scale(c->stream, op, sig, hv);
-        sop.vals = hv;
-    }
     const double *sg = jac ? sig : nullptr;
-    const Reduction red{pa, pb, c->state.p};
-    launch_cg_init<double, double>(c->stream, g, b, sg, x, r, s0, red, c->prm.residual, c->prm.max_iterations);
-    double *S[2] = {s0, s1};
-    int m = 0;
-    launch_dir_spmv_csr(c->stream, g, sop, r, S[0], S[1], q, red);
-    ++m;
-    int rc = drive(c, [&]() {
-        launch_axpy_norm<double>(c->stream, g, sg, x, r, S[m & 1], q, red);
-        launch_dir_spmv_csr(c->stream, g, sop, r, S[m & 1], S[(m + 1) & 1], q, red);
+    HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
+    launch_csr_diag(c->stream, op, diag, sig, c->count.p);
+    int rc = SHK_OK;
+    bool ran = false;
+    // the same choice as shk_solve_csr; the exchange slots go where the scaled values of the
+    // two-kernel solve would, which a solve this small never fills to the scratch's end
+    if (jac && (size_t)(cur - static_cast<double *>(base)) + resident_slot_words() <= kScratchBytes / sizeof(double) &&
+        (rc = solve_resident_csr(c, op, b, sg, x, q, reinterpret_cast<unsigned long long *>(cur), c->count.p, ran)))
+        return rc;
+    if (!ran) {
+        if (jac) {
+            // the Jacobi-PCG iterates as CG on D^-1/2 A D^-1/2 (scaled copy of the values)
+            double *hv = take((size_t)std::max<int64_t>(nnz, 1));
+            launch_csr_scale(c->stream, op, sig, hv);
+            sop.vals = hv;
+        }
+        const Reduction red{pa, pb, c->state.p};
+        launch_cg_init<double, double>(c->stream, g, b, sg, x, r, s0, red, c->prm.residual, c->prm.max_iterations);
+        double *S[2] = {s0, s1};
+        int m = 0;
+        launch_dir_spmv_csr(c->stream, g, sop, r, S[0], S[1], q, red);
         ++m;
-    });
-    if (rc) return rc;
-    if (jac) launch_unscale(c->stream, rows, x, sig);
+        rc = drive(c, [&]() {
+            launch_axpy_norm<double>(c->stream, g, sg, x, r, S[m & 1], q, red);
+            launch_dir_spmv_csr(c->stream, g, sop, r, S[m & 1], S[(m + 1) & 1], q, red);
+            ++m;
+        });
+        if (rc) return rc;
+        if (jac) launch_unscale(c->stream, rows, x, sig);
+    }
     HIPC(c, hipEventRecord(c->ev[1], c->stream));
     res->count = c->h_state->iter;
     res->status = c->h_state->status;
