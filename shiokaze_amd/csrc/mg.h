@@ -59,10 +59,32 @@ struct MgLevelDev {
 
 constexpr int kMgCoarseMax = 64;  // cells of the coarsest level (<= 4 per axis)
 
+// The coarse end of the hierarchy, run by one workgroup out of LDS: as many of the last
+// levels as hold kMgTailCells cells together (24 bytes a cell: 156 of the 160 KB) as dense
+// grids with a zero cell after each row, a zero row after each plane (3D) and a zero plane
+// before the first level and after each.  3D grids always get their last three levels
+// (at most 17^2 + 17^3 + 9^3 + 5^3).
+constexpr int kMgTailCells = 6656, kMgTailLevels = 12;
+struct MgTail {
+    int levels = 0;                    // the coarsest included
+    int first[kMgTailLevels + 1] = {};  // first[t] .. first[t + 1]: the cells of level t
+    int nx[kMgTailLevels] = {}, ny[kMgTailLevels] = {}, nz[kMgTailLevels] = {};
+    int sxy[kMgTailLevels] = {};       // cells of a plane (rows: nx + 1)
+    const float4 *op = nullptr;        // d, cx, cy, cz per cell
+    const int *src = nullptr;          // cells of the first level in its bricks, -1 outside them
+    const float *b = nullptr;          // of the first level, in its bricks
+    float *x = nullptr;
+    // coarsest level: unknowns, their cells, dense inverse by columns of kMgCoarseMax
+    int ncoarse = 0;
+    const int *idx = nullptr;
+    const float *inv = nullptr;
+};
+
 // level-0 diagonal of the scaled system: 1 on unknowns (sig > 0), else 0
 void launch_mg_mask(hipStream_t st, int64_t n, const double *sig, float *d0);
-// coarse operator of level `c` from level `f`
-void launch_mg_coarsen(hipStream_t st, const MgLevelDev &f, const MgLevelDev &c);
+// coarse operator of level `c` from level `f`; dense (may be null): also as a dense grid
+// of row stride sx and plane stride sxy (cells of missing bricks are not written)
+void launch_mg_coarsen(hipStream_t st, const MgLevelDev &f, const MgLevelDev &c, float4 *dense, int sx, int sxy);
 // b_c = P0' (b_f - A_f x_f), x_c = w b_c / d_c (or 0 with w = 0): the residual of a
 // level >= 1 and its restriction in one pass, the residual never stored
 void launch_mg_residual_restrict(hipStream_t st, const MgLevelDev &f, const MgLevelDev &c, float omega,
@@ -85,8 +107,8 @@ void launch_mg_pre0(hipStream_t st, const MgOp &op, const float *r, const int4 *
 void launch_mg_post0(hipStream_t st, const MgOp &op, const int4 *coord, const int *parent, const float *r,
                      const float *xc, float *y, const SolveState *state, const Grid &g, double *cell_part,
                      double *part);
-// coarsest level: x[idx[i]] = sum_j inv[i][j] b[idx[j]] (n <= kMgCoarseMax), other cells 0
-void launch_mg_coarse(hipStream_t st, int n, const int *idx, const float *inv, const float *b, float *x,
-                      int cells, const SolveState *state);
+// the levels of t, from the first one's b and x (pre-smoothed) to its x after the
+// post-smoothing, the coarsest solved exactly: x[idx[i]] = sum_j inv[i][j] b[idx[j]]
+void launch_mg_tail(hipStream_t st, int bx, const MgTail &t, float omega, float alpha, const SolveState *state);
 
 }  // namespace shk

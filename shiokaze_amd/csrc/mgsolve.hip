@@ -30,9 +30,13 @@ struct MgHierarchy {
     DevBuf<float> z;          // the preconditioned residual z = M r (level 0 bricks)
     DevBuf<double> pz;        // r.z partials (one per Krylov workgroup)
     DevBuf<double> pcell;     // r.z sums of the post-smoothing blocks (one per 256 cells)
-    DevBuf<int> cidx;         // coarsest: active cell indices
+    DevBuf<int> cidx;         // coarsest: active cells
     DevBuf<float> cinv;       // coarsest: dense inverse on them
-    int ncoarse = 0;
+    int ltail = 0;            // first level of the tail
+    MgTail tail;
+    DevBuf<float4> tail_op;   // the tail levels' operators as dense grids
+    DevBuf<int> tail_src;
+    std::vector<int> h_tail;
     std::vector<int> key;     // level-0 brick table the host tables were built for
     int key_dims[3] = {0, 0, 0};
 };
@@ -126,12 +130,48 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
             }
         }
     }
+    // the tail: the last levels, as long as their cells fit
+    MgTail &T = h->tail = MgTail{};
+    h->ltail = (int)h->lv.size();
+    const auto plane = [&](const MgLevelDev &v) { return (int64_t)(v.nx + 1) * (ay > 1 ? v.ny + 1 : 1); };
+    for (int64_t l = h->ltail - 1, sum = 0; l >= 1 && h->ltail > (int)h->lv.size() - kMgTailLevels; --l) {
+        const MgLevelDev &v = h->lv[l].v;
+        sum += plane(v) * (v.nz + 1);
+        if (sum + plane(v) > kMgTailCells) break;
+        h->ltail = (int)l;
+    }
+    T.first[0] = (int)plane(h->lv[h->ltail].v);
+    for (size_t l = h->ltail; l < h->lv.size(); ++l, ++T.levels) {
+        const MgLevelDev &v = h->lv[l].v;
+        const int t = T.levels;
+        T.nx[t] = v.nx;
+        T.ny[t] = v.ny;
+        T.nz[t] = v.nz;
+        T.sxy[t] = (int)plane(v);
+        T.first[t + 1] = T.first[t] + T.sxy[t] * (v.nz + 1);
+    }
+    const MgLevelHost &LT = h->lv[h->ltail];
+    h->h_tail.assign(T.first[1] - T.first[0], -1);
+    for (int k = 0; k < LT.v.nz; ++k)
+        for (int j = 0; j < LT.v.ny; ++j)
+            for (int i = 0; i < LT.v.nx; ++i) {
+                const int s = LT.h_slot[i / ex + LT.v.nbx * (j / ey + LT.v.nby * (k / ez))];
+                if (s < 0) continue;
+                h->h_tail[i + (LT.v.nx + 1) * j + T.sxy[0] * k] =
+                    s * kBrickCells + i % ex + ex * (j % ey) + kWave * (k % ez);
+            }
     h->key = c->h_slot;
     h->key_dims[0] = c->dims.nx;
     h->key_dims[1] = c->dims.ny;
     h->key_dims[2] = c->dims.nz;
     // device copies
     hipStream_t st = c->stream;
+    HIPC(c, h->tail_op.ensure((size_t)T.first[T.levels]));
+    HIPC(c, h->tail_src.ensure(h->h_tail.size()));
+    // the cells between and of missing bricks stay zero
+    HIPC(c, hipMemsetAsync(h->tail_op.p, 0, sizeof(float4) * (size_t)T.first[T.levels], st));
+    HIPC(c, hipMemcpyAsync(h->tail_src.p, h->h_tail.data(), sizeof(int) * h->h_tail.size(), hipMemcpyHostToDevice,
+                           st));
     for (size_t l = 0; l < h->lv.size(); ++l) {
         MgLevelHost &L = h->lv[l];
         const size_t n = (size_t)std::max(L.v.n_active, 1) * kBrickCells;
@@ -150,7 +190,8 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
             HIPC(c, L.d.ensure(n));
         }
         if (l > 0)  // level 0 keeps no vectors: its residual is restricted where it is computed
-            for (DevBuf<float> *b : {&L.b, &L.x, &L.t}) HIPC(c, b->ensure(n));
+            for (DevBuf<float> *b : {&L.b, &L.x, &L.t})
+                if (b != &L.t || (int)l < h->ltail) HIPC(c, b->ensure(n));
         if (!L.h_parent.empty()) {
             HIPC(c, L.parent.ensure(L.h_parent.size()));
             HIPC(c, hipMemcpyAsync(L.parent.p, L.h_parent.data(), sizeof(int) * L.h_parent.size(),
@@ -162,8 +203,8 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
     return SHK_OK;
 }
 
-// dense inverse (Cholesky, FP64) of the coarsest operator on its active cells;
-// the diagonal inverse when that operator is not positive definite
+// dense inverse (Cholesky, FP64) of the coarsest operator on its active cells, by
+// columns of kMgCoarseMax; the diagonal inverse when that operator is not positive definite
 void coarse_inverse(int bx, const std::vector<float> &d, const std::vector<float> &cx, const std::vector<float> &cy,
                     const std::vector<float> &cz, std::vector<int> &idx, std::vector<float> &inv) {
     const int ex = bx, ey = kWave / bx;
@@ -205,9 +246,10 @@ void coarse_inverse(int bx, const std::vector<float> &d, const std::vector<float
             Lm[(size_t)i * n + j] = t / ljj;
         }
     }
-    inv.assign((size_t)n * n, 0.0f);
+    inv.assign((size_t)kMgCoarseMax * kMgCoarseMax, 0.0f);
+    if (n > kMgCoarseMax) return;
     if (!ok) {
-        for (int i = 0; i < n; ++i) inv[(size_t)i * n + i] = (float)(1.0 / A[(size_t)i * n + i]);
+        for (int i = 0; i < n; ++i) inv[(size_t)i * kMgCoarseMax + i] = (float)(1.0 / A[(size_t)i * n + i]);
         return;
     }
     // columns of A^-1 by forward and back substitution
@@ -223,7 +265,7 @@ void coarse_inverse(int bx, const std::vector<float> &d, const std::vector<float
             for (int k = i + 1; k < n; ++k) s -= Lm[(size_t)k * n + i] * xcol[k];
             xcol[i] = s / Lm[(size_t)i * n + i];
         }
-        for (int i = 0; i < n; ++i) inv[(size_t)i * n + col] = (float)xcol[i];
+        for (int i = 0; i < n; ++i) inv[(size_t)col * kMgCoarseMax + i] = (float)xcol[i];
     }
 }
 
@@ -237,6 +279,8 @@ void mg_destroy(MgHierarchy *h) {
     h->pcell.release();
     h->cidx.release();
     h->cinv.release();
+    h->tail_op.release();
+    h->tail_src.release();
     delete h;
 }
 
@@ -268,27 +312,41 @@ int mg_setup(shk_ctx *c) {
         L.v.x = L.x.p;
         L.v.t = L.t.p;
     }
+    h->tail.op = h->tail_op.p;
+    h->tail.src = h->tail_src.p;
+    h->tail.b = h->lv[h->ltail].v.b;
+    h->tail.x = h->lv[h->ltail].v.x;
     for (size_t l = 1; l < h->lv.size(); ++l)
-        if (h->lv[l].v.n_active) launch_mg_coarsen(st, h->lv[l - 1].v, h->lv[l].v);
+        if (h->lv[l].v.n_active) {
+            const int t = (int)l - h->ltail;
+            const MgTail &T = h->tail;
+            launch_mg_coarsen(st, h->lv[l - 1].v, h->lv[l].v, t >= 0 ? h->tail_op.p + T.first[t] : nullptr,
+                              t >= 0 ? T.nx[t] + 1 : 0, t >= 0 ? T.sxy[t] : 0);
+        }
     HIPC(c, hipGetLastError());
     // coarsest level: one brick at most
     MgLevelHost &C = h->lv.back();
     std::vector<float> hd(kBrickCells, 0.0f), hx(kBrickCells, 0.0f), hy(kBrickCells, 0.0f), hz(kBrickCells, 0.0f);
     if (C.v.n_active >= 1) {
-        HIPC(c, hipMemcpyAsync(hd.data(), C.d.p, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
-        HIPC(c, hipMemcpyAsync(hx.data(), C.cx.p, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
-        HIPC(c, hipMemcpyAsync(hy.data(), C.cy.p, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
-        HIPC(c, hipMemcpyAsync(hz.data(), C.cz.p, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
+        HIPC(c, hipMemcpyAsync(hd.data(), C.v.d, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
+        HIPC(c, hipMemcpyAsync(hx.data(), C.v.cx, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
+        HIPC(c, hipMemcpyAsync(hy.data(), C.v.cy, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
+        HIPC(c, hipMemcpyAsync(hz.data(), C.v.cz, sizeof(float) * kBrickCells, hipMemcpyDeviceToHost, st));
     }
     HIPC(c, hipStreamSynchronize(st));
     std::vector<int> idx;
     std::vector<float> inv;
     coarse_inverse(c->dims.bx, hd, hx, hy, hz, idx, inv);
     if ((int)idx.size() > kMgCoarseMax) return c->fail(SHK_HIP_ERROR, "multigrid: coarsest level too large");
-    h->ncoarse = (int)idx.size();
+    h->tail.ncoarse = (int)idx.size();
     HIPC(c, h->cidx.ensure(std::max<size_t>(idx.size(), 1)));
     HIPC(c, h->cinv.ensure(std::max<size_t>(inv.size(), 1)));
+    h->tail.idx = h->cidx.p;
+    h->tail.inv = h->cinv.p;
     if (!idx.empty()) {
+        const int ex = c->dims.bx, ey = kWave / ex;
+        for (int &e : idx)
+            e = e % ex + (C.v.nx + 1) * ((e / ex) % ey) + h->tail.sxy[h->tail.levels - 1] * (e / kWave);
         HIPC(c, hipMemcpyAsync(h->cidx.p, idx.data(), sizeof(int) * idx.size(), hipMemcpyHostToDevice, st));
         HIPC(c, hipMemcpyAsync(h->cinv.p, inv.data(), sizeof(float) * inv.size(), hipMemcpyHostToDevice, st));
     }
@@ -309,18 +367,18 @@ void mg_vcycle(shk_ctx *c, const float *r, float *z, const SolveState *state, co
     // level from the residual of the level above, computed where it is restricted
     // (x_L = 0: w = 0)
     launch_mg_pre0(st, op0, r, c->coord.p, L0.parent.p, h->lv[1].v, L > 1 ? w : 0.0f, state);
-    for (int l = 1; l < L; ++l) {
+    for (int l = 1; l < h->ltail; ++l) {
         MgLevelHost &F = h->lv[l], &C = h->lv[l + 1];
         if (!C.v.n_active) continue;
         launch_mg_residual_restrict(st, F.v, C.v, l + 1 < L ? w : 0.0f, state);
     }
-    MgLevelHost &Cl = h->lv[L];
-    if (Cl.v.n_active) launch_mg_coarse(st, h->ncoarse, h->cidx.p, h->cinv.p, Cl.v.b, Cl.v.x, kBrickCells, state);
-    // up: the correction from the coarsest level, then the post-smoothing of each level,
-    // which also applies the correction of the level above it (level 0's is applied
-    // in its post-smoothing)
-    if (L > 1 && h->lv[L - 1].v.n_active) launch_mg_prolong(st, h->lv[L - 1].v, Cl.v, a, state);
-    for (int l = L - 1; l >= 1; --l) {
+    launch_mg_tail(st, c->dims.bx, h->tail, w, a, state);
+    // up: the correction from the tail, then the post-smoothing of each level above it,
+    // which also applies the correction of the next (level 0's is applied in its
+    // post-smoothing)
+    if (h->ltail > 1 && h->lv[h->ltail - 1].v.n_active)
+        launch_mg_prolong(st, h->lv[h->ltail - 1].v, h->lv[h->ltail].v, a, state);
+    for (int l = h->ltail - 1; l >= 1; --l) {
         MgLevelHost &F = h->lv[l];
         if (!F.v.n_active) continue;
         launch_mg_smooth(st, F.v, l > 1 ? &h->lv[l - 1].v : nullptr, w, a, state);
