@@ -24,9 +24,10 @@ struct Reduction {
     double *pa;       // s.q partials (>= blocks)
     double *pb;       // r.r and max|r| partials (>= 2 * blocks)
     SolveState *st;   // device state
-    // with a preconditioner z = M r: the r.z partials (>= blocks) written by the last
-    // kernel of M; dir_spmv is then given z in place of r and takes rho = r.z
+    // with a preconditioner z = M r: the r.z partials (nz; 0: one per workgroup) written by
+    // the last kernel of M; dir_spmv is then given z in place of r and takes rho = r.z
     double *pz = nullptr;
+    int nz = 0;
 };
 
 // Operator views.  Brick: vectors hold n_active bricks of 8x8x8 cells, x-fastest

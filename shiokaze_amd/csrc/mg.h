@@ -102,11 +102,14 @@ void launch_mg_smooth(hipStream_t st, const MgLevelDev &c, const MgLevelDev *fin
 void launch_mg_pre0(hipStream_t st, const MgOp &op, const float *r, const int4 *coord, const int *parent,
                     const MgLevelDev &c1, float omega_c, const SolveState *state);
 // y = x0' + w (r - A x0') with x0' = w r + alpha P0 x1 (prolongation fused into the
-// post-smoothing), one thread per cell; the r.y sums of its blocks (cell_part, one per
-// 256 cells) are folded in order into g.blocks partials `part` for the Krylov kernels
+// post-smoothing); the r.y sums of its blocks are mg_partials(op.n_active) partials `part`
+// for every Krylov workgroup to fold: those of the blocks themselves up to kMgMaxPartials,
+// above it folded in order from cell_part (at 5,102 the folding of all of them in every
+// workgroup costs the Krylov kernel the 4.4 us of the extra launch)
+constexpr int kMgMaxPartials = 2048;
+int mg_partials(int n_active);
 void launch_mg_post0(hipStream_t st, const MgOp &op, const int4 *coord, const int *parent, const float *r,
-                     const float *xc, float *y, const SolveState *state, const Grid &g, double *cell_part,
-                     double *part);
+                     const float *xc, float *y, const SolveState *state, double *cell_part, double *part);
 // the levels of t, from the first one's b and x (pre-smoothed) to its x after the
 // post-smoothing, the coarsest solved exactly: x[idx[i]] = sum_j inv[i][j] b[idx[j]]
 void launch_mg_tail(hipStream_t st, int bx, const MgTail &t, float omega, float alpha, const SolveState *state);

@@ -1,7 +1,8 @@
 // mg.hip -- aggregation multigrid V-cycle kernels on the brick layout (see mg.h).
 //
-// Every kernel returns at once when the Krylov state it is given has stopped, so
-// the V-cycles queued behind a converged iteration cost only their launches.
+// Every kernel returns when the Krylov state it is given has stopped, before it reads a
+// vector, so the V-cycles queued behind a converged iteration cost little more than their
+// launches; the brick tables are read before the state, so that the loads overlap.
 #include "mg.h"
 
 namespace shk {
@@ -170,7 +171,6 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(MgLevelDev f, MgLev
     using A = Agg<BX>;
     constexpr int X = A::X, Y = A::Y;
     static_assert(kBrickCells % NT == 0 && NT % (2 * kWave) == 0, "a block holds whole z pairs of one brick");
-    if (stopped(state)) return;
     __shared__ float ts[NT];
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
     if (e >= (int64_t)f.n_active * kBrickCells) return;  // whole blocks: n_active * 512 is a multiple of NT
@@ -179,6 +179,7 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(MgLevelDev f, MgLev
     // cell's diagonal, then the residual's operands (all in bounds whatever d is)
     const int ps = f.parent[slot];  // >= 0: the parent of an active brick is active
     const int64_t E = (int64_t)(ps > 0 ? ps : 0) * kBrickCells + coarse_local<BX>(f.coord[slot], l);
+    if (stopped(state)) return;
     const float dc = c.d[E];
     const MgOp op = f.op(0.0f, 0.0f);
     const float *__restrict__ xf = f.x;
@@ -199,14 +200,14 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(MgLevelDev f, MgLev
 // level above the coarsest; the others get theirs from k_mg_smooth)
 template <int BX>
 __global__ __launch_bounds__(NT) void k_mg_prolong(MgLevelDev f, MgLevelDev c, float alpha, const SolveState *state) {
-    if (stopped(state)) return;
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
     if (e >= (int64_t)f.n_active * kBrickCells) return;
     const int slot = (int)(e >> 9), l = (int)(e & 511);
-    if (!(f.d[e] > 0.0f)) return;
-    const int ps = f.parent[slot];
-    if (ps < 0) return;  // cannot happen: the parent of an active brick is active
-    f.x[e] = fmaf(alpha, c.x[(int64_t)ps * kBrickCells + coarse_local<BX>(f.coord[slot], l)], f.x[e]);
+    const int ps = f.parent[slot];  // >= 0: the parent of an active brick is active
+    const int64_t E = (int64_t)(ps > 0 ? ps : 0) * kBrickCells + coarse_local<BX>(f.coord[slot], l);
+    if (stopped(state)) return;
+    const float dv = f.d[e], xe = f.x[e], xc = c.x[E];
+    if (dv > 0.0f && ps >= 0) f.x[e] = fmaf(alpha, xc, xe);
 }
 
 // c.t = y = x + w (b - A x) / d on a level >= 1, one thread per cell; with a finer
@@ -217,13 +218,13 @@ template <int BX>
 __global__ __launch_bounds__(NT) void k_mg_smooth(MgLevelDev c, MgLevelDev f, bool prolong, float omega, float alpha,
                                                   const SolveState *state) {
     using A = Agg<BX>;
-    if (stopped(state)) return;
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
     if (e >= (int64_t)c.n_active * kBrickCells) return;
     const int slot = (int)(e >> 9), l = (int)(e & 511);
     // the children's d and x are loaded with the smoothing's operands, not after them
     int base = 0;
     const int fs = prolong ? children<BX>(f, c, slot, l, base) : -1;
+    if (stopped(state)) return;
     const int64_t fb = (int64_t)(fs > 0 ? fs : 0) * kBrickCells + base;
     float fd[A::NCH], fx[A::NCH];
 #pragma unroll
@@ -257,9 +258,11 @@ __device__ inline float xprime(const MgOp &op, const float *__restrict__ r, cons
 
 // ---------------------------------------------------------------- level 0, one wave per brick
 //
-// The two level-0 passes with one wave per brick: lane = i + X j holds one (x, y)
-// column (X x Y = 64: 8 x 8 for 3D bricks, 64 x 1 for the 64x1x8 bricks of 2D grids)
-// and walks the brick's 8 z-planes.  In-brick x and y neighbours come by lane
+// The two level-0 passes with PL z-planes of a brick per wave: lane = i + X j holds one
+// (x, y) column (X x Y = 64: 8 x 8 for 3D bricks, 64 x 1 for the 64x1x8 bricks of 2D grids)
+// of the planes.  PL = 8, the whole brick, reads least; PL = 2 puts four times the waves on
+// the chip and quarters each one's chain of shuffles, which is what bounds a small grid
+// (kMgSplitBricks).  In-brick x and y neighbours come by lane
 // shuffles (taken by all 64 lanes, outside any lane-dependent branch), z neighbours
 // from the lane's own registers, and the cells across the faces from one coalesced
 // load per neighbour plane (the neighbour brick's slot, coordinates and parent are
@@ -291,13 +294,15 @@ __device__ inline void halo_planes(const int nb[6], int lane, V value, float h[6
 }
 
 // the six neighbour values of cell (i, j, k) in face order x-, x+, y-, y+, z-, z+
-// (y values 0 without a y axis)
-template <int BX>
-__device__ inline void neighbours6(const float *v, const float h[6], int lane, int k, float n[6]) {
+// (y values 0 without a y axis); v: the wave's planes k0 .. k0 + PL - 1, zl and zh those
+// around them
+template <int BX, int PL>
+__device__ inline void neighbours6(const float *v, const float h[6], float zl, float zh, int lane, int k0, int p,
+                                   float n[6]) {
     using B = BrickShape<BX>;
     constexpr int X = B::X, Y = B::Y;
-    const int i = lane % X, j = lane / X;
-    const float x0 = v[k];
+    const int i = lane % X, j = lane / X, k = k0 + p;
+    const float x0 = v[p];
     float xm = lane_get(x0, lane - 1), xp = lane_get(x0, lane + 1);
     const float hxm = lane_get(h[0], j + Y * k), hxp = lane_get(h[1], j + Y * k);
     if (i == 0) xm = hxm;
@@ -314,8 +319,8 @@ __device__ inline void neighbours6(const float *v, const float h[6], int lane, i
     n[1] = xp;
     n[2] = ym;
     n[3] = yp;
-    n[4] = k > 0 ? v[k - 1] : h[4];
-    n[5] = k < 7 ? v[k + 1] : h[5];
+    n[4] = p > 0 ? v[p > 0 ? p - 1 : 0] : zl;
+    n[5] = p < PL - 1 ? v[p < PL - 1 ? p + 1 : p] : zh;
 }
 
 // the couplings of cell e across its faces (low faces live at e, high faces at the
@@ -350,16 +355,24 @@ __device__ inline void couplings6(const MgOp &op, int64_t e, const int nb[6], in
     c[5] = k < 7 ? op.cz[e + 64] : (nb[5] >= 0 ? op.cz[(int64_t)nb[5] * kBrickCells + lane] : 0.0f);
 }
 
+// the brick and the first plane of this wave
+template <int PL>
+__device__ inline int wave_brick(int &k0) {
+    const int w = blockIdx.x * (NT / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    k0 = PL * (w % (8 / PL));
+    return w / (8 / PL);
+}
+
 // t0 = r - A (w r) = r - w A r on the unknowns (0 elsewhere), by linearity, restricted
 // at once to level 1 (b_1 = P0' t0, x_1 = w_c b_1 / d_1)
-template <int BX>
+template <int BX, int PL>
 __global__ __launch_bounds__(NT) void k_mg_pre0_w(MgOp op, const float *__restrict__ r, const int4 *__restrict__ coord,
                                                   const int *__restrict__ parent, MgLevelDev c, float omega_c,
                                                   const SolveState *state) {
     constexpr int X = BrickShape<BX>::X, Y = BrickShape<BX>::Y;
-    if (stopped(state)) return;
     const int lane = threadIdx.x & 63;
-    const int slot = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+    int k0;
+    const int slot = wave_brick<PL>(k0);
     if (slot >= op.n_active) return;   // no block-wide synchronisation below
     int nb[6];
 #pragma unroll
@@ -368,42 +381,47 @@ __global__ __launch_bounds__(NT) void k_mg_pre0_w(MgOp op, const float *__restri
     const int64_t base = (int64_t)slot * kBrickCells + lane;
     const int ps = parent[slot];  // >= 0: the parent of an active brick is active
     const int4 Bf = coord[slot];
-    float dcm[4];  // level-1 diagonals of the cells this lane may restrict to, loaded early
+    if (stopped(state)) return;
+    float dcm[PL / 2];  // level-1 diagonals of the cells this lane may restrict to, loaded early
 #pragma unroll
-    for (int m = 0; m < 4; ++m) dcm[m] = c.d[(int64_t)(ps > 0 ? ps : 0) * kBrickCells + coarse_local<BX>(Bf, lane + 128 * m)];
-    float v[8];
+    for (int m = 0; m < PL / 2; ++m)
+        dcm[m] = c.d[(int64_t)(ps > 0 ? ps : 0) * kBrickCells + coarse_local<BX>(Bf, lane + 64 * (k0 + 2 * m))];
+    const auto value = [&](int ns, int l) { return r[(int64_t)ns * kBrickCells + l]; };
+    float v[PL];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = r[base + 64 * k];
+    for (int p = 0; p < PL; ++p) v[p] = r[base + 64 * (k0 + p)];
     float h[6];
-    halo_planes<BX>(nb, lane, [&](int ns, int l) { return r[(int64_t)ns * kBrickCells + l]; }, h);
-    float t[8];
+    halo_planes<BX>(nb, lane, value, h);
+    const float zl = k0 > 0 ? value(slot, lane + 64 * (k0 - 1)) : h[4];
+    const float zh = k0 + PL < 8 ? value(slot, lane + 64 * (k0 + PL)) : h[5];
+    float t[PL];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int64_t e = base + 64 * k;
+    for (int p = 0; p < PL; ++p) {
+        const int64_t e = base + 64 * (k0 + p);
         float n[6];
-        neighbours6<BX>(v, h, lane, k, n);
+        neighbours6<BX, PL>(v, h, zl, zh, lane, k0, p, n);
         float ax;
         if (kap != 0.0f) {
             // the y terms are 0.0f without a y axis
-            ax = v[k] - kap * (n[0] + n[1] + (Y > 1 ? n[2] : 0.0f) + (Y > 1 ? n[3] : 0.0f) + n[4] + n[5]);
+            ax = v[p] - kap * (n[0] + n[1] + (Y > 1 ? n[2] : 0.0f) + (Y > 1 ? n[3] : 0.0f) + n[4] + n[5]);
         } else {
             float c[6];
             bool has[6];
-            couplings6<BX>(op, e, nb, lane, k, kap, c, has);
-            ax = op.d[e] * v[k];
+            couplings6<BX>(op, e, nb, lane, k0 + p, kap, c, has);
+            ax = op.d[e] * v[p];
 #pragma unroll
             for (int f = 0; f < 6; ++f)
                 if (has[f]) ax -= c[f] * n[f];
         }
-        t[k] = diag_of(op, e, kap) > 0.0f ? v[k] - op.omega * ax : 0.0f;
+        t[p] = diag_of(op, e, kap) > 0.0f ? v[p] - op.omega * ax : 0.0f;
     }
     // b_1 = P0' t and x_1 = w_c b_1 / d_1 on the coarse cells whose children are in
     // this brick: a cell of even (i, j, k) sums the children (i+a, j+b, k+c) in the
     // order a, b, c (that of Agg<BX>::child), taken from lanes +1, +X, +X+1 and its
     // own next register; t is not stored
-    float sum[4];
+    float sum[PL / 2];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < PL / 2; ++m) {
         float q[8];
 #pragma unroll
         for (int cz = 0; cz < 2; ++cz) {
@@ -428,8 +446,8 @@ __global__ __launch_bounds__(NT) void k_mg_pre0_w(MgOp op, const float *__restri
     const int i = lane % X, j = lane / X;
     if ((i & 1) || (Y > 1 && (j & 1)) || ps < 0) return;  // ps < 0 cannot happen for an active brick
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const int64_t E = (int64_t)ps * kBrickCells + coarse_local<BX>(Bf, lane + 64 * (2 * m));
+    for (int m = 0; m < PL / 2; ++m) {
+        const int64_t E = (int64_t)ps * kBrickCells + coarse_local<BX>(Bf, lane + 64 * (k0 + 2 * m));
         const float dc = dcm[m];
         c.b[E] = dc > 0.0f ? sum[m] : 0.0f;
         c.x[E] = dc > 0.0f ? omega_c * sum[m] / dc : 0.0f;
@@ -438,53 +456,57 @@ __global__ __launch_bounds__(NT) void k_mg_pre0_w(MgOp op, const float *__restri
 
 // y = x0' + w (r - A x0') with x0' = w r + alpha P0 x1 computed on the fly (the
 // prolongation fused into the post-smoothing); part[block] = sum r*y over the block's
-// bricks
-template <int BX>
+// planes
+template <int BX, int PL>
 __global__ __launch_bounds__(NT) void k_mg_post0_w(MgOp op, const int4 *__restrict__ coord,
                                                    const int *__restrict__ parent, const float *__restrict__ r,
                                                    const float *__restrict__ xc, float *__restrict__ y,
                                                    const SolveState *state, double *__restrict__ part) {
-    if (stopped(state)) return;
     __shared__ double lds[NT / kWave];
     const int lane = threadIdx.x & 63;
-    const int slot = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+    int k0;
+    const int slot = wave_brick<PL>(k0);
+    const int sl = slot < op.n_active ? slot : 0;
     double acc = 0.0;
+    int nb[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) nb[f] = op.nbr[6 * sl + f];
+    const float kap = brick_kappa(op, sl);
+    const int4 B = coord[sl];
+    const int ps = parent[sl];
+    if (stopped(state)) return;
     if (slot < op.n_active) {
-        int nb[6];
-#pragma unroll
-        for (int f = 0; f < 6; ++f) nb[f] = op.nbr[6 * slot + f];
-        const float kap = brick_kappa(op, slot);
-        const int4 B = coord[slot];
-        const int ps = parent[slot];
         const int64_t base = (int64_t)slot * kBrickCells + lane;
-        float rv[8], xs[8];
+        const auto own = [&](int k) { return xprime<BX>(op, r, xc, slot, lane + 64 * k, B, ps); };
+        float rv[PL], xs[PL];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            rv[k] = r[base + 64 * k];
-            xs[k] = xprime<BX>(op, r, xc, slot, lane + 64 * k, B, ps);
+        for (int p = 0; p < PL; ++p) {
+            rv[p] = r[base + 64 * (k0 + p)];
+            xs[p] = own(k0 + p);
         }
         float h[6];
         halo_planes<BX>(nb, lane,
                         [&](int ns, int l) { return xprime<BX>(op, r, xc, ns, l, coord[ns], parent[ns]); }, h);
+        const float zl = k0 > 0 ? own(k0 - 1) : h[4], zh = k0 + PL < 8 ? own(k0 + PL) : h[5];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int64_t e = base + 64 * k;
+        for (int p = 0; p < PL; ++p) {
+            const int64_t e = base + 64 * (k0 + p);
             float yv = 0.0f;
             // every lane takes part in the shuffles, whether its cell is an unknown or not
             float n[6];
-            neighbours6<BX>(xs, h, lane, k, n);
+            neighbours6<BX, PL>(xs, h, zl, zh, lane, k0, p, n);
             if (diag_of(op, e, kap) > 0.0f) {
                 float c[6];
                 bool has[6];
-                couplings6<BX>(op, e, nb, lane, k, kap, c, has);
+                couplings6<BX>(op, e, nb, lane, k0 + p, kap, c, has);
                 float sum = 0.0f;
 #pragma unroll
                 for (int f = 0; f < 6; ++f)
                     if (has[f] && c[f] != 0.0f) sum += c[f] * n[f];
-                yv = xs[k] + op.omega * (rv[k] - (xs[k] - sum));
+                yv = xs[p] + op.omega * (rv[p] - (xs[p] - sum));
             }
             y[e] = yv;
-            acc += (double)rv[k] * (double)yv;
+            acc += (double)rv[p] * (double)yv;
         }
     }
     const double s = block_sum<NT>(acc, lds);
@@ -492,7 +514,7 @@ __global__ __launch_bounds__(NT) void k_mg_post0_w(MgOp op, const int4 *__restri
 }
 
 // out[t] = sum of in[t*per .. (t+1)*per) for t < n_out, in a fixed order (the
-// per-block partials of k_mg_post0_w folded to the Krylov grid's partial count)
+// per-block partials of k_mg_post0_w, where the Krylov kernels should not fold them all)
 __global__ __launch_bounds__(NT) void k_mg_fold(int n_in, const double *__restrict__ in, int n_out,
                                                 double *__restrict__ out, const SolveState *state) {
     if (stopped(state)) return;
@@ -714,18 +736,44 @@ void launch_mg_smooth(hipStream_t st, const MgLevelDev &c, const MgLevelDev *fin
                   fine != nullptr, omega, alpha, state);
 }
 
+// Level-0 grids of up to this many bricks are split four ways per brick, above it the chip is
+// full and a wave keeps its brick.  One iteration, whole bricks / split: 70x61x52 (284 bricks)
+// 72.5 / 68.3 us (k_mg_pre0_w 6.6 / 4.7, k_mg_post0_w 8.5 / 5.8), 652,000 unknowns 99.1 / 95.7,
+// 842,000 109.6 / 107.7, 1,287,000 122.0 / 126.7, 1,645,000 125.1 / 131.0 us.
+constexpr int kMgSplitBricks = 2048;
+
+#define SHK_MG_LAUNCH0(kernel, op, ...)                                                            \
+    do {                                                                                           \
+        const bool split = (op).n_active <= kMgSplitBricks;                                        \
+        const dim3 grid(blocks((int64_t)(op).n_active * (split ? 256 : 64))), block(NT);           \
+        if ((op).bx == 64 && split)                                                                \
+            hipLaunchKernelGGL((kernel<64, 2>), grid, block, 0, __VA_ARGS__);                      \
+        else if ((op).bx == 64)                                                                    \
+            hipLaunchKernelGGL((kernel<64, 8>), grid, block, 0, __VA_ARGS__);                      \
+        else if (split)                                                                            \
+            hipLaunchKernelGGL((kernel<8, 2>), grid, block, 0, __VA_ARGS__);                       \
+        else                                                                                       \
+            hipLaunchKernelGGL((kernel<8, 8>), grid, block, 0, __VA_ARGS__);                       \
+    } while (0)
+
 void launch_mg_pre0(hipStream_t st, const MgOp &op, const float *r, const int4 *coord, const int *parent,
                     const MgLevelDev &c1, float omega_c, const SolveState *state) {
-    SHK_MG_LAUNCH(k_mg_pre0_w, op.bx, blocks((int64_t)op.n_active * 64), st, op, r, coord, parent, c1, omega_c, state);
+    SHK_MG_LAUNCH0(k_mg_pre0_w, op, st, op, r, coord, parent, c1, omega_c, state);
+}
+
+int mg_partials(int n_active) {
+    const int nb = (int)blocks((int64_t)n_active * (n_active <= kMgSplitBricks ? 256 : 64));
+    return nb <= kMgMaxPartials ? nb : kMaxBlocks;
 }
 
 void launch_mg_post0(hipStream_t st, const MgOp &op, const int4 *coord, const int *parent, const float *r,
-                     const float *xc, float *y, const SolveState *state, const Grid &g, double *cell_part,
-                     double *part) {
-    const unsigned nb = blocks((int64_t)op.n_active * 64);   // one wave per brick
-    SHK_MG_LAUNCH(k_mg_post0_w, op.bx, nb, st, op, coord, parent, r, xc, y, state, cell_part);
-    hipLaunchKernelGGL(k_mg_fold, dim3((g.blocks + NT - 1) / NT), dim3(NT), 0, st, (int)nb, cell_part, g.blocks, part,
-                       state);
+                     const float *xc, float *y, const SolveState *state, double *cell_part, double *part) {
+    const int nb = (int)blocks((int64_t)op.n_active * (op.n_active <= kMgSplitBricks ? 256 : 64));
+    const bool fold = nb > kMgMaxPartials;
+    SHK_MG_LAUNCH0(k_mg_post0_w, op, st, op, coord, parent, r, xc, y, state, fold ? cell_part : part);
+    if (fold)
+        hipLaunchKernelGGL(k_mg_fold, dim3((kMaxBlocks + NT - 1) / NT), dim3(NT), 0, st, nb, cell_part, kMaxBlocks,
+                           part, state);
 }
 
 void launch_mg_tail(hipStream_t st, int bx, const MgTail &t, float omega, float alpha, const SolveState *state) {

@@ -28,7 +28,7 @@ struct MgLevelHost {
 struct MgHierarchy {
     std::vector<MgLevelHost> lv;
     DevBuf<float> z;          // the preconditioned residual z = M r (level 0 bricks)
-    DevBuf<double> pz;        // r.z partials (one per Krylov workgroup)
+    DevBuf<double> pz;        // r.z partials (mg_partials)
     DevBuf<double> pcell;     // r.z sums of the post-smoothing blocks (one per 256 cells)
     DevBuf<int> cidx;         // coarsest: active cells
     DevBuf<float> cinv;       // coarsest: dense inverse on them
@@ -295,7 +295,7 @@ int mg_setup(shk_ctx *c) {
     MgLevelHost &L0 = h->lv[0];
     const int64_t n0 = (int64_t)c->n_active * kBrickCells;
     HIPC(c, h->z.ensure((size_t)std::max<int64_t>(n0, 1)));
-    HIPC(c, h->pz.ensure((size_t)kMaxBlocks + 64));
+    HIPC(c, h->pz.ensure((size_t)std::max(kMaxBlocks, kMgMaxPartials)));
     HIPC(c, h->pcell.ensure((size_t)std::max<int64_t>((n0 + 255) / 256, 1)));
     launch_mg_mask(st, n0, c->sig64.p, L0.d.p);
     for (size_t l = 0; l < h->lv.size(); ++l) {
@@ -354,9 +354,8 @@ int mg_setup(shk_ctx *c) {
     return SHK_OK;
 }
 
-// z = M r on level 0 (brick layout).  The last kernel runs on the Krylov grid g and
-// writes the r.z partials into part.
-void mg_vcycle(shk_ctx *c, const float *r, float *z, const SolveState *state, const Grid *g, double *part) {
+// z = M r on level 0 (brick layout); its mg_partials(n_active) r.z partials go to part.
+void mg_vcycle(shk_ctx *c, const float *r, float *z, const SolveState *state, double *part) {
     MgHierarchy *h = c->mg;
     hipStream_t st = c->stream;
     const int L = (int)h->lv.size() - 1;
@@ -385,7 +384,7 @@ void mg_vcycle(shk_ctx *c, const float *r, float *z, const SolveState *state, co
         std::swap(F.v.x, F.v.t);
         std::swap(F.x.p, F.t.p);
     }
-    launch_mg_post0(st, op0, c->coord.p, L0.parent.p, r, h->lv[1].v.x, z, state, *g, h->pcell.p, part);
+    launch_mg_post0(st, op0, c->coord.p, L0.parent.p, r, h->lv[1].v.x, z, state, h->pcell.p, part);
 }
 
 // Mixed-precision refinement loop with MG-preconditioned inner CG.
@@ -407,6 +406,7 @@ int solve_mg(shk_ctx *c, shk_result *res) {
     const BrickOp<float> op = op32(c);
     Reduction red = reduction(c);
     red.pz = h->pz.p;
+    red.nz = mg_partials(c->n_active);
     const int interval = std::min(std::max(1, c->prm.check_interval), 4);
     while (r_inf > tol_abs && outer < std::max(1, c->prm.outer_max)) {
         double inner_rel = std::max(c->prm.inner_residual, 0.5 * tol_abs / r_inf);
@@ -415,7 +415,7 @@ int solve_mg(shk_ctx *c, shk_result *res) {
                                      c->prm.max_iterations - total);
         float *S[2] = {c->s32.p, c->t32.p};
         int m = 0;
-        mg_vcycle(c, c->r32.p, h->z.p, c->state.p, &g, h->pz.p);
+        mg_vcycle(c, c->r32.p, h->z.p, c->state.p, h->pz.p);
         launch_dir_spmv<float, float>(c->stream, g, op, h->z.p, S[0], S[1], c->q32.p, red);
         ++m;
         rc = drive(
@@ -423,7 +423,7 @@ int solve_mg(shk_ctx *c, shk_result *res) {
             [&]() {
                 launch_axpy_norm<float>(c->stream, g, nullptr, c->x32.p, c->r32.p, S[m & 1], c->q32.p, red,
                                         c->next_events());
-                mg_vcycle(c, c->r32.p, h->z.p, c->state.p, &g, h->pz.p);
+                mg_vcycle(c, c->r32.p, h->z.p, c->state.p, h->pz.p);
                 launch_dir_spmv<float, float>(c->stream, g, op, h->z.p, S[m & 1], S[(m + 1) & 1], c->q32.p, red,
                                               c->next_events());
                 ++m;
@@ -499,7 +499,7 @@ extern "C" int shk_mg_apply(shk_ctx *c, const float *r, float *z) {
     else
         hipLaunchKernelGGL(k_dense_to_bricks<8>, dim3(gb), dim3(256), 0, st, d.nx, d.ny, d.nz, c->coord.p,
                            c->n_active, r, c->r32.p);
-    mg_vcycle(c, c->r32.p, c->mg->z.p, nullptr, &c->grid, c->mg->pz.p);
+    mg_vcycle(c, c->r32.p, c->mg->z.p, nullptr, c->mg->pz.p);
     if (d.bx == 64)
         hipLaunchKernelGGL(k_bricks_to_dense<64>, dim3(gd), dim3(256), 0, st, d.nx, d.ny, d.nz, c->brick_slot.p,
                            c->nbx, c->nby, c->mg->z.p, z);
