@@ -74,43 +74,55 @@ int ensure_partials(shk_ctx *c) {
 }
 
 // Builds the active brick list, slot map and neighbour table from the brick flags.
-int build_bricks(shk_ctx *c) {
+// The flags, the number of unknowns (returned in nunk) and the tables pass through one pinned
+// buffer: a copy from or to pageable memory is staged by the runtime and holds the host up,
+// four of them and a second wait were a tenth of the projection of a small grid (24x20x18).
+int build_bricks(shk_ctx *c, unsigned long long &nunk) {
     const int64_t nb = (int64_t)c->nbx * c->nby * c->nbz;
-    c->h_flag.resize(nb);
-    HIPC(c, hipMemcpyAsync(c->h_flag.data(), c->brick_flag.p, nb, hipMemcpyDeviceToHost, c->stream));
-    HIPC(c, hipStreamSynchronize(c->stream));
+    const size_t o_slot = 8 + ((size_t)nb + 15) / 16 * 16 + 8, o_coord = o_slot + ((size_t)nb + 3) / 4 * 16,
+                 o_nbr = o_coord + sizeof(int4) * (size_t)nb;
+    if (!c->h_tables) HIPC(c, hipHostMalloc((void **)&c->h_tables, o_nbr + 6 * sizeof(int) * (size_t)nb,
+                                            hipHostMallocDefault));
+    uint8_t *const h = c->h_tables;
+    HIPC(c, hipMemcpyAsync(h, c->count.p, sizeof nunk, hipMemcpyDeviceToHost, c->stream));
+    HIPC(c, hipMemcpyAsync(h + 8, c->brick_flag.p, nb, hipMemcpyDeviceToHost, c->stream));
+    HIPC(c, hipStreamSynchronize(c->stream));   // also for the last call's reads of the buffer
+    std::memcpy(&nunk, h, sizeof nunk);
+    const uint8_t *const flag = h + 8;
     c->h_slot.assign(nb, -1);
     c->h_coord.clear();
     for (int bz = 0; bz < c->nbz; ++bz)
         for (int by = 0; by < c->nby; ++by)
             for (int bx = 0; bx < c->nbx; ++bx) {
                 const int64_t b = bx + (int64_t)c->nbx * (by + (int64_t)c->nby * bz);
-                if (c->h_flag[b]) {
+                if (flag[b]) {
                     c->h_slot[b] = (int)c->h_coord.size();
                     c->h_coord.push_back(make_int4(bx, by, bz, 0));
                 }
             }
     c->n_active = (int)c->h_coord.size();
-    c->h_nbr.assign(6 * (size_t)std::max(c->n_active, 1), -1);
+    std::memcpy(h + o_slot, c->h_slot.data(), sizeof(int) * nb);
+    if (c->n_active) std::memcpy(h + o_coord, c->h_coord.data(), sizeof(int4) * c->n_active);
+    int *const nbr = reinterpret_cast<int *>(h + o_nbr);
     for (int s = 0; s < c->n_active; ++s) {
         const int4 q = c->h_coord[s];
-        const int off[6][3] = {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}};
-        for (int f = 0; f < 6; ++f) {
-            const int x = q.x + off[f][0], y = q.y + off[f][1], z = q.z + off[f][2];
-            if (x < 0 || y < 0 || z < 0 || x >= c->nbx || y >= c->nby || z >= c->nbz) continue;
-            c->h_nbr[6 * s + f] = c->h_slot[x + (int64_t)c->nbx * (y + (int64_t)c->nby * z)];
-        }
+        const int64_t b = q.x + (int64_t)c->nbx * (q.y + (int64_t)c->nby * q.z), by = c->nbx,
+                      bz = (int64_t)c->nbx * c->nby;
+        nbr[6 * s + 0] = q.x > 0 ? c->h_slot[b - 1] : -1;
+        nbr[6 * s + 1] = q.x < c->nbx - 1 ? c->h_slot[b + 1] : -1;
+        nbr[6 * s + 2] = q.y > 0 ? c->h_slot[b - by] : -1;
+        nbr[6 * s + 3] = q.y < c->nby - 1 ? c->h_slot[b + by] : -1;
+        nbr[6 * s + 4] = q.z > 0 ? c->h_slot[b - bz] : -1;
+        nbr[6 * s + 5] = q.z < c->nbz - 1 ? c->h_slot[b + bz] : -1;
     }
     HIPC(c, c->brick_slot.ensure(nb));
-    HIPC(c, hipMemcpyAsync(c->brick_slot.p, c->h_slot.data(), sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
+    HIPC(c, hipMemcpyAsync(c->brick_slot.p, h + o_slot, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
     if (c->n_active == 0) return SHK_OK;
     const size_t n = (size_t)c->n_active * kBrickCells;
     HIPC(c, c->coord.ensure(c->n_active));
     HIPC(c, c->nbr.ensure(6 * (size_t)c->n_active));
-    HIPC(c, hipMemcpyAsync(c->coord.p, c->h_coord.data(), sizeof(int4) * c->n_active, hipMemcpyHostToDevice,
-                           c->stream));
-    HIPC(c, hipMemcpyAsync(c->nbr.p, c->h_nbr.data(), sizeof(int) * 6 * c->n_active, hipMemcpyHostToDevice,
-                           c->stream));
+    HIPC(c, hipMemcpyAsync(c->coord.p, h + o_coord, sizeof(int4) * c->n_active, hipMemcpyHostToDevice, c->stream));
+    HIPC(c, hipMemcpyAsync(c->nbr.p, nbr, sizeof(int) * 6 * c->n_active, hipMemcpyHostToDevice, c->stream));
     for (DevBuf<double> *b : {&c->diag64, &c->cx64, &c->cy64, &c->cz64, &c->b64, &c->sig64, &c->x64, &c->r64,
                               &c->s64, &c->t64, &c->q64})
         HIPC(c, b->ensure(n));
@@ -135,8 +147,6 @@ int build_bricks(shk_ctx *c) {
         }
     }
     c->grid = make_grid((int64_t)c->n_active * kBrickCells);
-    // host-side buffers must outlive the async copies above
-    HIPC(c, hipStreamSynchronize(c->stream));
     return ensure_partials(c);
 }
 
@@ -500,6 +510,7 @@ void shk_destroy(shk_ctx *c) {
     c->slots.release();
     if (c->h_state) (void)hipHostFree(c->h_state);
     if (c->h_misc) (void)hipHostFree(c->h_misc);
+    if (c->h_tables) (void)hipHostFree(c->h_tables);
     for (auto &ev : c->ev)
         if (ev) (void)hipEventDestroy(ev);
     for (auto &ev : c->uev)
@@ -820,8 +831,7 @@ int project_impl(shk_ctx *c, double dt, float *const user_vel[3], const float *c
     launch_label(c->stream, d, dfluid, area, rho, c->label.p, c->brick_flag.p, c->nbx, c->nby, c->count.p);
     HIPC(c, hipGetLastError());
     unsigned long long nunk = 0;
-    HIPC(c, hipMemcpyAsync(&nunk, c->count.p, sizeof nunk, hipMemcpyDeviceToHost, c->stream));
-    if ((rc = build_bricks(c))) return rc;
+    if ((rc = build_bricks(c, nunk))) return rc;
     c->unknowns = (int64_t)nunk;
     res->unknowns = c->unknowns;
     res->active_bricks = c->n_active;

@@ -120,8 +120,8 @@ struct shk_ctx {
     int64_t unknowns = 0;
     bool have_system = false;
     std::vector<int4> h_coord;
-    std::vector<int> h_nbr, h_slot;
-    std::vector<uint8_t> h_flag;
+    std::vector<int> h_slot;
+    uint8_t *h_tables = nullptr;   // pinned: brick flags in, brick tables out (build_bricks)
     DevBuf<int4> coord;
     DevBuf<int> nbr;
     // unscaled FP64 operator (diag, couplings zero off unknown pairs), rhs, sig = 1/sqrt(diag)
