@@ -10,8 +10,8 @@ to 1e-6.
 Prints one JSON line (rank 0).  `roofline` is for the dominant Krylov kernel:
 algorithmic bytes per launch / its average launch duration, timed with HIP events
 on the library's stream (ProfileKernels=1) over --profile-steps further steps of
-the same context right after the timed ones (the events add a little time per
-launch, so the timed steps themselves run without them).
+the same context right after the timed ones.  Those steps run two kernels per
+iteration; the timed ones run the solve in one launch where it fits the chip.
 `cpu_baseline` is the oracle (the FP64 CPU restatement of the reference's path) on the
 host: the whole projection with the CG-equivalent solve to the same stop, timed in full
 on the host threads, beside the reference-faithful serial CG (its discarded MIC(0) work

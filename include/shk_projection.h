@@ -138,7 +138,9 @@ void shk_destroy(shk_ctx *ctx);
  *   Report         0 | 1: RCMatrix_utility::report statistics of every assembled
  *                  system into shk_result.report_* (RCMatrix_utility.h:98-146) (0)
  *   ProfileKernels 0 | 1: time every Krylov kernel launch with HIP events on the
- *                  context's stream (read with shk_kernel_stats; resets the counters)
+ *                  context's stream (read with shk_kernel_stats; resets the counters);
+ *                  solves then launch two kernels per iteration also where they would
+ *                  run in one launch
  * Unknown keys and unparsable values return SHK_BAD_ARG. */
 int shk_configure(shk_ctx *ctx, const char *key, const char *value);
 

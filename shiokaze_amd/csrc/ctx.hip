@@ -76,7 +76,7 @@ int ensure_partials(shk_ctx *c) {
 // Builds the active brick list, slot map and neighbour table from the brick flags.
 // The flags, the number of unknowns (returned in nunk) and the tables pass through one pinned
 // buffer: a copy from or to pageable memory is staged by the runtime and holds the host up,
-// four of them and a second wait were a tenth of the projection of a small grid (24x20x18).
+// four of them and a second wait were a tenth of the projection of a small grid (32x36x28).
 int build_bricks(shk_ctx *c, unsigned long long &nunk) {
     const int64_t nb = (int64_t)c->nbx * c->nby * c->nbz;
     const size_t o_slot = 8 + ((size_t)nb + 15) / 16 * 16 + 8, o_coord = o_slot + ((size_t)nb + 3) / 4 * 16,

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(NT) void k_mg_residual_restrict(MgLevelDev f, MgLev
 }
 
 // x_f += alpha P0 x_c on the unknowns of a level f >= 1, one thread per cell (the
-// level above the coarsest; the others get theirs from k_mg_smooth)
+// level above the tail; the others get theirs from k_mg_smooth)
 template <int BX>
 __global__ __launch_bounds__(NT) void k_mg_prolong(MgLevelDev f, MgLevelDev c, float alpha, const SolveState *state) {
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
