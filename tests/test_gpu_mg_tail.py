@@ -1,7 +1,7 @@
 """One V-cycle against the numpy restatement at the sizes where the one-workgroup coarse end
 (k_mg_tail, csrc/mg.hip) changes shape: the coarsest level alone, odd and even extents, the
 first level that fits as a dense grid (16^3, 64^2) and one that no longer does (17^3, 65 x 64),
-and thin grids.  FP32 passes of at most 16 terms a cell against FP64: a few roundings (6e-8)
+and uneven grids.  FP32 passes of at most 16 terms a cell against FP64: a few roundings (6e-8)
 per level, two passes each way, far below the 1e-5 asked for."""
 import numpy as np
 import pytest
