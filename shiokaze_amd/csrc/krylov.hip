@@ -696,15 +696,16 @@ __global__ __launch_bounds__(NT) void k_csr_diag(CsrOp op, double *__restrict__ 
                                                  unsigned long long *__restrict__ longest) {
     __shared__ double lds[NT / kWave];
     const int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x;
+    const int64_t p0 = e < op.rows ? op.rowptr[e] : 0, p1 = e < op.rows ? op.rowptr[e + 1] : 0;
+    // rowptr out of order or below zero counts as a row that fits nowhere; such a row is not walked
+    const bool bad = p0 < 0 || p1 < p0;
     if (longest) {
-        // a length below zero (rowptr out of order) counts as one that fits nowhere
-        const int64_t n = e < op.rows ? op.rowptr[e + 1] - op.rowptr[e] : 0;
-        const double len = block_max<NT>(n < 0 ? 1e18 : (double)n, lds);
+        const double len = block_max<NT>(bad ? 1e18 : (double)(p1 - p0), lds);
         if (threadIdx.x == 0) atomicMax(longest, (unsigned long long)len);
     }
     if (e < op.rows) {
         double dv = 0.0;
-        for (int64_t p = op.rowptr[e]; p < op.rowptr[e + 1]; ++p)
+        for (int64_t p = bad ? p1 : p0; p < p1; ++p)
             if (op.cols[p] == e) dv = op.vals[p];
         diag[e] = dv;
         if (sig) sig[e] = dv > 0.0 ? 1.0 / sqrt(dv) : 0.0;

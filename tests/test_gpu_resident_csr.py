@@ -54,3 +54,16 @@ def test_csr_resident(n, band):
     z, r = s.solve(*dev[:3], torch.zeros_like(dev[3]))
     assert r["status"] == 0 and r["count"] == 0 and not z.any()
     s.close()
+
+
+@pytest.mark.parametrize("rowptr", [(-8, -4, -1), (-3, -2, -1), (5, 3, -1)])
+def test_rowptr_below_zero_is_refused(rowptr):
+    """Rows of few entries whose rowptr ends below 0: refused before a kernel follows it."""
+    import torch
+    import shiokaze_amd as shk
+    s = shk.PCGSolver(config={"Preconditioner": "jacobi"})
+    dev = (torch.tensor(rowptr, device="cuda"), torch.zeros(8, dtype=torch.int64, device="cuda"),
+           torch.ones(8, dtype=torch.float64, device="cuda"), torch.ones(2, dtype=torch.float64, device="cuda"))
+    with pytest.raises(shk.ShkError, match="rowptr"):
+        s.solve(*dev)
+    s.close()
