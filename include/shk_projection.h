@@ -128,6 +128,13 @@ void shk_destroy(shk_ctx *ctx);
  *   OuterMax       refinement steps for mixed (3)
  *   InnerResidual  relative stop of each mixed inner solve (1e-6, floor)
  *   CheckInterval  iterations launched between host convergence polls (32)
+ *   OneLaunchWait  seconds (0.67): a Jacobi or plain CG solve that fits the chip runs in
+ *                  one launch whose workgroups wait for each other.  Where some cannot get
+ *                  onto the chip for this long (another process's kernels, a CU mask), the
+ *                  solve runs in two kernels per iteration instead, and so do the next 32
+ *                  solves, 64 after a second time and so on up to 4096.  0: never in one
+ *                  launch (its kernels also hold most of the chip for the whole solve, so
+ *                  other streams' work may have to wait that long)
  *   HostPointers   0 | 1                   (0)
  *   UnetWeights    path of a trained preconditioner blob (for Preconditioner=unet)
  *   UnetSmoothing  smoothing steps after each network application inside the
@@ -272,7 +279,9 @@ size_t shk_noalloc_scratch_bytes(void);
 /* Accumulated launch count and total milliseconds of one Krylov kernel
  * ("spmv_dot": direction update fused with the stencil and s.As, or "axpy_norm")
  * since ProfileKernels was last set.
- * Only launches that did work are counted. */
+ * Only launches that did work are counted.  "one_launch" and "one_launch_gave_up" count
+ * the solves that ran in one launch and those that gave up waiting, with ProfileKernels=0
+ * too (total_ms 0). */
 int shk_kernel_stats(shk_ctx *ctx, const char *kernel, int64_t *launches, double *total_ms);
 
 /* ------------------------------------------------------------------ multigrid preconditioner */

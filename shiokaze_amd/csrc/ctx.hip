@@ -225,27 +225,31 @@ template <class T>
 int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces, double tol_rel,
                    int64_t max_iter, bool &ran) {
     ran = false;
-    if (c->profile) return SHK_OK;  // ProfileKernels times the launches of the two-kernel iteration
+    // ProfileKernels times the launches of the two-kernel iteration
+    if (c->profile || c->prm.one_launch_wait == 0.0) return SHK_OK;
     const ResidentPlan p = resident_plan<T>(op, c->device, c->cus);
-    if (p.blocks < 1) return SHK_OK;
+    if (p.blocks < 1 || c->one_launch.resting()) return SHK_OK;
     HIPC(c, c->slots.ensure(resident_slot_words()));
     HIPC(c, resident_cg<T>(c->stream, p, op, rhs, sig, x, faces, c->slots.p, c->state.p, c->h_state, tol_rel, max_iter,
-                           c->device, c->cus));
+                           c->prm.one_launch_wait, c->device, c->cus));
     ran = c->h_state->aborted == 0;
+    c->one_launch.ended(!ran);
     return SHK_OK;
 }
 int solve_resident_csr(shk_ctx *c, const CsrOp &op, const double *rhs, const double *sig, double *x, double *pub,
                        unsigned long long *slots, const unsigned long long *longest, bool &ran) {
     ran = false;
-    if (c->profile || resident_csr_plan(op.rows, 1, c->device, c->cus).blocks < 1) return SHK_OK;
+    if (c->profile || c->prm.one_launch_wait == 0.0 || resident_csr_plan(op.rows, 1, c->device, c->cus).blocks < 1)
+        return SHK_OK;
     unsigned long long len = 0;
     HIPC(c, hipMemcpyAsync(&len, longest, sizeof len, hipMemcpyDeviceToHost, c->stream));
     HIPC(c, hipStreamSynchronize(c->stream));
     const ResidentPlan p = resident_csr_plan(op.rows, (int64_t)len, c->device, c->cus);
-    if (p.blocks < 1) return SHK_OK;
+    if (p.blocks < 1 || c->one_launch.resting()) return SHK_OK;
     HIPC(c, resident_csr(c->stream, p, op, rhs, sig, x, pub, slots, c->state.p, c->h_state, c->prm.residual,
-                         c->prm.max_iterations, c->device, c->cus));
+                         c->prm.max_iterations, c->prm.one_launch_wait, c->device, c->cus));
     ran = c->h_state->aborted == 0;
+    c->one_launch.ended(!ran);
     return SHK_OK;
 }
 
@@ -626,6 +630,12 @@ int shk_configure(shk_ctx *c, const char *key, const char *value) {
     } else if (k == "CheckInterval") {
         if (!parse_int(value, i) || i < 1 || i > 4096) return c->fail(SHK_BAD_ARG, "bad CheckInterval '%s'", value);
         p.check_interval = (int)i;
+    } else if (k == "OneLaunchWait") {
+        if (!parse_double(value, d) || !(d >= 0.0) || d > 30.0)
+            return c->fail(SHK_BAD_ARG, "bad OneLaunchWait '%s' (0..30 seconds)", value);
+        p.one_launch_wait = d;
+        c->one_launch.left = 0;
+        c->one_launch.next = OneLaunchRest::kFirst;
     } else if (k == "HostPointers") {
         if (!parse_bool(value, b)) return c->fail(SHK_BAD_ARG, "bad HostPointers '%s'", value);
         p.host_pointers = b;
@@ -638,6 +648,7 @@ int shk_configure(shk_ctx *c, const char *key, const char *value) {
         }
         c->ucount = 0;
         c->ums = 0.0;
+        c->one_launch.ran = c->one_launch.gave_up = 0;
     } else if (k == "MgOmega" || k == "MgAlpha") {
         if (!parse_double(value, d) || !(d > 0.0) || !(d < 2.0))
             return c->fail(SHK_BAD_ARG, "bad %s '%s' (0 < value < 2)", k.c_str(), value);
@@ -1022,11 +1033,17 @@ int shk_kernel_stats(shk_ctx *c, const char *kernel, int64_t *launches, double *
         *total_ms = c->ums;
         return SHK_OK;
     }
+    if (k == "one_launch" || k == "one_launch_gave_up") {
+        *launches = k == "one_launch" ? c->one_launch.ran : c->one_launch.gave_up;
+        *total_ms = 0.0;
+        return SHK_OK;
+    }
     int idx = -1;
     for (int q = 0; q < shk_ctx::kKernels; ++q)
         if (k == names[q]) idx = q;
     if (idx < 0)
-        return c->fail(SHK_BAD_ARG, "unknown kernel '%s' (axpy_norm, spmv_dot, unet_apply)", kernel);
+        return c->fail(SHK_BAD_ARG, "unknown kernel '%s' (axpy_norm, spmv_dot, unet_apply, one_launch, "
+                                    "one_launch_gave_up)", kernel);
     *launches = c->pcount[idx];
     *total_ms = c->pms[idx];
     return SHK_OK;

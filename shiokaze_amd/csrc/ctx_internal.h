@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
@@ -63,6 +64,7 @@ struct Params {
     int outer_max = 3;
     double inner_residual = 1e-6;
     int check_interval = 32;
+    double one_launch_wait = 0.67;    // seconds until a one-launch solve gives up; 0: none is tried
     bool host_pointers = false;
     std::string unet_weights;
     int unet_smooth = 10;             // smoothing steps after each network application in FCG
@@ -78,6 +80,21 @@ struct Params {
     bool redist_rk2 = false;          // pderedistancer3.cpp:207 (RedistTemporalScheme Euler)
     bool solid_wall_extrap = true;    // gridutility3.cpp:394, 413 (SolidWallExtrapolation)
     bool horizontal_extrap = true;    // gridutility3.cpp:395, 414 (HorizontalSolidWallExtrapolation)
+};
+
+// When a context tries one-launch solves.  One that gave up has cost its wait: the next
+// kFirst solves that could run in one launch do not try, and twice as many after each
+// further give-up; a solve that runs through ends that.
+struct OneLaunchRest {
+    static constexpr int kFirst = 32, kMost = 4096;
+    int64_t ran = 0, gave_up = 0;  // solves since ProfileKernels was last set
+    int left = 0, next = kFirst;
+    bool resting() { return left > 0 && left-- > 0; }
+    void ended(bool aborted) {
+        (aborted ? gave_up : ran) += 1;
+        left = aborted ? next : 0;
+        next = aborted ? std::min(2 * next, kMost) : kFirst;
+    }
 };
 
 }  // namespace shk
@@ -144,6 +161,7 @@ struct shk_ctx {
     shk::Grid grid;
     int cus = 0;                       // compute units of the device
     DevBuf<unsigned long long> slots;  // exchange slots of the resident solve
+    shk::OneLaunchRest one_launch;
     DevBuf<SolveState> state;
     SolveState *h_state = nullptr;
     double *h_misc = nullptr;

@@ -103,8 +103,9 @@ void launch_axpy_norm(hipStream_t st, const Grid &g, const double *sig, T *x, T 
 // The whole CG solve in one launch with the vectors on the chip (resident.hip), for brick
 // operators with kappa (and kdiag).  The plan has blocks = 0 when the system does not fit;
 // sig as in launch_cg_init (FP64 with a unit diagonal only).  faces: n_active * 384
-// elements of scratch, slots: resident_slot_words().  Synchronises; *h_state then holds
-// the final state, and h_state->aborted says that the solve has to be run another way.
+// elements of scratch, slots: resident_slot_words(), wait: seconds until a workgroup gives
+// up on the others (below 10 ns: at once).  Synchronises; *h_state then holds the final
+// state, and h_state->aborted says that the solve has to be run another way.
 struct ResidentPlan {
     int bpw = 0;     // bricks per wave
     int blocks = 0;  // workgroups, at most one per CU
@@ -116,14 +117,14 @@ ResidentPlan resident_plan(const BrickOp<T> &op, int device, int cus);
 template <class T>
 hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig,
                        T *x, T *faces, unsigned long long *slots, SolveState *state, SolveState *h_state,
-                       double tol_rel, int64_t max_iter, int device, int cus);
+                       double tol_rel, int64_t max_iter, double wait, int device, int cus);
 
 // The same for a CSR matrix whose longest row has `longest` entries (bpw: rows per thread);
 // sig: solve the scaled system D^-1/2 A D^-1/2 and return the unscaled x.  pub: rows doubles.
 ResidentPlan resident_csr_plan(int64_t rows, int64_t longest, int device, int cus);
 hipError_t resident_csr(hipStream_t st, const ResidentPlan &p, const CsrOp &op, const double *rhs, const double *sig,
                         double *x, double *pub, unsigned long long *slots, SolveState *state, SolveState *h_state,
-                        double tol_rel, int64_t max_iter, int device, int cus);
+                        double tol_rel, int64_t max_iter, double wait, int device, int cus);
 
 // r = b - A x in FP64 (unscaled operator with its diagonal); part holds 4*blocks
 // partials; out = {max|r|, sum r^2, sum b^2, max|b|}.  Optionally rs = (float)

@@ -31,9 +31,12 @@
 // the slowest workgroup, 7 the halo planes, 9 the update and the faces.
 //
 // All workgroups have to be on the chip at once.  A launch takes at most one workgroup
-// per CU, the launches of a process share that budget (CuBudget), and a wait that lasts
-// kWaitTicks gives up: every workgroup then leaves, the state says kResidentAborted and
-// the caller runs the two-kernel solve instead.
+// per CU and the launches of a process share that budget (CuBudget), but another process
+// or a CU mask can keep a part of the workgroups out.  So a wait that lasts its limit
+// gives up: every workgroup then leaves, the state says aborted, the caller runs the
+// two-kernel solve, and the context leaves this form alone for a number of solves that
+// doubles with every further give-up (OneLaunchRest): 0.67 s of waiting for each 10 ms
+// solve would be paid on every call otherwise.
 #include <hip/hip_runtime.h>
 
 #include <condition_variable>
@@ -58,7 +61,7 @@ constexpr int kRep = 8;
 constexpr int kRepWords = 2 * kMaxWg + 32, kSetWords = kRep * kRepWords, kSlotWords = 4 * kSetWords;
 constexpr int kCsrW = 8;              // entries of a CSR row held in registers
 constexpr unsigned long long kEmpty = 0xFFF8DEADBEEF0001ull;  // a NaN that no sum produces
-constexpr unsigned long long kWaitTicks = 1ull << 26;         // 0.67 s of the 100 MHz clock
+constexpr double kTicksPerSecond = 1e8;  // s_memrealtime; 32 bits of it are 42 s
 
 __device__ inline void st_agent(unsigned long long *p, unsigned long long v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -108,6 +111,7 @@ struct ExchLds {
     double sum[RW], mx[RW];
     double tot[2];
     int gone;
+    uint32_t limit;  // clock ticks until a wait gives up (here, not in a register kept for it)
 };
 
 // Sum of `v` (and, with MAX, the maximum of `m`) over the grid, the same bits in every
@@ -144,7 +148,8 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
             }
             const unsigned long long *mine = set + (size_t)(blockIdx.x % kRep) * kRepWords;
             unsigned long long a[kMaxWg / kWave], b[kMaxWg / kWave];
-            const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+            const unsigned long long end =
+                __builtin_amdgcn_s_memrealtime() + (uint32_t)__builtin_amdgcn_readfirstlane((int)l.limit);
             for (;;) {
                 bool ok = true;
 #pragma unroll
@@ -159,7 +164,7 @@ __device__ inline bool exchange(double v, double m, unsigned e, unsigned long lo
 #pragma unroll
                 for (int c = 0; c < kMaxWg / kWave; ++c) ok = ok && a[c] != kEmpty && b[c] != kEmpty;
                 if (__all(ok)) break;
-                if (__builtin_amdgcn_s_memrealtime() - t0 > kWaitTicks) {
+                if (__builtin_amdgcn_s_memrealtime() > end) {
                     gone = 1;
                     break;
                 }
@@ -359,7 +364,8 @@ template <class T, bool UNIT, int BX, bool SCALED, int BPW>
 __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *__restrict__ rhs,
                                                        const double *__restrict__ sig, T *__restrict__ xout,
                                                        T *__restrict__ faces, unsigned long long *__restrict__ slots,
-                                                       SolveState *__restrict__ st, double tol_rel, int64_t max_iter) {
+                                                       SolveState *__restrict__ st, double tol_rel, int64_t max_iter,
+                                                       uint32_t limit) {
     using B = BrickShape<BX>;
     constexpr int X = B::X, Y = B::Y;
     // with few bricks x and the couplings stay in registers too; else the couplings are read
@@ -427,7 +433,8 @@ __global__ __launch_bounds__(RT, 2) void k_cg_resident(BrickOp<T> op, const T *_
         if (on) publish<T, BX>(r[b], scr, faces + (int64_t)slot * 384, lane, nb[b]);
     }
     double rho = 0.0, rn = 0.0, sigma = 0.0, alpha = 0.0, beta = 0.0;
-    bool alive = exchange<true>(acc, mx, e++, slots, xl_, rho, rn);
+    if (threadIdx.x == 0) xl_.limit = limit;
+    bool alive = exchange<true>(acc, mx, e++, slots, xl_, rho, rn) && limit != 0;  // 0: all give up
     const double rnorm0 = rn;
     const double tol_abs = (tol_rel < 1e-30 ? 1e-30 : tol_rel) * rnorm0;  // pcg_solver.h:235
     int64_t it = 0;
@@ -641,7 +648,8 @@ template <int RPT>
 __global__ __launch_bounds__(RT, 2) void k_csr_resident(CsrOp op, const double *__restrict__ rhs,
                                                         const double *__restrict__ sig, double *__restrict__ xout,
                                                         double *__restrict__ pub, unsigned long long *__restrict__ slots,
-                                                        SolveState *__restrict__ st, double tol_rel, int64_t max_iter) {
+                                                        SolveState *__restrict__ st, double tol_rel, int64_t max_iter,
+                                                        uint32_t limit) {
     constexpr int W = kCsrW;
     __shared__ ExchLds xl_;
     const int row0 = blockIdx.x * (RT * RPT) + threadIdx.x, rows = (int)op.rows;
@@ -671,7 +679,8 @@ __global__ __launch_bounds__(RT, 2) void k_csr_resident(CsrOp op, const double *
         if (on) st_face(pub + row, r[k]);
     }
     double rho = 0.0, rn = 0.0, sigma = 0.0, alpha = 0.0, beta = 0.0;
-    bool alive = exchange<true>(acc, mx, e++, slots, xl_, rho, rn);
+    if (threadIdx.x == 0) xl_.limit = limit;
+    bool alive = exchange<true>(acc, mx, e++, slots, xl_, rho, rn) && limit != 0;  // 0: all give up
     const double rnorm0 = rn;
     const double tol_abs = (tol_rel < 1e-30 ? 1e-30 : tol_rel) * rnorm0;  // pcg_solver.h:235
     int64_t it = 0;
@@ -748,17 +757,19 @@ constexpr int kBpwF64[] = {1, 2};
 
 template <class T, bool UNIT, int BX, bool SCALED, int BPW>
 void launch_one(hipStream_t st, int blocks, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces,
-                unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter) {
+                unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter, uint32_t limit) {
     hipLaunchKernelGGL((k_cg_resident<T, UNIT, BX, SCALED, BPW>), dim3(blocks), dim3(RT), 0, st, op, rhs, sig, x,
-                       faces, slots, state, tol_rel, max_iter);
+                       faces, slots, state, tol_rel, max_iter, limit);
 }
 
 template <class T, bool UNIT, int BX, bool SCALED>
 void launch_bpw(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig, T *x,
-                T *faces, unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter) {
+                T *faces, unsigned long long *slots, SolveState *state, double tol_rel, int64_t max_iter,
+                uint32_t limit) {
 #define SHK_RES(N)                                                                                                  \
     case N:                                                                                                         \
-        launch_one<T, UNIT, BX, SCALED, N>(st, p.blocks, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter); \
+        launch_one<T, UNIT, BX, SCALED, N>(st, p.blocks, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter,   \
+                                           limit);                                                                 \
         break
     if constexpr (sizeof(T) == 4) {
         switch (p.bpw) {
@@ -846,39 +857,42 @@ ResidentPlan resident_csr_plan(int64_t rows, int64_t longest, int device, int cu
 
 hipError_t resident_csr(hipStream_t st, const ResidentPlan &p, const CsrOp &op, const double *rhs, const double *sig,
                         double *x, double *pub, unsigned long long *slots, SolveState *state, SolveState *h_state,
-                        double tol_rel, int64_t max_iter, int device, int cus) {
+                        double tol_rel, int64_t max_iter, double wait, int device, int cus) {
+    const uint32_t limit = (uint32_t)(wait * kTicksPerSecond);
     const CuHold hold(device, p.blocks, cus);
     hipLaunchKernelGGL(k_resident_begin, dim3((kSlotWords + 255) / 256), dim3(256), 0, st, state, slots);
     auto kern = p.bpw == 1 ? k_csr_resident<1> : p.bpw == 2 ? k_csr_resident<2> : k_csr_resident<3>;
-    hipLaunchKernelGGL(kern, dim3(p.blocks), dim3(RT), 0, st, op, rhs, sig, x, pub, slots, state, tol_rel, max_iter);
+    hipLaunchKernelGGL(kern, dim3(p.blocks), dim3(RT), 0, st, op, rhs, sig, x, pub, slots, state, tol_rel, max_iter,
+                       limit);
     return finish_resident(st, state, h_state);
 }
 
 template <class T>
 hipError_t resident_cg(hipStream_t st, const ResidentPlan &p, const BrickOp<T> &op, const T *rhs, const double *sig,
                        T *x, T *faces, unsigned long long *slots, SolveState *state, SolveState *h_state,
-                       double tol_rel, int64_t max_iter, int device, int cus) {
+                       double tol_rel, int64_t max_iter, double wait, int device, int cus) {
+    const uint32_t limit = (uint32_t)(wait * kTicksPerSecond);
     const CuHold hold(device, p.blocks, cus);
     hipLaunchKernelGGL(k_resident_begin, dim3((kSlotWords + 255) / 256), dim3(256), 0, st, state, slots);
     const bool unit = op.diag == nullptr, flat = op.bx == 64;
     if constexpr (sizeof(T) == 4) {
         if (unit && flat)
-            launch_bpw<T, true, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, true, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else if (unit)
-            launch_bpw<T, true, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, true, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else if (flat)
-            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else
-            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
     } else {
         if (unit && flat)
-            launch_bpw<T, true, 64, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, true, 64, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else if (unit)
-            launch_bpw<T, true, 8, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, true, 8, true>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else if (flat)
-            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, false, 64, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
         else
-            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter);
+            launch_bpw<T, false, 8, false>(st, p, op, rhs, sig, x, faces, slots, state, tol_rel, max_iter, limit);
     }
     return finish_resident(st, state, h_state);
 }
@@ -887,9 +901,9 @@ template ResidentPlan resident_plan<float>(const BrickOp<float> &, int, int);
 template ResidentPlan resident_plan<double>(const BrickOp<double> &, int, int);
 template hipError_t resident_cg<float>(hipStream_t, const ResidentPlan &, const BrickOp<float> &, const float *,
                                        const double *, float *, float *, unsigned long long *, SolveState *,
-                                       SolveState *, double, int64_t, int, int);
+                                       SolveState *, double, int64_t, double, int, int);
 template hipError_t resident_cg<double>(hipStream_t, const ResidentPlan &, const BrickOp<double> &, const double *,
                                         const double *, double *, double *, unsigned long long *, SolveState *,
-                                        SolveState *, double, int64_t, int, int);
+                                        SolveState *, double, int64_t, double, int, int);
 
 }  // namespace shk
