@@ -39,9 +39,7 @@
 // solve would be paid on every call otherwise.
 #include <hip/hip_runtime.h>
 
-#include <condition_variable>
-#include <mutex>
-
+#include "cu_budget.h"
 #include "krylov.h"
 #include "shk_projection.h"
 
@@ -740,13 +738,6 @@ __global__ void k_resident_begin(SolveState *st, unsigned long long *slots) {
     if (i == 0) st->aborted = 0;
 }
 
-// Workgroups of resident launches in flight per device: their sum never exceeds the CUs,
-// so that every launch gets all of its workgroups onto the chip.
-struct CuBudget {
-    std::mutex m;
-    std::condition_variable cv;
-    int used = 0;
-};
 constexpr int kMaxDevices = 64;
 CuBudget g_budget[kMaxDevices];
 
@@ -819,18 +810,8 @@ namespace {
 struct CuHold {
     CuBudget &bud;
     const int blocks;
-    CuHold(int device, int blocks_, int cus) : bud(g_budget[device]), blocks(blocks_) {
-        std::unique_lock<std::mutex> lk(bud.m);
-        bud.cv.wait(lk, [&] { return bud.used + blocks <= cus; });
-        bud.used += blocks;
-    }
-    ~CuHold() {
-        {
-            std::lock_guard<std::mutex> lk(bud.m);
-            bud.used -= blocks;
-        }
-        bud.cv.notify_all();
-    }
+    CuHold(int device, int blocks_, int cus) : bud(g_budget[device]), blocks(blocks_) { bud.acquire(blocks, cus); }
+    ~CuHold() { bud.release(blocks); }
 };
 // the state to the host; waits also after an error, for what runs
 hipError_t finish_resident(hipStream_t st, const SolveState *state, SolveState *h_state) {
