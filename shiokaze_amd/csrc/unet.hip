@@ -262,9 +262,13 @@ int ensure_grid(UnetNet *n, Grid3 m) {
              {&n->d16, v0 * 16},   {&n->dcat0, v0 * 48}, {&n->dd1, v1 * 32},  {&n->dcat1, v1 * 96}, {&n->dd2, v2 * 64},
              {&n->dcat2, v2 * 192}, {&n->dbott, v3 * 128}, {&n->dp3, v3 * 64}, {&n->de2, v2 * 64},  {&n->dp2, v2 * 32},
              {&n->de1, v1 * 32},   {&n->dp1, v1 * 16},  {&n->de0, v0 * 16},   {&n->tmp, v0 * 64}};
-    for (auto &x : a) UHIP(n, dalloc(*x.p, (size_t)x.n));
-    UHIP(n, dalloc(n->u, (size_t)v0));
-    UHIP(n, dalloc(n->du, (size_t)v0));
+    hipError_t e = hipSuccess;
+    for (auto &x : a)
+        if (e == hipSuccess) e = dalloc(*x.p, (size_t)x.n);
+    if (e == hipSuccess) e = dalloc(n->u, (size_t)v0);
+    if (e == hipSuccess) e = dalloc(n->du, (size_t)v0);
+    if (e != hipSuccess) n->L[0] = Grid3{};  // not this grid's: some buffers are missing
+    UHIP(n, e);
     return SHK_OK;
 }
 
@@ -275,6 +279,7 @@ int ensure_wgrad(UnetNet *n) {
     for (int l = 0; l < kLayers; ++l)
         want = std::max(want, conv_wgrad_part_elems(n->L[level[l]], kSpec[l].cin, kSpec[l].cout));
     if (want <= n->wpart_cap) return SHK_OK;
+    n->wpart_cap = 0;  // until the larger one is there
     UHIP(n, dalloc(n->wpart, (size_t)want));
     n->wpart_cap = want;
     return SHK_OK;
@@ -282,6 +287,7 @@ int ensure_wgrad(UnetNet *n) {
 
 int ensure_fine(UnetNet *n, int64_t nf) {
     if (nf <= n->fine_cap) return SHK_OK;
+    n->fine_cap = 0;
     UHIP(n, dalloc(n->fz, (size_t)nf));
     UHIP(n, dalloc(n->fe, (size_t)nf));
     UHIP(n, dalloc(n->fae, (size_t)nf));
@@ -701,6 +707,7 @@ int ensure_precond(shk_ctx *c) {
     u->pad = Grid3{(c->dims.nx + 15) / 16 * 16, (c->dims.ny + 15) / 16 * 16, (c->dims.nz + 15) / 16 * 16};
     const int64_t n = (int64_t)c->n_active * kBrickCells;
     if (n > u->cap) {
+        u->cap = 0;
         for (float **p : {&u->mask, &u->z, &u->p2}) HIPC(c, dalloc(*p, (size_t)n));
         HIPC(c, dalloc(u->c16, (size_t)(3 * n)));
         u->cap = n;
