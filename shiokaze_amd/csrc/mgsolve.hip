@@ -81,6 +81,7 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
     const int ay = ey > 1 ? 2 : 1;
     for (MgLevelHost &L : h->lv) L.v.bx = bx;
     if (same) return SHK_OK;
+    h->key_dims[0] = 0;  // until the tables and their buffers are whole
     for (size_t l = 1; l < h->lv.size(); ++l) release(h->lv[l]);
     h->lv.resize(1);
     L0.h_slot = c->h_slot;
@@ -160,10 +161,6 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
                 h->h_tail[i + (LT.v.nx + 1) * j + T.sxy[0] * k] =
                     s * kBrickCells + i % ex + ex * (j % ey) + kWave * (k % ez);
             }
-    h->key = c->h_slot;
-    h->key_dims[0] = c->dims.nx;
-    h->key_dims[1] = c->dims.ny;
-    h->key_dims[2] = c->dims.nz;
     // device copies
     hipStream_t st = c->stream;
     HIPC(c, h->tail_op.ensure((size_t)T.first[T.levels]));
@@ -200,6 +197,10 @@ int build_tables(shk_ctx *c, MgHierarchy *h) {
     }
     // the host vectors must outlive the asynchronous copies
     HIPC(c, hipStreamSynchronize(st));
+    h->key = c->h_slot;
+    h->key_dims[0] = c->dims.nx;
+    h->key_dims[1] = c->dims.ny;
+    h->key_dims[2] = c->dims.nz;
     return SHK_OK;
 }
 

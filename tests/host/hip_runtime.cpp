@@ -8,15 +8,12 @@
 namespace {
 std::set<void *> g_live;
 long g_calls = 0, g_fail = 0;
+double g_fill = 0.0;
 int allocate(void **p, size_t n) {
     *p = nullptr;
     if (++g_calls == g_fail) return 2;  // hipErrorOutOfMemory
     *p = std::malloc(n ? n : 1);
-    // ones as doubles, so that sums read back from a kernel's output are positive
-    for (size_t i = 0; i + 8 <= n && i < ((size_t)1 << 20); i += 8) {
-        const double one = 1.0;
-        std::memcpy((char *)*p + i, &one, 8);
-    }
+    for (size_t i = 0; i + 8 <= n; i += 8) std::memcpy((char *)*p + i, &g_fill, 8);
     g_live.insert(*p);
     return 0;
 }
@@ -32,6 +29,8 @@ void fail_allocation(long n) {
     g_calls = 0;
     g_fail = n;
 }
+// what new memory holds, as doubles: what is read back from kernels that did nothing
+void fill_memory(double v) { g_fill = v; }
 long allocations() { return g_calls; }
 long live_allocations() { return (long)g_live.size(); }
 

@@ -6,6 +6,7 @@
 #include "shk_projection.h"
 
 void fail_allocation(long n);
+void fill_memory(double v);
 long allocations();
 long live_allocations();
 
@@ -16,6 +17,7 @@ int train(shk_unet *net, int nx, int ny, int nz) {
 }
 
 int main() {
+    fill_memory(1.0);  // sums of kernels: positive
     int bad = 0;
     long whole = 0, tried = 0;
     for (long k = 0; k < 2 || k / 2 <= tried; ++k) {

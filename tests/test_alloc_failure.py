@@ -40,3 +40,7 @@ def _run(tmp_path, program, sources):
 
 def test_training_step(tmp_path):
     _run(tmp_path, "unet_alloc", ("unet", "unet_kernels"))
+
+
+def test_multigrid_tables(tmp_path):
+    _run(tmp_path, "mg_alloc", ("mgsolve", "mg"))
