@@ -615,14 +615,15 @@ int amg_setup(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int64_t *co
     if (!spd_inverse(C.n, dense))
         return c->fail(SHK_BREAKDOWN, "multigrid: the coarsest matrix is not positive definite");
     HIPC(c, upload(h->cinv, dense, st));
-    h->key_rows = rows;
-    h->key_nnz = nnz0;
-    h->key_x = key[0];
-    h->key_s = key[1];
     HIPC(c, h->z.ensure((size_t)std::max<int64_t>(rows, 1)));
     HIPC(c, h->x0.ensure((size_t)std::max<int64_t>(rows, 1)));
     HIPC(c, h->pz.ensure((size_t)kMaxBlocks + 64));
     HIPC(c, hipStreamSynchronize(st));
+    // the hierarchy is whole: the next solve may take it
+    h->key_rows = rows;
+    h->key_nnz = nnz0;
+    h->key_x = key[0];
+    h->key_s = key[1];
     return SHK_OK;
 }
 

@@ -44,3 +44,7 @@ def test_training_step(tmp_path):
 
 def test_multigrid_tables(tmp_path):
     _run(tmp_path, "mg_alloc", ("mgsolve", "mg"))
+
+
+def test_csr_multigrid_hierarchy(tmp_path):
+    _run(tmp_path, "amg_alloc", ("amg",))
