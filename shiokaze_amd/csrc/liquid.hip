@@ -34,6 +34,8 @@ struct LiquidWork {
     DevBuf<unsigned int> slots;
     DevBuf<uint32_t> list;        // a narrow band's cells (bands.h)
     DevBuf<unsigned int> counts;  // its length, counted cells
+    DevBuf<unsigned int> lens;    // lengths of advected bands: a call uses one and clears the other
+    int turn = -1;                // which; -1: neither is known to be 0
     DevBuf<double> part;
     std::vector<double> h_part;
     void release() {
@@ -48,6 +50,7 @@ struct LiquidWork {
         slots.release();
         list.release();
         counts.release();
+        lens.release();
         part.release();
     }
 };
@@ -635,94 +638,145 @@ __device__ inline bool cell_velocity(const Dims &d, const CFaces &f, int i, int 
     return u[0] != 0.0 || u[1] != 0.0 || u[2] != 0.0;
 }
 
-// MacCormack advection of the active cells of a cell-centred level set by the MAC
-// velocity (macadvection3.cpp:178-277, advect_scalar as the level-set tracker calls
-// it), over the list of those cells (what bounded one thread per cell of the grid was the
-// 65,536 workgroups of 256^3, of which a few percent had work: 58 us per pass).
-// Forward pass (lo != 0): out = semi-Lagrangian value (vec3d departure), the limiter's
-// bounds (min from FLT_MAX, max from FLT_MIN) and the narrow-band flag of the level set
-// before the step at the departure point.  Backward pass (fin_out != 0): the
-// semi-Lagrangian value of q0 over -dt, combined into the final value.  q0 is a new array
-// of the level set's type (macadvection3.cpp:248): off the band (mq, null: none) it reads
-// the background value.  Inactive cells of the output are left alone, and the passes read
-// no output of their own, so that the caller's array needs no copy.
-template <bool WENO>
-__global__ __launch_bounds__(kNT) void k_advect_cell(Dims d, Split sp, double dx, double dt, const uint32_t *list,
-                                                     const unsigned int *count, const float *q, const uint8_t *mq,
-                                                     CFaces vel, const float *fluid, int trim, float *out, float *lo,
-                                                     float *hi, uint8_t *band, const float *fin_qin,
-                                                     const float *fin_lo, const float *fin_hi,
-                                                     const uint8_t *fin_band, float *fin_out, float background) {
+// Advection of the active cells of a cell-centred level set by the MAC velocity
+// (macadvection3.cpp:178-277, advect_scalar as the level-set tracker calls it), MacCormack's
+// two passes or the semi-Lagrangian one alone, over the list of those cells or, where the
+// grid is small or the band wide, over all cells.  What bounds a pass over a thin band with
+// one thread per cell of the grid is the 65,536 workgroups of 256^3, of which a few percent
+// have work (58 us per pass, 25 over the list); one over a wide band the latency of its
+// loads, so the passes are instances of their own that leave room for 8 waves per SIMD.
+// Whole calls at 256^3, one thread per cell / here: all cells 646 / 623 us, a half 410 / 371,
+// a quarter 266 / 229, a tenth 192 / 150, 4% 161 / 92.
+// Forward: q0 = semi-Lagrangian value of phi (vec3d departure), the limiter's bounds (min
+// from FLT_MAX, max from FLT_MIN) and the narrow-band flag of the level set before the step
+// at the departure point.  Backward: the semi-Lagrangian value of q0 over -dt, combined into
+// the final value.  q0 is a new array of the level set's type (macadvection3.cpp:248): off
+// the band it reads the background value, which a pass over the list takes from the mask
+// (MASKED) and a forward pass over all cells writes there.  Inactive cells of phi are left
+// alone, and the passes read no output of their own, so that the caller's array needs no copy.
+enum AdvectPass { kForward, kBackward, kPlain };
+struct AdvectCell {
+    double dx, dt;
+    CFaces vel;
+    float *phi, *q0, *lo, *hi;
+    uint8_t *band;
+    int trim;
+    float background;
+    unsigned int *clear;  // a counter to set to 0, or null
+};
+template <bool WENO, AdvectPass PASS, bool MASKED>
+__device__ inline void advect_cell(const Dims &d, const Split &sp, const AdvectCell &a, const uint8_t *mask, int64_t c) {
 #pragma clang fp contract(off)
     const FS cs{d.nx, d.ny, d.nz};
-    const unsigned int len = *count;
-    for (unsigned int at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) {
-        const int64_t c = list[at];
-        int i, j, k;
-        decompose(c, sp, i, j, k);
-        double u[3];
-        const bool moving = cell_velocity(d, vel, i, j, k, u);
-        double p[3] = {(double)i, (double)j, (double)k};
-        const float here = q[c];
-        float value = here;
-        int ci = 0, cj = 0, ck = 0;
-        float vals[8];
-        if (moving) {
+    const float *q = PASS == kBackward ? a.q0 : a.phi;
+    const uint8_t *mq = PASS == kBackward && MASKED ? mask : nullptr;
+    int i, j, k;
+    decompose(c, sp, i, j, k);
+    double u[3];
+    const bool moving = cell_velocity(d, a.vel, i, j, k, u);
+    double p[3] = {(double)i, (double)j, (double)k};
+    const float here = q[c];
+    float value = here;
+    int ci = 0, cj = 0, ck = 0;
+    float vals[8];
+    if (moving) {
 #pragma unroll
-            for (int a = 0; a < 3; ++a) p[a] = p[a] - dt * u[a] / dx;
-            double coef[8];
-            interp_coef(cs, p, ci, cj, ck, coef);
-            float acc = 0.0f;
+        for (int m = 0; m < 3; ++m) p[m] = p[m] - a.dt * u[m] / a.dx;
+        double coef[8];
+        interp_coef(cs, p, ci, cj, ck, coef);
+        float acc = 0.0f;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            vals[n] = rd_bg(q, mq, corner(cs, ci, cj, ck, n), a.background);
+            if (coef[n] != 0.0) acc = (float)((double)acc + (double)vals[n] * coef[n]);
+        }
+        // WENO=1 (macadvection3.cpp:193-194)
+        value = WENO ? (float)weno3(q, mq, cs, p, a.background) : acc;
+    }
+    if (PASS != kBackward) a.q0[c] = value;
+    if (PASS == kForward) {
+        if (moving) {
+            double mn = FLT_MAX, mx = FLT_MIN;
 #pragma unroll
             for (int n = 0; n < 8; ++n) {
-                vals[n] = rd_bg(q, mq, corner(cs, ci, cj, ck, n), background);
-                if (coef[n] != 0.0) acc = (float)((double)acc + (double)vals[n] * coef[n]);
+                mn = fmin(mn, (double)vals[n]);
+                mx = fmax(mx, (double)vals[n]);
             }
-            // WENO=1 (macadvection3.cpp:193-194)
-            value = WENO ? (float)weno3(q, mq, cs, p, background) : acc;
+            a.lo[c] = (float)mn;
+            a.hi[c] = (float)mx;
+            a.band[c] = (double)interp(a.phi, nullptr, cs, p) > -a.dx * (double)a.trim;
+        } else {
+            a.lo[c] = here;
+            a.hi[c] = here;
+            a.band[c] = (double)here > -a.dx * (double)a.trim;
         }
-        if (out) out[c] = value;
-        if (lo) {
-            if (moving) {
-                double mn = FLT_MAX, mx = FLT_MIN;
-#pragma unroll
-                for (int n = 0; n < 8; ++n) {
-                    mn = fmin(mn, (double)vals[n]);
-                    mx = fmax(mx, (double)vals[n]);
-                }
-                lo[c] = (float)mn;
-                hi[c] = (float)mx;
-                band[c] = (double)interp(fluid, nullptr, cs, p) > -dx * (double)trim;
-            } else {
-                lo[c] = here;
-                hi[c] = here;
-                band[c] = (double)fluid[c] > -dx * (double)trim;
-            }
+    }
+    if (PASS == kBackward) {
+        float r;
+        if (a.band[c]) {
+            r = here;
+        } else {
+            const double mn = a.lo[c], mx = a.hi[c], q0 = here;
+            const double corr = 0.5 * ((double)a.phi[c] - (double)value);
+            if (q0 + corr < mn)
+                r = (float)mn;
+            else if (q0 + corr > mx)
+                r = (float)mx;
+            else
+                r = (float)(q0 + corr);
         }
-        if (fin_out) {
-            float r;
-            if (fin_band[c]) {
-                r = here;
-            } else {
-                const double mn = fin_lo[c], mx = fin_hi[c], q0 = here;
-                const double corr = 0.5 * ((double)fin_qin[c] - (double)value);
-                if (q0 + corr < mn)
-                    r = (float)mn;
-                else if (q0 + corr > mx)
-                    r = (float)mx;
-                else
-                    r = (float)(q0 + corr);
-            }
-            fin_out[c] = r;
-        }
+        a.phi[c] = r;
     }
 }
 
-// dst = src on the list's cells
-__global__ __launch_bounds__(kNT) void k_put_cells(const uint32_t *list, const unsigned int *count, const float *src,
-                                                   float *dst) {
-    const unsigned int len = *count;
-    for (unsigned int at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) dst[list[at]] = src[list[at]];
+template <bool WENO, AdvectPass PASS>
+__global__ __launch_bounds__(kNT) void k_advect_cell(Dims d, Split sp, BandPass cells, AdvectCell a) {
+    if (a.clear && blockIdx.x == 0 && threadIdx.x == 0) *a.clear = 0u;
+    bool wide;
+    const uint32_t len = cells.length(wide);
+    if (!wide) {
+        for (uint32_t at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT)
+            advect_cell<WENO, PASS, true>(d, sp, a, cells.mask, cells.list[at]);
+        return;
+    }
+    // the blocks change places every round: a band that follows the grid's rows would else be
+    // the same blocks' every time
+    uint32_t b = blockIdx.x;
+    for (uint32_t base = 0; base < len; base += gridDim.x * kNT) {
+        const uint32_t at = base + b * kNT + threadIdx.x;
+        b += (25u * gridDim.x) >> 6;
+        b = b < gridDim.x ? b : b - gridDim.x;
+        if (at >= len) continue;
+        if (cells.mask[at])
+            advect_cell<WENO, PASS, false>(d, sp, a, cells.mask, at);
+        else if (PASS == kForward)
+            a.q0[at] = a.background;
+    }
+}
+
+// dst = src on the band's cells, four of a wide band per thread (vec: 16-byte aligned arrays)
+__global__ __launch_bounds__(kNT) void k_put_cells(BandPass cells, int vec, const float *src, float *dst) {
+    bool wide;
+    const uint32_t len = cells.length(wide);
+    if (!wide) {
+        for (uint32_t at = blockIdx.x * kNT + threadIdx.x; at < len; at += gridDim.x * kNT) {
+            const uint32_t c = cells.list[at];
+            dst[c] = src[c];
+        }
+        return;
+    }
+    for (uint32_t g = blockIdx.x * kNT + threadIdx.x; g < (len + 3) / 4; g += gridDim.x * kNT) {
+        const uint32_t c = 4 * g;
+        if (vec && c + 4 <= len) {
+            const uchar4 m = *reinterpret_cast<const uchar4 *>(cells.mask + c);
+            if (m.x && m.y && m.z && m.w) {
+                *reinterpret_cast<float4 *>(dst + c) = *reinterpret_cast<const float4 *>(src + c);
+                continue;
+            }
+        }
+        for (uint32_t e = c; e < len && e < c + 4; ++e)
+            if (cells.mask[e]) dst[e] = src[e];
+    }
 }
 
 // ---------------------------------------------------------------- gravity, activity
@@ -1119,11 +1173,12 @@ int shk_extrapolate_levelset(shk_ctx *c, const float *solid, const uint8_t *soli
         HIPC(c, lw->list.ensure((size_t)n));
         hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, flag, 2);  // flag: now the list's length
         hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(n)), dim3(kBandNT), 0, st, n, band,
-                           aligned16({band}) ? 1 : 0, lw->list.p, flag);
+                           aligned16({band}) ? 1 : 0, 0, lw->list.p, flag);
         const unsigned gl = std::min(gb, kBandBlocks);
         hipLaunchKernelGGL(k_exls_wall, dim3(gl), dim3(kNT), 0, st, d, sp, c->dx, solid, lw->list.p, flag, phi,
                            lw->a[0].p, background, c->prm.solid_wall_extrap ? 1 : 0, c->prm.horizontal_extrap ? 1 : 0);
-        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, lw->list.p, flag, lw->a[0].p, phi);
+        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, BandPass{lw->list.p, flag, band, (uint32_t)n}, 0,
+                           lw->a[0].p, phi);
         hipLaunchKernelGGL(k_exls_dilate, dim3(gb), dim3(kNT), 0, st, d, sp, c->dx, phi, band, lw->a[1].p,
                            lw->band[0].p);
         hipLaunchKernelGGL(k_exls_combine, dim3(std::min(gb, 4 * kBandBlocks)), dim3(kNT), 0, st, d, sp, c->dx, solid,
@@ -1262,8 +1317,14 @@ int shk_advect_levelset(shk_ctx *c, double dt, float *phi, const uint8_t *mphi, 
     const bool mc = c->prm.maccormack;
     const int64_t G = (int64_t)d.nx * d.ny * d.nz;
     // scratch: the band's cells, q0 (b[0]), limiter bounds, band
-    HIPC(c, lw->list.ensure(G));
-    HIPC(c, lw->counts.ensure(2));
+    // a grid whose cells are all in flight at once needs no list (64^3: 51.7 us with it, 47.0
+    // without), and one pass pays for it later than two (128^3 semi-Lagrangian, with and
+    // without: thin band 47.6 and 48.4, all cells 64.6 and 58.1)
+    const bool listed = G > (int64_t)(mc ? 1 : 4) * kBandBlocks * kNT;
+    if (listed) {
+        HIPC(c, lw->list.ensure(G));
+        HIPC(c, lw->lens.ensure(2));
+    }
     HIPC(c, lw->b[0].ensure(G));
     if (mc) {
         HIPC(c, lw->lo[0].ensure(G));
@@ -1272,24 +1333,46 @@ int shk_advect_levelset(shk_ctx *c, double dt, float *phi, const uint8_t *mphi, 
     }
     const CFaces vel{{u, v, w}, {mu, mv, mw}};
     hipStream_t st = c->stream;
-    unsigned int *len = lw->counts.p;
-    hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, len, 2);
-    hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(G)), dim3(kBandNT), 0, st, G, mphi,
-                       aligned16({mphi}) ? 1 : 0, lw->list.p, len);
-    const unsigned gl = std::min(blocks_for(G), kBandBlocks);
-    auto kern = c->prm.weno ? k_advect_cell<true> : k_advect_cell<false>;
-    hipLaunchKernelGGL(kern, dim3(gl), dim3(kNT), 0, st, d, cells_split(d), c->dx, dt, lw->list.p, len, phi, nullptr,
-                       vel, phi, c->prm.trim_narrowband, lw->b[0].p, mc ? lw->lo[0].p : nullptr,
-                       mc ? lw->hi[0].p : nullptr, mc ? lw->band[0].p : nullptr, nullptr, nullptr, nullptr, nullptr,
-                       nullptr, background);
-    if (mc)  // reads q0 and, cell by cell, the level set it replaces
-        hipLaunchKernelGGL(kern, dim3(gl), dim3(kNT), 0, st, d, cells_split(d), c->dx, -dt, lw->list.p, len,
-                           lw->b[0].p, mphi, vel, nullptr, c->prm.trim_narrowband, nullptr, nullptr, nullptr, nullptr,
-                           phi, lw->lo[0].p, lw->hi[0].p, lw->band[0].p, phi, background);
-    else
-        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, lw->list.p, len, lw->b[0].p, phi);
+    unsigned int *len = nullptr, *next = nullptr;
+    if (listed) {
+        if (lw->turn < 0) hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, lw->lens.p, 2);
+        len = lw->lens.p + std::max(lw->turn, 0);
+        next = lw->lens.p + 1 - std::max(lw->turn, 0);
+        lw->turn = -1;  // until the call has gone through
+        hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(G)), dim3(kBandNT), 0, st, G, mphi,
+                           aligned16({mphi}) ? 1 : 0, kBandWideOf256, lw->list.p, len);
+    }
+    const BandPass cells{listed ? lw->list.p : nullptr, len, mphi, (uint32_t)G};
+    // enough blocks that those of a wide band are replaced as they end (256^3, all cells: 706 us
+    // with 2,048 blocks, 623 with 16,384); over the list of a thin one they cost nothing
+    const unsigned gl = std::min(blocks_for(G), 8 * kBandBlocks);
+    AdvectCell a{c->dx, dt, vel, phi, lw->b[0].p, nullptr, nullptr, nullptr, c->prm.trim_narrowband, background,
+                 next};
+    if (mc) {
+        a.lo = lw->lo[0].p;
+        a.hi = lw->hi[0].p;
+        a.band = lw->band[0].p;
+    }
+    if (!mc && !listed) {
+        // the pass reads a copy and writes in place: cheaper here than writing the band back
+        HIPC(c, hipMemcpyAsync(lw->b[0].p, phi, sizeof(float) * G, hipMemcpyDeviceToDevice, st));
+        std::swap(a.phi, a.q0);
+    }
+    const bool weno = c->prm.weno;
+    auto first = mc ? (weno ? k_advect_cell<true, kForward> : k_advect_cell<false, kForward>)
+                    : (weno ? k_advect_cell<true, kPlain> : k_advect_cell<false, kPlain>);
+    hipLaunchKernelGGL(first, dim3(gl), dim3(kNT), 0, st, d, cells_split(d), cells, a);
+    a.dt = -dt;
+    a.clear = nullptr;
+    if (mc)
+        hipLaunchKernelGGL((weno ? k_advect_cell<true, kBackward> : k_advect_cell<false, kBackward>), dim3(gl), dim3(kNT),
+                           0, st, d, cells_split(d), cells, a);
+    else if (listed)
+        hipLaunchKernelGGL(k_put_cells, dim3(gl), dim3(kNT), 0, st, cells, aligned16({mphi, phi, lw->b[0].p}) ? 1 : 0,
+                           lw->b[0].p, phi);
     HIPC(c, hipGetLastError());
     HIPC(c, hipStreamSynchronize(c->stream));
+    if (listed) lw->turn = next == lw->lens.p ? 0 : 1;
     return SHK_OK;
 }
 

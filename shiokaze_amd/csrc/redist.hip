@@ -405,7 +405,7 @@ extern "C" int shk_redistance(shk_ctx *c, float *phi, uint8_t *band, int width, 
     hipLaunchKernelGGL(k_redist_trim, dim3(g4), dim3(256), 0, st, s, sp, phi, band, vec_band, w->m.p);
     for (int r = 1; r <= width; ++r)
         hipLaunchKernelGGL(k_redist_dilate, dim3(g4), dim3(256), 0, st, s, sp, r, s.nx % 4 == 0 ? 1 : 0, w->m.p);
-    hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(n)), dim3(kBandNT), 0, st, n, m, 1, w->list.p, len);
+    hipLaunchKernelGGL(k_band_list, dim3(band_list_blocks(n)), dim3(kBandNT), 0, st, n, m, 1, 0, w->list.p, len);
     hipLaunchKernelGGL(k_redist_init, dim3(gl), dim3(256), 0, st, dx, w->list.p, len, m, phi, w->phi0.p, w->sgn.p);
     // the steps alternate between the caller's array and the work array
     float *P[2] = {phi, w->p.p};

@@ -94,3 +94,34 @@ def test_extrapolate_levelset(oracle, shape, offset):
             assert cnt == ocnt
             np.testing.assert_array_equal(dband.cpu().numpy(), oband)
             np.testing.assert_array_equal(dphi.cpu().numpy(), ophi)
+
+
+@pytest.mark.parametrize("offset,weno", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("maccormack,shape", [(1, (103, 84, 67)), (0, (151, 130, 109))])
+@pytest.mark.parametrize("kind", ["thin", "third", "all"])
+def test_advect_levelset_thin_and_wide_bands(oracle, kind, maccormack, shape, offset, weno):
+    """Grids large enough for a list (more than 524,288 cells, 2,097,152 for the one
+    semi-Lagrangian pass): a band of a few percent goes by its list, one of a third and one
+    of all cells by the mask (bands.h).  A second call uses the other counter."""
+    nx, ny, nz = shape
+    dx = 1.0 / nx
+    z, y, x = np.meshgrid(*[(np.arange(n) + 0.5) * dx for n in (nz, ny, nx)], indexing="ij")
+    phi = (y - 0.4 * ny * dx + 0.05 * np.sin(9 * x) * np.cos(7 * z)).astype(np.float32)
+    band = (np.abs(phi) < {"thin": 2 * dx, "third": 0.12, "all": 9.0}[kind]).astype(np.uint8)
+    low, high = {"thin": (0, 0.05), "third": (0.25, 0.5), "all": (0.99, 1)}[kind]
+    assert low < band.mean() <= high
+    rng = np.random.default_rng(5)
+    faces = [(nz, ny, nx + 1), (nz, ny + 1, nx), (nz + 1, ny, nx)]
+    vel = [rng.uniform(-2, 2, s).astype(np.float32) for s in faces]
+    masks = [(rng.random(s) < 0.9).astype(np.uint8) for s in faces]
+    ps, lv = _liquid(shape, dx)
+    with ps:
+        ps.configure("MacCormack", maccormack)
+        ps.configure("WENO", weno)
+        dphi, dband = _dev(phi, offset), _dev(band, offset)
+        dvel, dmasks = [_dev(v, 0) for v in vel], [_dev(m, 0) for m in masks]
+        for _ in range(2):
+            phi = oracle.advect_levelset(dx, 0.7 * dx, phi, band, vel, masks, 3 * dx, maccormack=bool(maccormack),
+                                         weno=bool(weno))
+            lv.advect_levelset(0.7 * dx, dphi, dband, dvel, dmasks, 3 * dx)
+            np.testing.assert_array_equal(dphi.cpu().numpy(), phi)
