@@ -1151,8 +1151,9 @@ int solve_csr_device(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int6
     const Grid g = make_grid(rows);
     HIPC(c, hipEventRecord(c->ev[0], c->stream));
     if (amg && (rc = amg_setup(c, rows, rowptr, cols, vals))) return rc;
-    HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
-    launch_csr_diag(c->stream, op, c->diag64.p, c->sig64.p, c->count.p);
+    // only Jacobi asks for the longest row
+    if (jac) HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
+    launch_csr_diag(c->stream, op, c->diag64.p, c->sig64.p, jac ? c->count.p : nullptr);
     const double *sig = jac ? c->sig64.p : nullptr;
     bool ran = false;
     // Plain CG keeps the two-kernel solve: unscaled, the iteration count follows the order of

@@ -115,8 +115,8 @@ int shk_solve_csr_noalloc(shk_ctx *c, int64_t rows, const int64_t *rowptr, const
     const Grid g = make_grid(rows);
     HIPC(c, hipEventRecord(c->ev[0], c->stream));
     const double *sg = jac ? sig : nullptr;
-    HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
-    launch_csr_diag(c->stream, op, diag, sig, c->count.p);
+    if (jac) HIPC(c, hipMemsetAsync(c->count.p, 0, sizeof(unsigned long long), c->stream));
+    launch_csr_diag(c->stream, op, diag, sig, jac ? c->count.p : nullptr);
     int rc = SHK_OK;
     bool ran = false;
     // the same choice as shk_solve_csr; the exchange slots go where the scaled values of the
