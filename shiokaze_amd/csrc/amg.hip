@@ -64,7 +64,6 @@ struct AmgLevel {
     DevBuf<int32_t> d_col;
     DevBuf<double> d_val;
     DevBuf<double> dinv;
-    DevBuf<int32_t> agg;            // row -> row of the next level
     DevBuf<int64_t> mptr;           // next level's row -> its rows mem[mptr[I] .. mptr[I+1])
     DevBuf<int32_t> mem;
     DevBuf<double> b;               // levels >= 1: the V-cycle's rhs
@@ -94,7 +93,6 @@ void amg_destroy(CsrAmg *h) {
         L.d_col.release();
         L.d_val.release();
         L.dinv.release();
-        L.agg.release();
         L.mptr.release();
         L.mem.release();
         L.b.release();
@@ -598,7 +596,6 @@ int amg_setup(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int64_t *co
         std::vector<int64_t> mptr, mem;
         members(agg, n2, mptr, mem);
         L.nc = n2;
-        HIPC(c, upload(L.agg, std::vector<int32_t>(agg.begin(), agg.end()), st));
         HIPC(c, upload(L.mptr, mptr, st));
         HIPC(c, upload(L.mem, std::vector<int32_t>(mem.begin(), mem.end()), st));
         // P'AP of the composed aggregation = the second pass's product of the first's

@@ -110,7 +110,6 @@ struct ResidentPlan {
     int bpw = 0;     // bricks per wave
     int blocks = 0;  // workgroups, at most one per CU
 };
-constexpr int kResidentAborted = -1;
 size_t resident_slot_words();
 template <class T>
 ResidentPlan resident_plan(const BrickOp<T> &op, int device, int cus);

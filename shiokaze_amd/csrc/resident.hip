@@ -339,7 +339,8 @@ __device__ inline bool next_direction(double rho_new, double rn, double tol_abs,
 }
 __device__ inline void end_state(SolveState *st, bool alive, double rho, double alpha, double beta, double sigma,
                                  double rn, double rnorm0, double tol_abs, int64_t it, int64_t max_iter, int status) {
-    // an aborted wait is seen by some workgroups only: any of them says so
+    // a wait that gave up is seen by some workgroups only: any of them says so, and the rest
+    // of the state counts for nothing
     if (threadIdx.x != 0) return;
     if (blockIdx.x == 0) {
         st->rho_k1 = rho;
@@ -353,7 +354,7 @@ __device__ inline void end_state(SolveState *st, bool alive, double rho, double 
         st->iter = it;
         st->max_iter = max_iter;
         st->done = 1;
-        st->status = alive ? status : kResidentAborted;
+        st->status = status;
     }
     if (!alive) st->aborted = 1;
 }
