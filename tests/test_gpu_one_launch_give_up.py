@@ -10,21 +10,11 @@ import numpy as np
 import pytest
 
 from test_gpu_resident import _fields, _project, _solver
-from test_gpu_resident_csr import _system
+from test_gpu_resident_csr import _counts, _system
 
 pytestmark = pytest.mark.gpu
 
 NOW, SOON = "1e-9", "2e-6"
-
-
-def _counts(s):
-    import ctypes
-    out = []
-    for name in (b"one_launch", b"one_launch_gave_up"):
-        n, ms = ctypes.c_int64(), ctypes.c_double()
-        assert s.lib.shk_kernel_stats(s.ctx, name, ctypes.byref(n), ctypes.byref(ms)) == 0
-        out.append(n.value)
-    return tuple(out)
 
 
 @pytest.mark.parametrize("wait", [NOW, SOON])

@@ -2,9 +2,12 @@
 
 ProfileKernels=1 runs the two-kernel iteration, so both solve the same system on one
 context.  Each stops with max|b - A x| <= tol max|b|, hence max|A (x1 - x2)| <= 2 tol
-max|b| whatever the summation orders; the sizes are the edges of the launch shape: one
-brick, a full and a started second workgroup (8 waves of 1 brick each), and systems that
-take 2 and 3 bricks per wave on 256 compute units.
+max|b| whatever the summation orders.  The sizes are the edges of the launch shape: one
+brick, a started second workgroup (8 waves of 1 brick each), and on 256 compute units both
+sides of the 2048, 4096, 6144, 8192 and 12,288 bricks at which a wave takes 2, 3, 4 and 6
+FP32 bricks (2 FP64 ones up to 4096) and the two-kernel iteration takes over, in 2D one size
+of each.  The active bricks are asserted, so that no row drifts to another kernel, and
+shk_kernel_stats' counters say which solve ran.
 """
 import threading
 
@@ -50,32 +53,52 @@ def _apply(sy, x):
     return y
 
 
-SHAPES = [(8, 8, 8), (19, 24, 13), (33, 30, 41), (16, 120, 100), (122, 130, 127), (176, 170, 182), (70, 37), (129, 264)]
+# shape, the bricks it lies between (more than, at most), bricks per wave in FP32 and FP64 (0: two
+# kernels)
+SHAPES = [((8, 8, 8), 0, 1, 1, 1), ((19, 24, 13), 0, 2048, 1, 1), ((33, 30, 41), 0, 2048, 1, 1),
+          ((16, 120, 100), 0, 2048, 1, 1), ((115, 126, 135), 1950, 2048, 1, 1), ((122, 130, 127), 1950, 2048, 1, 1),
+          ((129, 117, 127), 2048, 2200, 2, 2), ((145, 156, 165), 3900, 4096, 2, 2), ((162, 150, 160), 4096, 4200, 3, 0),
+          ((176, 170, 182), 4096, 6144, 3, 0), ((175, 186, 195), 5950, 6144, 3, 0), ((187, 187, 187), 6144, 6300, 4, 0),
+          ((196, 207, 216), 8000, 8192, 4, 0), ((210, 198, 208), 8192, 8400, 6, 0),
+          ((223, 234, 243), 12000, 12288, 6, 0), ((241, 241, 241), 12288, 12500, 0, 0),
+          ((70, 37), 0, 2048, 1, 1), ((129, 264), 0, 2048, 1, 1), ((1500, 1200), 0, 2048, 1, 1),
+          ((2000, 1800), 2048, 4096, 2, 2), ((2600, 2600), 4096, 6144, 3, 0), ((3000, 2700), 6144, 8192, 4, 0),
+          ((3300, 3200), 8192, 12288, 6, 0)]
 
 
-@pytest.mark.parametrize("precision,precond", [("fp64", "none"), ("fp64", "jacobi"), ("mixed", "none"),
-                                               ("mixed", "jacobi")])
-@pytest.mark.parametrize("shape", SHAPES, ids=str)
-def test_resident_matches_two_kernels(shape, precision, precond):
+# where two kernels run anyway the Jacobi row shows it
+ROWS = [(*row[:3], row[4] if precision == "fp64" else row[3], precision, precond) for row in SHAPES
+        for precision in ("fp64", "mixed") for precond in ("none", "jacobi")
+        if precond == "jacobi" or (row[4] if precision == "fp64" else row[3])]
+
+
+@pytest.mark.parametrize("shape,above,most,per_wave,precision,precond", ROWS,
+                         ids=["{0}-{4}-{5}".format(*row) for row in ROWS])
+def test_resident_matches_two_kernels(shape, above, most, per_wave, precision, precond):
     d, dx = _fields(shape, 3 if min(shape) > 12 else 1, 4)
-    tol = 1e-6
+    # plain CG of the large 2D grids does not get to 1e-6 in the 30,000 iterations of the default cap
+    tol = 1e-3 if precond == "none" and len(shape) == 2 and most > 4096 else 1e-6
     with _solver(shape, dx, Precision=precision, Preconditioner=precond, Residual=tol) as ps:
         xs, its = [], []
         for profile in (0, 1):
             ps.configure("ProfileKernels", profile)
             r, _ = _project(ps, d)
-            assert r["status"] == 0 and r["true_relres_inf"] <= tol * (1 + 1e-6)
+            # the recurrence residual of an FP64 solve differs from the true one by rounding
+            assert r["status"] == 0 and r["true_relres_inf"] <= tol * (1 + 1e-4)
             its.append(r["count"])
-            # only the two-kernel iteration launches (and times) its kernels one by one
+            assert above < r["active_bricks"] <= most
+            ran = ps.kernel_stats("one_launch")[0], ps.kernel_stats("one_launch_gave_up")[0]
+            assert ran == (r["outer"] if per_wave and not profile else 0, 0)
             assert (ps.kernel_stats("axpy_norm")[0] > 0) == (profile == 1)
             sy = ps.export_system()
             xs.append(sy["x"].clone())
         bmax = float(sy["rhs"].abs().max())
-        # the recurrence residual of an FP64 solve differs from the true one by rounding
         assert float(_apply(sy, xs[0] - xs[1]).abs().max()) <= 2 * tol * bmax * (1 + 1e-3)
-        # 20 random renumberings of the unknowns alone spread the plain CG of the small shapes
-        # over 246..270, 558..593 and 1322..1397 iterations (the oracle's CPU solve)
-        assert abs(its[0] - its[1]) <= max(3, 0.1 * its[1])
+        print(f"[gpu] {shape} {precision} {precond}: {r['active_bricks']} bricks, {per_wave} a wave, its {its}")
+        # FP64 plain CG: 20 random renumberings of the unknowns alone spread the counts of the small
+        # shapes over 246..270, 558..593 and 1322..1397 (the oracle's CPU solve).  The others do
+        # not see the order of the FP64 sums
+        assert abs(its[0] - its[1]) <= (max(3, 0.1 * its[1]) if (precision, precond) == ("fp64", "none") else 2)
 
 
 def test_resident_outcomes():
