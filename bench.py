@@ -11,7 +11,9 @@ Prints one JSON line (rank 0).  `roofline` is for the dominant Krylov kernel:
 algorithmic bytes per launch / its average launch duration, timed with HIP events
 on the library's stream (ProfileKernels=1) over --profile-steps further steps of
 the same context right after the timed ones.  Those steps run two kernels per
-iteration; the timed ones run the solve in one launch where it fits the chip.
+iteration; the timed ones run the solve in one launch where it fits the chip: `timed_solve`
+says which form they took and what an iteration of it costs, `roofline.of` what the
+roofline belongs to.
 `cpu_baseline` is the oracle (the FP64 CPU restatement of the reference's path) on the
 host: the whole projection with the CG-equivalent solve to the same stop, timed in full
 on the host threads, beside the reference-faithful serial CG (its discarded MIC(0) work
@@ -53,6 +55,21 @@ def log(msg):
 # those workloads.
 MEASURED_TRAFFIC_PER_CELL = {256: {"spmv_dot": 26.11, "axpy_norm": 24.03},
                              512: {"spmv_dot": 25.42, "axpy_norm": 24.01}}
+
+
+def timed_solve(ps, last):
+    """How the timed steps solved (read before ProfileKernels=1, which clears the counters and
+    runs two kernels per iteration): in one launch where the system fits the chip, and the time
+    of an iteration, refinement included."""
+    one, gave_up = ps.kernel_stats("one_launch")[0], ps.kernel_stats("one_launch_gave_up")[0]
+    return {"form": "one launch" if one and not gave_up else "launches per iteration",
+            "one_launch_solves": one, "one_launch_gave_up": gave_up,
+            "us_per_iteration": round(1e3 * last["ms_solve"] / max(last["count"], 1), 3)}
+
+
+def roofline_scope(solve):
+    return "two kernels per iteration, profile steps" + ("; the timed steps solve in one launch"
+                                                         if solve["one_launch_solves"] else "")
 
 
 def kernel_bytes_per_cell(kernel: str, precision: str, precond: str) -> int:
@@ -401,6 +418,7 @@ def main():
         results.append(step(ps))
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t_start
+    solve = timed_solve(ps, results[-1])
     if not args.no_profile and args.profile_steps > 0:
         # per-kernel durations: HIP events recorded on the library's stream around
         # every Krylov launch of these extra steps (same context, same scene)
@@ -441,6 +459,7 @@ def main():
             solve_bytes = sum(kernels[k].get("bytes_per_launch", 0) * kernels[k]["launches"] for k in kernels)
             solve_ms = sum(kernels[k]["total_ms"] for k in kernels)
             roofline["krylov_loop_GBs"] = round(solve_bytes / (solve_ms * 1e-3) / 1e9, 1)
+            roofline["of"] = roofline_scope(solve)
 
     # ---- the CPU leg: the oracle's FP64 truth, its CG-equivalent solve timed in full and
     # the reference-faithful serial CG (see cpu_leg)
@@ -626,6 +645,7 @@ def main():
             "ms_update": round(last["ms_update"], 3),
             **({"fallback": last.get("fallback", 0), "set": args.set} if args.preconditioner == "unet" else {}),
         },
+        "timed_solve": solve,
         "roofline": roofline,
         "kernels": kernels,
         "accuracy": accuracy,
@@ -764,6 +784,7 @@ def bench_2d(args, torch, shiokaze_amd, S):
         last = step(ps)
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
+    solve = timed_solve(ps, last)
     value = args.steps / elapsed
     log(f"2D timed: {args.steps} steps in {elapsed:.3f}s -> {value:.3f} solves/s, iters={last['count']}")
     cells = last["active_bricks"] * 512
@@ -784,7 +805,7 @@ def bench_2d(args, torch, shiokaze_amd, S):
             kd = kernels[dom]
             roofline = {"bound": "hbm", "kernel": dom, "achieved": kd["GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": kd["frac"], "traffic": None, "bytes_per_launch": kd["bytes_per_launch"],
-                        "avg_launch_us": kd["avg_us"]}
+                        "avg_launch_us": kd["avg_us"], "of": roofline_scope(solve)}
     accuracy = {}
     if not args.no_accuracy:
         sysb = ps.export_system()
@@ -837,7 +858,8 @@ def bench_2d(args, torch, shiokaze_amd, S):
                    "n": n, "dim": 2, "scene": args.scene, "seed": args.seed, "unknowns": last["unknowns"],
                    "active_bricks": last["active_bricks"], "pcg_iters": last["count"], "outer": last["outer"],
                    "precision": args.precision, "preconditioner": args.preconditioner},
-        "roofline": roofline, "kernels": kernels, "accuracy": accuracy, "cpu_baseline": cpu, "extra": extra,
+        "timed_solve": solve, "roofline": roofline, "kernels": kernels, "accuracy": accuracy, "cpu_baseline": cpu,
+        "extra": extra,
     }
     print(json.dumps(out), flush=True)
     ps.close()
