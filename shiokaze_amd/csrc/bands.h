@@ -54,7 +54,8 @@ __device__ inline unsigned int block_count(unsigned int v) {
 // instead of one thread per cell of the grid (256^3: 65,536 workgroups that mostly read one
 // byte and leave, 55..100 us per pass).  Each block compacts 4096 cells, in order, into a
 // range that one atomic reserves; the ranges' order does not matter, every cell of a pass
-// being independent.  *count starts at 0.  vec: mask is 16-byte aligned.
+// being independent.  *count starts at 0.  vec: mask is 16-byte aligned.  The list has room
+// for every cell (4 bytes each, 0.5 GB at 512^3), a band of any width being allowed.
 //
 // A wide band is better left where it lies: writing its list takes 113 us for the 16.8 million
 // cells of 256^3, the ranges come in the order in which blocks arrive, and a pass over them

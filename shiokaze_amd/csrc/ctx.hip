@@ -217,10 +217,13 @@ void fill_true_residual(shk_result *res, const double rr[4]) {
     res->true_relres_l2 = rr[2] > 0 ? std::sqrt(rr[1] / rr[2]) : 0.0;
 }
 
-// The sums of a solve here are taken in another order than the two-kernel iteration's.  In
-// mixed precision and with Jacobi the results stay the same to all digits that matter; FP64
-// plain CG, whose iterate at the stop follows that order, ends as near to the 1e-13 solution on
-// average (64 tanks of 16 to 90 cells a side: 5.3e-6 here, 5.5e-6 there, 19 of them farther).
+// The sums of a solve here are taken in another order than the two-kernel iteration's.  The rule
+// for taking it: iteration counts stay in the band that the parity tests of the entry allow, which
+// is what renumbering the unknowns alone does to the oracle's, and errors do not grow.  In mixed
+// precision (FP32 steps hide the last bits of the FP64 sums) and with Jacobi the counts are the
+// same throughout (23 grids up to 241^3 and 3300 x 3200).  FP64 plain CG follows the order: counts
+// move by up to 1.9%, and the iterate at the stop ends as near to the 1e-13 solution on average
+// (64 tanks of 16 to 90 cells a side: 5.3e-6 here, 5.5e-6 there, 19 of them farther).
 template <class T>
 int solve_resident(shk_ctx *c, const BrickOp<T> &op, const T *rhs, const double *sig, T *x, T *faces, double tol_rel,
                    int64_t max_iter, bool &ran) {
@@ -1156,9 +1159,10 @@ int solve_csr_device(shk_ctx *c, int64_t rows, const int64_t *rowptr, const int6
     launch_csr_diag(c->stream, op, c->diag64.p, c->sig64.p, jac ? c->count.p : nullptr);
     const double *sig = jac ? c->sig64.p : nullptr;
     bool ran = false;
-    // Plain CG keeps the two-kernel solve: unscaled, the iteration count follows the order of
-    // the sums (13 940 rows of the 32^3 glugging system: 604 to 638 iterations over ten orders),
-    // so another order would show in it, and it is the option that is used to compare against.
+    // Plain CG keeps the two-kernel solve by the rule above solve_resident: in k_csr_resident's
+    // order the 13,940 rows that this entry's parity test solves take 605 iterations, and it asks
+    // for 634..651 (the oracle's renumberings) with 2% to either side; two kernels take 623.
+    // Accuracy is not the reason: over eight systems neither order ends nearer to the solution.
     if (jac) {
         HIPC(c, c->slots.ensure(resident_slot_words()));
         if ((rc = solve_resident_csr(c, op, b, sig, x, c->q64.p, c->slots.p, c->count.p, ran))) return rc;

@@ -3,13 +3,14 @@
 // 39-183) on a dense level set with a per-cell activity mask (the narrow band).
 //
 // The trim, the dilations and the last step pass over the grid, the initial values and the
-// pseudo-time steps over a list of the band's cells (bands.h): at 256^3 the band holds about
-// 4% of the cells, and what bounded the dense passes was not memory but their 16.8 million
-// threads, each with a 64-bit index division, most of which found nothing to do.  The dense
-// passes take four cells per thread and skip groups without work.  The level set evolves in
-// the caller's array and one work array (cells off the band keep the caller's values, which
-// carry their side).  256^3 pool+sphere, width 3: the kernels of the call 0.95 -> 0.33 ms; its counts
-// went to one address per wave (0.24 ms of it), now per block.
+// pseudo-time steps over a list of the band's cells, made after the dilations (bands.h): at
+// 256^3 the band holds about 4% of the cells, and what bounded the dense passes was not
+// memory but their 16.8 million threads, each with a 64-bit index division, most of which
+// found nothing to do.  The dense passes take four cells per thread and skip groups without
+// work.  The level set evolves in the caller's array and one work array (cells off the band
+// keep the caller's values, which carry their side).  256^3 pool+sphere, width 3: the kernels
+// of the call 0.95 -> 0.33 ms; its counts went to one address per wave (0.24 ms of it), now
+// per block.
 //
 // Steps:
 //   1. trim_narrowband (src/utility/gridutility3.cpp:184-216): an active cell stays active

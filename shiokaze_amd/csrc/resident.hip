@@ -27,8 +27,9 @@
 // Measured against the two-kernel iteration, whole projections to 1e-6: 32x36x28 mixed
 // Jacobi 2.38 -> 0.90 ms, 100x77x90 FP64 Jacobi 6.9 -> 2.8 ms, 256^3 mixed Jacobi 32.1 ->
 // 13.3 ms, 600x450 (2D) mixed Jacobi 20.3 -> 7.2 ms.  One iteration at 256^3 takes 48.5
-// thousand cycles (52 us before): 16 the stencil, 17 the two exchanges with the wait for
-// the slowest workgroup, 7 the halo planes, 9 the update and the faces.
+// thousand cycles (52 us before): 14.6 the stencil (11 to 18 by the bricks a workgroup has),
+// 18.6 the two exchanges with the wait for the slowest workgroup, 6.8 the halo planes, 8.6 the
+// update and the faces.
 //
 // All workgroups have to be on the chip at once.  A launch takes at most one workgroup
 // per CU and the launches of a process share that budget (CuBudget), but another process

@@ -1759,7 +1759,7 @@ struct WgradPlan {
     int xw, tx, ty, tiles, splits, pairs;
 };
 // The voxels of a K step along x: 32, or 16 or 8 where that pads the rows less (rows of 24:
-// 24 instead of 32).  Blocks: about three per CU over the (ci, co) tiles, so that the
+// 24 instead of 32).  Blocks: about two per CU over the (ci, co) tiles, so that the
 // partial sums (28 KB per block) stay small beside the tensors.
 WgradPlan wgrad_plan(Grid3 g, int cin, int cout) {
     WgradPlan p;
