@@ -686,21 +686,27 @@ int ensure_precond(shk_ctx *c) {
             delete u;
             return c->fail(rc, "cannot create the U-Net");
         }
-        c->unet = u;
         if ((rc = unet_net_load(u->net, c->prm.unet_weights.c_str()))) {
             const std::string m = u->net->err;
             unet_destroy(u);
-            c->unet = nullptr;
             return c->fail(rc, "UnetWeights: %s", m.c_str());
         }
-        HIPC(c, dalloc(u->part1, (size_t)kPartCap));
-        HIPC(c, dalloc(u->part2, (size_t)kPartCap));
-        HIPC(c, dalloc(u->part3, (size_t)kPartCap));
-        HIPC(c, dalloc(u->fst, 4));
-        HIPC(c, hipHostMalloc((void **)&u->h_out, sizeof(double) * (kPartCap + 4), hipHostMallocDefault));
-        HIPC(c, hipMalloc((void **)&u->fs, 2 * sizeof(FcgState)));
-        HIPC(c, hipHostMalloc((void **)&u->h_fs, sizeof(FcgState) * UnetPrecond::kRing, hipHostMallocCoherent));
-        for (hipEvent_t &e : u->fev) HIPC(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        const auto allocate = [&]() -> int {
+            HIPC(c, dalloc(u->part1, (size_t)kPartCap));
+            HIPC(c, dalloc(u->part2, (size_t)kPartCap));
+            HIPC(c, dalloc(u->part3, (size_t)kPartCap));
+            HIPC(c, dalloc(u->fst, 4));
+            HIPC(c, hipHostMalloc((void **)&u->h_out, sizeof(double) * (kPartCap + 4), hipHostMallocDefault));
+            HIPC(c, hipMalloc((void **)&u->fs, 2 * sizeof(FcgState)));
+            HIPC(c, hipHostMalloc((void **)&u->h_fs, sizeof(FcgState) * UnetPrecond::kRing, hipHostMallocCoherent));
+            for (hipEvent_t &e : u->fev) HIPC(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            return SHK_OK;
+        };
+        if ((rc = allocate())) {
+            unet_destroy(u);
+            return rc;
+        }
+        c->unet = u;  // whole
     }
     UnetPrecond *u = c->unet;
     u->net->stream = c->stream;

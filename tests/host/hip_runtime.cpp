@@ -72,6 +72,15 @@ int hipStreamCreateWithFlags(void **s, unsigned) {
     return 0;
 }
 int hipStreamDestroy(void *) { return 0; }
+int hipEventCreate(void **e) {
+    *e = nullptr;
+    return 0;
+}
+int hipEventCreateWithFlags(void **e, unsigned) {
+    *e = nullptr;
+    return 0;
+}
+int hipEventDestroy(void *) { return 0; }
 int hipGetLastError() { return 0; }
 const char *hipGetErrorString(int) { return "error"; }
 int hipLaunchKernel(const void *, ...) { return 0; }

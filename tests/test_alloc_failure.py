@@ -34,7 +34,7 @@ def _run(tmp_path, program, sources):
     exe = tmp_path / "prog"
     # kernels and the functions that the program does not reach stay undefined
     subprocess.run(["g++", "-no-pie", *objs, "-o", str(exe), "-Wl,--unresolved-symbols=ignore-all"], check=True)
-    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    r = subprocess.run([str(exe), str(tmp_path / "file")], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
 
 
@@ -48,3 +48,7 @@ def test_multigrid_tables(tmp_path):
 
 def test_csr_multigrid_hierarchy(tmp_path):
     _run(tmp_path, "amg_alloc", ("amg",))
+
+
+def test_learned_preconditioner(tmp_path):
+    _run(tmp_path, "precond_alloc", ("unet", "unet_kernels"))
